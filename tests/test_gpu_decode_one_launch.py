@@ -1,0 +1,105 @@
+"""GPU parity of the one-launch single-token attention (decode_step.hip) where
+its dispatch and its loops can go wrong: F32, F16 and BF16 caches at the edges
+of a wave's keys and of a chunk, several chunks per workgroup, in-launch merge
+and merge kernel, ragged streams whose short windows leave splits without a
+key, strided K and V, scales of either sign.
+
+Each call is compared with the general row kernel (attn_path 1) on the same
+cache and with the fp64 oracle: 2e-3 max-abs / 1e-3 mean-abs for the 16-bit
+types, 1e-4 for F32 (the tolerances of these paths everywhere)."""
+import numpy as np
+import pytest
+
+import vva
+from gpu_util import as_f32, assert_close, fill_cache, oracle_attn, to_gpu
+
+pytestmark = pytest.mark.gpu
+
+TOL = {vva.F32: (1e-4, 1e-4), vva.F16: (2e-3, 1e-3), vva.BF16: (2e-3, 1e-3)}
+
+CASES = [
+    # d, Hq, Hkv, lens after the step, workgroups planned for (0: automatic)
+    (64, 14, 2, [1], 0),
+    (64, 8, 1, [16, 17, 32, 33], 0),
+    (128, 28, 4, [63, 64, 65], 0),
+    (128, 12, 2, [127, 128, 129], 0),
+    (128, 28, 4, [3001, 70], 0),          # the second stream has far fewer chunks than there are splits
+    (64, 14, 2, [2500, 2049], 8),         # 2 splits per stream and head: many chunks each, in-launch merge
+    (128, 12, 2, [4600], 2),              # one split: no merge
+    (128, 4, 4, [4097, 1], 160),          # one query head per kv head, 20 splits at most: merge kernel
+]
+
+
+@pytest.mark.parametrize("t", [vva.F32, vva.F16, vva.BF16])
+@pytest.mark.parametrize("d,Hq,Hkv,lens,wgs", CASES)
+def test_one_launch_step_and_attention(ctx, torch_gpu, d, Hq, Hkv, lens, wgs, t):
+    torch = torch_gpu
+    B = len(lens)
+    print(f"one-launch d={d} Hq={Hq} Hkv={Hkv} type={t} lens={lens} wgs={wgs}", flush=True)
+    past = [n - 1 for n in lens]
+    a = vva.KVCache(ctx, 1, Hkv, d, max(lens), B, t)
+    u = vva.KVCache(ctx, 1, Hkv, d, max(lens), B, t)
+    for kv in (a, u):
+        fill_cache(kv, past, seed=d + sum(lens))
+    rng = np.random.default_rng(11)
+    for it in (vva.F32, vva.BF16):
+        q, k, v = (to_gpu(torch, rng.standard_normal((B, 1, n, d)), it) for n in (Hq, Hkv, Hkv))
+        pos = torch.tensor([[n] for n in past], dtype=torch.int32, device="cuda")
+        qa, qu = torch.empty_like(q), torch.empty_like(q)
+        oa, ou, of = (torch.full((B, 1, Hq, d), float("nan"), device="cuda") for _ in range(3))
+        with ctx.schedule(decode_wgs=wgs):
+            ctx.decode_step(a, 0, q, k, v, pos, qa, oa, d ** -0.5)
+            splits = ctx.last_decode_splits()
+            ctx.rope_append(u, 0, q, k, v, pos, qu)
+            ctx.attn(u, 0, qu, of, d ** -0.5)             # the attention alone, same kernel
+        ctx.set_attn_path(1)
+        try:
+            ctx.attn(u, 0, qu, ou, d ** -0.5)             # the row kernel
+        finally:
+            ctx.set_attn_path(0)
+        torch.cuda.synchronize()
+        assert torch.equal(qa, qu), "rotated q differs"
+        assert torch.equal(oa, of), "the step differs from append + attention"
+        for s in range(B):
+            for x, y in zip(a.download(0, s, lens[s]), u.download(0, s, lens[s])):
+                np.testing.assert_array_equal(x, y)
+        assert_close(as_f32(torch, oa), as_f32(torch, ou), *TOL[t], what="vs the row kernel")
+        ref = oracle_attn(as_f32(torch, qa), a, 0, range(B), lens, 1, d ** -0.5)
+        mx, mn = assert_close(as_f32(torch, oa), ref, *TOL[t], what="vs exact")
+        print(f"  q type {it}: {splits} splits, vs exact max {mx:.2e} mean {mn:.2e}")
+    # scales of either sign and zero (a uniform mean of V)
+    for scale in (-0.2, 0.0):
+        ctx.attn(u, 0, qu, of, scale)
+        torch.cuda.synchronize()
+        ref = oracle_attn(as_f32(torch, qu), u, 0, range(B), lens, 1, scale)
+        assert_close(as_f32(torch, of), ref, *TOL[t], what=f"scale {scale}")
+    a.free()
+    u.free()
+
+
+@pytest.mark.parametrize("dt", ["float32", "float16", "bfloat16"])
+def test_one_token_flash_on_strided_rows(ctx, torch_gpu, dt):
+    """vva_flash_attn_ext, one token, K and V of different strides (V inside a
+    wider tensor), equal to the same values laid out densely."""
+    torch = torch_gpu
+    d, Hq, Hkv, L, B = 64, 14, 2, 777, 2
+    print(f"flash one token strided {dt}", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    typ = getattr(torch, dt)
+    q = torch.randn((B, Hq, 1, d), generator=gen, device="cuda")
+    k = torch.randn((B, L, Hkv, d), generator=gen, device="cuda").to(typ).transpose(1, 2)    # [B, Hkv, L, d] view
+    wide = torch.randn((B, Hkv, L, 2 * d), generator=gen, device="cuda").to(typ)
+    v = wide[..., d:]
+    outs = []
+    for kk, vv in ((k, v), (k.contiguous(), v.contiguous())):
+        out = torch.full((B, 1, Hq, d), float("nan"), device="cuda")
+        ctx.flash_attn_ext(q, kk, vv, out, d ** -0.5)
+        torch.cuda.synchronize()
+        outs.append(out)
+    assert torch.equal(outs[0], outs[1])
+    g = Hq // Hkv
+    qd = q.to(typ).double()                               # Q rounded to K's type
+    s = torch.matmul(qd.view(B, Hkv, g, d), k.double().transpose(2, 3).contiguous()) * d ** -0.5
+    ref = torch.matmul(torch.softmax(s, -1), v.double().contiguous()).view(B, 1, Hq, d)
+    tol = 1e-4 if dt == "float32" else 2e-3
+    assert (outs[0].double() - ref).abs().max().item() <= tol

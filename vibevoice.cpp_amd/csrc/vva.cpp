@@ -256,6 +256,36 @@ vva_status run_attention(vva_context* ctx, AttnArgs& a, bool fixed = false) {
         ctx->last_splits = ctx->logged_splits = n_splits;
         return VVA_OK;
     }
+    if (ctx->attn_path != 1 && a.T == 1 && a.k_type == a.v_type && a.mask_mode != kMaskExplicit) {
+        // F32 / F16 / BF16 rows without an explicit mask: every key is visible to the one token
+        StepArgs sa{};
+        sa.q = a.q; sa.q_type = a.q_type; sa.q_nb_h = a.q_nb_h; sa.q_nb_b = a.q_nb_b;
+        for (int b = 0; b < a.B; ++b) {
+            sa.kc[b] = const_cast<char*>(a.k[b]);
+            sa.vc[b] = const_cast<char*>(a.v[b]);
+            sa.past[b] = a.L[b] - 1;
+        }
+        sa.k_nb_tok = a.k_nb_tok; sa.k_nb_head = a.k_nb_head;
+        sa.v_nb_tok = a.v_nb_tok; sa.v_nb_head = a.v_nb_head;
+        sa.cache_type = a.k_type;
+        sa.scale = a.scale;
+        sa.out = a.out; sa.o_nb_h = a.o_nb_h; sa.o_nb_b = a.o_nb_b;
+        sa.tickets = ctx->tickets;
+        sa.d = a.d; sa.Hq = a.Hq; sa.Hkv = a.Hkv; sa.B = a.B; sa.G = a.Hq / a.Hkv;
+        if (decode_step_supported(sa)) {
+            const int n_splits = decode_step_splits(sa, ctx->n_cu, ctx->sched_decode_wgs);
+            vva_status st = get_ws(ctx, fixed, decode_step_ws_bytes(sa, n_splits), &ws);
+            if (st != VVA_OK) return st;
+            sa.ws = ws;
+            e = launch_decode_attn(sa, n_splits, ctx->stream);
+            if (e != hipSuccess) return hip_fail(ctx, e, "decode launch");
+            if (n_splits != ctx->logged_splits)
+                log_msg(VVA_LOG_DEBUG, "decode: one-launch kernel, %d key splits per kv head (B=%d, L[0]=%d)", n_splits,
+                        a.B, a.L[0]);
+            ctx->last_splits = ctx->logged_splits = n_splits;
+            return VVA_OK;
+        }
+    }
     if (ctx->attn_path != 1 && a.T == 1 && decode_supported(a)) {
         const int nw = decode_waves(a);
         int Lmax = 1;
@@ -1263,7 +1293,8 @@ extern "C" vva_status vva_decode_step(vva_context* ctx, vva_kv* kv, int layer, c
     a.v = (const char*)v->data; a.v_type = v->type; a.v_nb_h = v->nb[1]; a.v_nb_b = v->nb[3];
     a.pos = (const int32_t*)pos->data; a.pos_stride_b = ps;
     a.q_out = (char*)q_out->data; a.q_out_type = q_out->type; a.qo_nb_h = q_out->nb[1]; a.qo_nb_b = q_out->nb[3];
-    a.cache_row_bytes = kv->row_bytes; a.cache_head_bytes = kv->head_bytes; a.cache_type = kv->desc.type;
+    a.k_nb_tok = a.v_nb_tok = kv->row_bytes; a.k_nb_head = a.v_nb_head = kv->head_bytes;
+    a.cache_type = kv->desc.type;
     a.theta_scale = powf(freq_base, -2.0f / (float)d);
     a.scale = scale;
     a.out = (float*)out->data; a.o_nb_h = out->nb[1]; a.o_nb_b = out->nb[3];
@@ -1320,10 +1351,8 @@ extern "C" vva_status vva_decode_step(vva_context* ctx, vva_kv* kv, int layer, c
         if ((st = vva_rope_append(ctx, kv, layer, q, k, v, pos, seq_ids, freq_base, q_out)) != VVA_OK) return st;
         return vva_attn(ctx, kv, layer, q_out, seq_ids, nullptr, scale, out);
     }
-    const int n_splits = decode_step_splits(a);
-    if (n_splits > 1) {
-        if ((st = ensure_ws(ctx, (size_t)n_splits * B * Hq * (d + 2) * sizeof(float))) != VVA_OK) return st;
-    }
+    const int n_splits = decode_step_splits(a, ctx->n_cu, ctx->sched_decode_wgs);
+    if ((st = ensure_ws(ctx, decode_step_ws_bytes(a, n_splits))) != VVA_OK) return st;
     a.ws = ctx->ws;
     hipError_t e = launch_decode_step(a, n_splits, ctx->stream);
     if (e != hipSuccess) return hip_fail(ctx, e, "decode_step launch");

@@ -93,10 +93,10 @@ size_t window_f16_bytes(const AttnArgs& a);
 hipError_t launch_window_to_f16(const AttnArgs& a, void* dst, unsigned long long* ovf, unsigned long long epoch,
                                 hipStream_t s);
 
-// Single-token decode step in one launch (decode_step.hip): RoPE + append +
-// split attention + in-kernel merge.  F16 / BF16 caches, len + 1 <=
-// kMaxStepSplits * 128 keys, B * Hkv <= kMaxStepTickets.
-constexpr int kMaxStepSplits = 64;
+// Single-token attention over F32 / F16 / BF16 caches (decode_step.hip): the
+// decode step (RoPE + append + attention), or the attention alone
+// (launch_decode_attn: q already rotated; k, v, pos and q_out unused).
+// B * Hkv <= kMaxStepTickets.
 constexpr int kMaxStepTickets = 256;
 struct StepArgs {
     const char* q; int q_type; int64_t q_nb_h, q_nb_b;    // ne = [d, Hq, 1, B]
@@ -105,18 +105,21 @@ struct StepArgs {
     const int32_t* pos; int64_t pos_stride_b;
     char* q_out; int q_out_type; int64_t qo_nb_h, qo_nb_b;
     char* kc[kMaxBatch]; char* vc[kMaxBatch];              // row 0 of each sequence's K / V of the layer
-    int64_t cache_row_bytes, cache_head_bytes; int cache_type;
-    int past[kMaxBatch];                                   // the new row's index = len(seq_b)
+    int64_t k_nb_tok, k_nb_head, v_nb_tok, v_nb_head; int cache_type;
+    int past[kMaxBatch];                                   // the last key's index (a step: the new row's, len(seq_b))
     float theta_scale, scale;
     float* out; int64_t o_nb_h, o_nb_b;
-    float* ws;                                             // split partials
+    float* ws;                                             // split partials (decode_step_ws_bytes)
     unsigned* tickets;                                     // [B * Hkv], zero between calls
     int d, Hq, Hkv, B;
     int G;                                                 // Hq / Hkv
 };
 bool decode_step_supported(const StepArgs& a);
-int decode_step_splits(const StepArgs& a);
+// Key splits per (sequence, kv head); wgs > 0: workgroups to plan for
+int decode_step_splits(const StepArgs& a, int n_cu, int wgs);
+size_t decode_step_ws_bytes(const StepArgs& a, int n_splits);
 hipError_t launch_decode_step(const StepArgs& a, int n_splits, hipStream_t s);
+hipError_t launch_decode_attn(const StepArgs& a, int n_splits, hipStream_t s);
 
 // Linear layers around the attention (proj.hip).  Token row n = b * T + t.
 // kProjQKVRope: the few-row GEMV of kProjQKV with the RoPE and the append in
