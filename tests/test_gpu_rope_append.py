@@ -176,3 +176,43 @@ def test_vector_and_scalar_paths_agree_bit_for_bit(ctx, torch_gpu, in_t, cache_t
         np.testing.assert_array_equal(a0[0], a1[0])
         np.testing.assert_array_equal(a0[1], a1[1])
     kv.free()
+
+
+@pytest.mark.parametrize("d,Hq,Hkv", [(128, 28, 4), (64, 14, 2)])
+@pytest.mark.parametrize("T,B,cache_t,q_t,kv_t,out_t", [
+    (1, 2, vva.Q8_0, vva.F32, vva.F32, vva.F32),       # a decode step: slices of one token's items
+    (33, 1, vva.Q8_0, vva.BF16, vva.BF16, vva.BF16),
+    (511, 2, vva.Q8_0, vva.F32, vva.F16, vva.F16),     # 1022 rows: the last one-token count; mixed input types
+    (1025, 1, vva.F32, vva.F16, vva.BF16, vva.F32),    # two tokens per workgroup, the last one alone
+])
+def test_vector_path_edges_equal_the_scalar_path(ctx, torch_gpu, d, Hq, Hkv, T, B, cache_t, q_t, kv_t, out_t):
+    """The vector path's token counts, slices and types (Q8_0 caches among
+    them) against the scalar path, which the same values take 8 bytes off
+    every 16-byte boundary: Q and the cache bytes identical."""
+    torch = torch_gpu
+    print(f"rope vec d={d} T={T} B={B} cache={cache_t} in={q_t},{kv_t} out={out_t}", flush=True)
+    rng = np.random.default_rng(T)
+    sets = [[], []]
+    for H, t in ((Hq, q_t), (Hkv, kv_t), (Hkv, kv_t)):
+        x = to_gpu(torch, rng.standard_normal((B, T, H, d)), t)
+        off = 8 // x.element_size()
+        big = torch.zeros(x.shape[:-1] + (d + 8,), dtype=x.dtype, device="cuda")
+        big[..., off:off + d] = x
+        sets[0].append(x)
+        sets[1].append(big[..., off:off + d])
+    pos = torch.tensor(np.array([[30000 * b + t for t in range(T)] for b in range(B)], np.int32)).to("cuda")
+    kv = vva.KVCache(ctx, 2, Hkv, d, T + 3, B, cache_t)
+    for s in range(B):
+        kv.set_len(s, 2)
+    outs = []
+    for layer, (q, k, v) in enumerate(sets):
+        q_out = torch.zeros((B, T, Hq, d), device="cuda").to({vva.F32: torch.float32, vva.F16: torch.float16,
+                                                              vva.BF16: torch.bfloat16}[out_t])
+        ctx.rope_append(kv, layer, q, k, v, pos, q_out)
+        outs.append(q_out)
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0], outs[1])
+    for b in range(B):
+        for x, y in zip(kv.download(0, b, T + 3), kv.download(1, b, T + 3)):
+            np.testing.assert_array_equal(x, y)
+    kv.free()
