@@ -509,3 +509,56 @@ def test_prefill_q8_0_window_beyond_the_f16_range(ctx, torch_gpu, which):
         mx, mn = assert_close(got, ref, *TOL, what="K * 2^16, Q * 2^-16")
     print(f"  {which} up to {vmax:.3g}: max {mx:.2e} mean {mn:.2e}")
     kv.free()
+
+
+def test_bf16_v_converted_ahead_equals_converted_in_the_kernel(ctx, torch_gpu):
+    """A BF16 cache whose V window is converted to f16 ahead of the kernel
+    (vva_attn) and one that cannot be, its f16 window not fitting the static
+    scratch (vva_attn_noalloc): the same rounding, so the same bytes."""
+    torch = torch_gpu
+    d, Hq, Hkv, T, past = 128, 28, 4, 200, 36900
+    print(f"bf16 V window T={T} past={past}", flush=True)
+    assert (past + T) * Hkv * d * 2 > 36 << 20
+    kv = vva.KVCache(ctx, 1, Hkv, d, past + T, 1, vva.BF16)
+    fill_cache(kv, [past + T], seed=5)
+    kv.set_len(0, past)
+    q = torch.randn((1, T, Hq, d), device="cuda").to(torch.bfloat16)
+    outs = [torch.full((1, T, Hq, d), float("nan"), device="cuda") for _ in range(2)]
+    with ctx.schedule(prefill_splits=2):
+        ctx.attn(kv, 0, q, outs[0], d ** -0.5)
+        ctx.attn_noalloc(kv, 0, q, outs[1], d ** -0.5)
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0], outs[1])
+    kv.free()
+
+
+def test_bf16_v_window_of_ragged_and_strided_views(ctx, torch_gpu):
+    """The converted V window's offsets: ragged sequences (against the oracle)
+    and V inside a wider tensor (against the same values laid out densely)."""
+    torch = torch_gpu
+    d, Hq, Hkv, T, pasts = 64, 14, 2, 1500, [2600, 0, 700]
+    print(f"bf16 V window ragged T={T} past={pasts}", flush=True)
+    L = [p + T for p in pasts]
+    kv = vva.KVCache(ctx, 1, Hkv, d, max(L), 3, vva.BF16)
+    fill_cache(kv, L, seed=6)
+    for s, p in enumerate(pasts):
+        kv.set_len(s, p)
+    q = torch.randn((3, T, Hq, d), device="cuda")
+    out = torch.full((3, T, Hq, d), float("nan"), device="cuda")
+    ctx.attn(kv, 0, q, out, d ** -0.5)
+    torch.cuda.synchronize()
+    pick = np.array([0, 1, 36, 37, 700, T - 1], np.int32)
+    rows = (np.arange(3, dtype=np.int32)[:, None] * T + pick).reshape(-1)         # flattened rows b T + t
+    ref = oracle_attn(as_f32(torch, q), kv, 0, range(3), L, T, d ** -0.5, rows=rows)
+    assert_close(as_f32(torch, out)[:, pick], ref[:, pick], 2e-3, 1e-3, what="ragged BF16 windows")
+    kv.free()
+    k = torch.randn((2, 4000, Hkv, d), device="cuda").bfloat16().transpose(1, 2)
+    v = torch.randn((2, Hkv, 4000, 3 * d), device="cuda").bfloat16()[..., d:2 * d]
+    qf = torch.randn((2, Hq, T, d), device="cuda")
+    got = []
+    for kk, vv in ((k, v), (k.contiguous(), v.contiguous())):
+        o = torch.full((2, T, Hq, d), float("nan"), device="cuda")
+        ctx.flash_attn_ext(qf, kk, vv, o, d ** -0.5)
+        torch.cuda.synchronize()
+        got.append(o)
+    assert torch.equal(got[0], got[1])

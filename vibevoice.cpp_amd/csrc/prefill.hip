@@ -44,7 +44,9 @@
 // Tiles whose last key some row of the wave must not see (the diagonal, the
 // length boundary, or an explicit mask) set those scores to -inf first.
 // P and V enter the second product as f16 (BF16 V is converted after the
-// transposing read): an 8-bit-mantissa P would cost up to ~4e-3 on short
+// transposing read, or ahead of the kernel where window_bf16_v_bytes says so:
+// 8 waves x 32 rows each convert every fragment otherwise; 1.5B, 4096 tokens
+// 111 -> 97 us with the RoPE + append, 0.5B 83.7 -> 74.8): an 8-bit-mantissa P would cost up to ~4e-3 on short
 // rows, f16 P stays below 4e-4.  Q is rounded to K's type, as ggml's CPU
 // flash attention does.  Q8_0 and F32 windows are converted to f16 first by
 // window_to_f16_kernel (the reference casts F32 windows the same way before
@@ -135,8 +137,10 @@ __device__ __forceinline__ float bits16_to_f32(uint32_t v, int type) {
 
 __device__ __forceinline__ const lds_char* lds_at(uint32_t addr) { return (const lds_char*)(uintptr_t)addr; }
 
-// EXPL: explicit F16 mask (otherwise implicit causal / length masking only).
-template <int D, int KT, bool EXPL>
+// KT, VT: types of the K and V rows (VT = F16 beside BF16 K: V already
+// converted by window_bf16_v_kernel).  EXPL: explicit mask (otherwise
+// implicit causal / length masking only).
+template <int D, int KT, int VT, bool EXPL>
 __global__ void __launch_bounds__(kWaves * 64) prefill_kernel(AttnArgs a, float* __restrict__ ws, unsigned* tickets,
                                                                PrefillPlan plan) {
     prefetch_kernargs<sizeof(AttnArgs)>();
@@ -418,7 +422,7 @@ __global__ void __launch_bounds__(kWaves * 64) prefill_kernel(AttnArgs a, float*
         };
         auto read_v = [&](int p) {
             const int kk = (p / DT) * 16, dt = p % DT;
-            vf[p] = v_frag<KT>(va + dt * 64 + kk * VP, va + dt * 64 + (kk + 8) * VP);
+            vf[p] = v_frag<VT>(va + dt * 64 + kk * VP, va + dt * 64 + (kk + 8) * VP);
         };
         // The softmax of score v (p = 2^(s * scale * log2 e - m), then f16
         // pairs packed into chunk v / 8 = one 16-key MFMA step's P^T, and
@@ -658,6 +662,13 @@ __global__ void __launch_bounds__(kWaves * 64) prefill_kernel(AttnArgs a, float*
 // Combines the key splits of every split query row: one thread per (row,
 // 4 dims), log-sum-exp over the row tile's partials (exp2 domain),
 // normalized into out.  Rows of unsplit row tiles were written directly.
+// The partials of kMergeBatch splits are loaded together and summed under a
+// running max: a call of few rows (10 splits of 5 tokens) is bound by its
+// memory round trips, one per batch (0.5B, 5 tokens behind 611: 5.6 + 7.8 us with one per split,
+// the call now 9.8; 7B, 20 tokens behind 16000: 46.2 -> 34.4).
+// Up to kMergeBatch splits this is the in-launch merge's arithmetic, bit for
+// bit.
+constexpr int kMergeBatch = 8;
 template <int D>
 __global__ void __launch_bounds__(256) prefill_merge_kernel(AttnArgs a, const float* __restrict__ ws, PrefillPlan plan) {
     prefetch_kernargs<sizeof(AttnArgs)>();
@@ -672,20 +683,37 @@ __global__ void __launch_bounds__(256) prefill_merge_kernel(AttnArgs a, const fl
     const int n_ks = rt_splits(plan, rt);
     if (n_ks == 1) return;
     const float* ml = ws + nr_all * D * plan.max_ks;
-    float M = -INFINITY;
-    for (int k = 0; k < n_ks; ++k) M = fmaxf(M, ml[((int64_t)k * nr_all + rg) * 2]);
-    float den = 0.0f;
+    float M = -INFINITY, den = 0.0f;
     float4 num = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    if (M != -INFINITY) {
-        for (int k = 0; k < n_ks; ++k) {
-            const float2 e = *(const float2*)(ml + ((int64_t)k * nr_all + rg) * 2);
-            const float f = __builtin_amdgcn_exp2f(e.x - M);          // 0 for an empty split
-            const float4 v = *(const float4*)(ws + ((int64_t)k * nr_all + rg) * D + 4 * d4);
-            num.x = fmaf(v.x, f, num.x);
-            num.y = fmaf(v.y, f, num.y);
-            num.z = fmaf(v.z, f, num.z);
-            num.w = fmaf(v.w, f, num.w);
-            den = fmaf(e.y, f, den);
+    for (int k0 = 0; k0 < n_ks; k0 += kMergeBatch) {
+        float2 e[kMergeBatch];
+        float4 v[kMergeBatch];
+#pragma unroll
+        for (int u = 0; u < kMergeBatch; ++u) {
+            const int64_t r = (int64_t)min(k0 + u, n_ks - 1) * nr_all + rg;     // clamped: unconditional loads
+            e[u] = *(const float2*)(ml + r * 2);
+            v[u] = *(const float4*)(ws + r * D + 4 * d4);
+            if (k0 + u >= n_ks) e[u] = make_float2(-INFINITY, 0.0f);
+        }
+        float mb = M;
+#pragma unroll
+        for (int u = 0; u < kMergeBatch; ++u) mb = fmaxf(mb, e[u].x);
+        const float base = mb == -INFINITY ? 0.0f : mb;
+        const float f0 = __builtin_amdgcn_exp2f(M - base);                      // 0 while M = -inf
+        M = mb;
+        num.x *= f0;
+        num.y *= f0;
+        num.z *= f0;
+        num.w *= f0;
+        den *= f0;
+#pragma unroll
+        for (int u = 0; u < kMergeBatch; ++u) {
+            const float f = __builtin_amdgcn_exp2f(e[u].x - base);              // 0 for an empty split
+            num.x = fmaf(v[u].x, f, num.x);
+            num.y = fmaf(v[u].y, f, num.y);
+            num.z = fmaf(v[u].z, f, num.z);
+            num.w = fmaf(v[u].w, f, num.w);
+            den = fmaf(e[u].y, f, den);
         }
     }
     const float inv = den > 0.0f ? 1.0f / den : 0.0f;
@@ -693,19 +721,43 @@ __global__ void __launch_bounds__(256) prefill_merge_kernel(AttnArgs a, const fl
     *(float4*)(orow + 4 * d4) = make_float4(num.x * inv, num.y * inv, num.z * inv, num.w * inv);
 }
 
-template <int D, int KT>
+template <int D, int KT, int VT>
 hipError_t launch_pf(const AttnArgs& a, float* ws, unsigned* tickets, const PrefillPlan& p, hipStream_t s) {
     const int n_rt = (a.T * (a.Hq / a.Hkv) + kRowsWG - 1) / kRowsWG;
     dim3 grid(plan_pieces(p, n_rt) * a.Hkv, 1, a.B);
     if (a.mask_mode == kMaskExplicit)
-        hipLaunchKernelGGL((prefill_kernel<D, KT, true>), grid, dim3(kWaves * 64), 0, s, a, ws, tickets, p);
+        hipLaunchKernelGGL((prefill_kernel<D, KT, VT, true>), grid, dim3(kWaves * 64), 0, s, a, ws, tickets, p);
     else
-        hipLaunchKernelGGL((prefill_kernel<D, KT, false>), grid, dim3(kWaves * 64), 0, s, a, ws, tickets, p);
+        hipLaunchKernelGGL((prefill_kernel<D, KT, VT, false>), grid, dim3(kWaves * 64), 0, s, a, ws, tickets, p);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || p.max_ks == 1 || p.in_launch) return e;
     const int64_t threads = (int64_t)a.B * a.T * a.Hq * (D / 4);
     hipLaunchKernelGGL(prefill_merge_kernel<D>, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, a, ws, p);
     return hipGetLastError();
+}
+
+// BF16 V rows [0, L_b) to f16, contiguous [L_b][Hkv][d] per sequence: the
+// rounding the prefill kernel applies to each V^T fragment it reads, done
+// once per value instead of once per 32 query rows.  8 values per thread.
+__global__ void __launch_bounds__(256) window_bf16_v_kernel(AttnArgs a, uint16_t* __restrict__ dst) {
+    prefetch_kernargs<sizeof(AttnArgs)>();
+    const int b = blockIdx.y;
+    const int cpr = a.d / 8;                                          // 16-byte chunks of a head row
+    const int64_t n = (int64_t)a.L[b] * a.Hkv * cpr;
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    size_t off = 0;
+    for (int b2 = 0; b2 < b; ++b2) off += (size_t)a.L[b2] * a.Hkv * a.d;
+    const int c = (int)(i % cpr), h = (int)((i / cpr) % a.Hkv);
+    const int64_t row = i / ((int64_t)cpr * a.Hkv);
+    const uint4 u = *(const uint4*)(a.v[b] + row * a.v_nb_tok + h * a.v_nb_head + c * 16);
+    const uint32_t w[4] = {u.x, u.y, u.z, u.w};
+    uint32_t r[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+        r[e] = (uint32_t)f32_to_f16(__uint_as_float(w[e] << 16)) |
+               ((uint32_t)f32_to_f16(__uint_as_float(w[e] & 0xffff0000u)) << 16);
+    *(uint4*)(dst + off + i * 8) = make_uint4(r[0], r[1], r[2], r[3]);
 }
 
 // Strided windows (and F32 ones): quarter q of 32-element block k of a K or
@@ -877,6 +929,31 @@ size_t window_f16_bytes(const AttnArgs& a) {
     return (n + 255) / 256 * 256;
 }
 
+// Whether converting the BF16 V window once pays.  It costs a launch (3.5 us)
+// and the window's bytes (4 TB/s); it saves the conversions of every 32 query
+// rows' V^T fragments, 25 us of a 1.5B prefill of 4096 tokens (1e8 visible
+// (row, key) pairs at d = 128).
+size_t window_bf16_v_bytes(const AttnArgs& a) {
+    if (a.k_type != VVA_TYPE_BF16 || a.v_type != VVA_TYPE_BF16) return 0;
+    double pairs = 0.0, bytes = 0.0;
+    size_t n = 0;
+    for (int b = 0; b < a.B; ++b) {
+        const double keys = a.mask_mode == kMaskCausal ? a.past[b] + 0.5 * a.T : a.L[b];
+        pairs += keys * a.T * a.Hq;
+        n += (size_t)a.L[b] * a.Hkv * a.d * 2;
+    }
+    bytes = 2.0 * n;
+    if (pairs * a.d / 128 * 2.5e-7 < 1.25 * (3.5 + bytes / 4.0e6)) return 0;
+    return (n + 255) / 256 * 256;
+}
+hipError_t launch_window_bf16_v(const AttnArgs& a, void* dst, hipStream_t s) {
+    int Lmax = 1;
+    for (int b = 0; b < a.B; ++b) Lmax = max(Lmax, a.L[b]);
+    const int64_t n = (int64_t)Lmax * a.Hkv * (a.d / 8);
+    hipLaunchKernelGGL(window_bf16_v_kernel, dim3((unsigned)((n + 255) / 256), a.B), dim3(256), 0, s, a, (uint16_t*)dst);
+    return hipGetLastError();
+}
+
 hipError_t launch_window_to_f16(const AttnArgs& a, void* dst, unsigned long long* ovf, unsigned long long epoch,
                                 hipStream_t s) {
     int Lmax = 1;
@@ -1029,12 +1106,12 @@ bool prefill_in_launch_ok(const AttnArgs& a, const PrefillPlan& p) {
 
 hipError_t launch_prefill(const AttnArgs& a, float* ws, unsigned* tickets, const PrefillPlan& p, hipStream_t s) {
     if (p.in_launch && (!tickets || !prefill_in_launch_ok(a, p))) return hipErrorInvalidValue;
-    if (a.d == 64) {
-        return a.k_type == VVA_TYPE_F16 ? launch_pf<64, VVA_TYPE_F16>(a, ws, tickets, p, s)
-                                        : launch_pf<64, VVA_TYPE_BF16>(a, ws, tickets, p, s);
-    }
-    return a.k_type == VVA_TYPE_F16 ? launch_pf<128, VVA_TYPE_F16>(a, ws, tickets, p, s)
-                                    : launch_pf<128, VVA_TYPE_BF16>(a, ws, tickets, p, s);
+#define VVA_PF(D)                                                                                          \
+    (a.k_type == VVA_TYPE_F16   ? launch_pf<D, VVA_TYPE_F16, VVA_TYPE_F16>(a, ws, tickets, p, s)           \
+     : a.v_type == VVA_TYPE_F16 ? launch_pf<D, VVA_TYPE_BF16, VVA_TYPE_F16>(a, ws, tickets, p, s)          \
+                                : launch_pf<D, VVA_TYPE_BF16, VVA_TYPE_BF16>(a, ws, tickets, p, s))
+    return a.d == 64 ? VVA_PF(64) : VVA_PF(128);
+#undef VVA_PF
 }
 
 }  // namespace vva

@@ -217,6 +217,13 @@ vva_status ensure_ws(vva_context* ctx, size_t bytes) {
     return VVA_OK;
 }
 
+// Whether ensure_ws(bytes) would not have to grow during a capture.
+bool ws_can_hold(vva_context* ctx, size_t bytes) {
+    if (bytes <= ctx->ws_bytes) return true;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(ctx->stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone;
+}
+
 // Split workspace of one call: the context's, grown on demand, or (fixed)
 // the device's static scratch, which never allocates and refuses sizes
 // beyond kScratchBytes.
@@ -397,11 +404,32 @@ vva_status run_attention(vva_context* ctx, AttnArgs& a, bool fixed = false) {
     }
     if (ctx->attn_path != 1 && a.T > 1 && prefill_supported(a)) {
         const PrefillPlan plan = plan_for(a, fixed ? kScratchBytes : ((size_t)1 << 34));
-        if (plan.max_ks > 1) {
-            vva_status st = get_ws(ctx, fixed, prefill_ws_bytes(a, plan), &ws);
+        // BF16 V converted to f16 ahead of the kernel where that pays and the
+        // workspace can hold it beside the partials (the static scratch is
+        // what it is, and a stream under capture cannot grow the context's:
+        // the kernel then converts as it reads, with the same result)
+        const size_t pb = prefill_ws_bytes(a, plan), vb = window_bf16_v_bytes(a);
+        const bool conv_v = vb > 0 && (fixed ? pb + vb <= kScratchBytes : ws_can_hold(ctx, pb + vb));
+        if (conv_v || plan.max_ks > 1) {
+            vva_status st = get_ws(ctx, fixed, pb + (conv_v ? vb : 0), &ws);
             if (st != VVA_OK) return st;
         }
-        e = launch_prefill(a, ws, ctx->tickets + kMaxStepTickets, plan, ctx->stream);
+        if (conv_v) {
+            AttnArgs c = a;
+            char* p = (char*)ws;
+            e = launch_window_bf16_v(a, p, ctx->stream);
+            c.v_type = VVA_TYPE_F16;
+            c.v_nb_head = (int64_t)a.d * 2;
+            c.v_nb_tok = (int64_t)a.Hkv * a.d * 2;
+            for (int b = 0; b < a.B; ++b) {
+                c.v[b] = p;
+                p += (size_t)a.L[b] * a.Hkv * a.d * 2;
+            }
+            if (e == hipSuccess)
+                e = launch_prefill(c, (float*)((char*)ws + vb), ctx->tickets + kMaxStepTickets, plan, ctx->stream);
+        } else {
+            e = launch_prefill(a, ws, ctx->tickets + kMaxStepTickets, plan, ctx->stream);
+        }
         if (e != hipSuccess) return hip_fail(ctx, e, "prefill launch");
         ctx->last_splits = plan.max_ks;
         return VVA_OK;

@@ -93,6 +93,12 @@ size_t window_f16_bytes(const AttnArgs& a);
 hipError_t launch_window_to_f16(const AttnArgs& a, void* dst, unsigned long long* ovf, unsigned long long epoch,
                                 hipStream_t s);
 
+// BF16 V rows [0, L_b) of each sequence converted to f16 ([L_b][Hkv][d], one
+// after the other) for the MFMA prefill, which otherwise converts per 32 query
+// rows: the bytes, or 0 where the conversion does not pay.
+size_t window_bf16_v_bytes(const AttnArgs& a);
+hipError_t launch_window_bf16_v(const AttnArgs& a, void* dst, hipStream_t s);
+
 // Single-token attention over F32 / F16 / BF16 caches (decode_step.hip): the
 // decode step (RoPE + append + attention), or the attention alone
 // (launch_decode_attn: q already rotated; k, v, pos and q_out unused).
@@ -211,7 +217,7 @@ hipError_t launch_decode_stream_step(const AttnArgs& a, const StreamStep& st, fl
 // takes the sequence's tiles s, s + n_splits, s + 2 n_splits, ...
 int decode_stream_plan(const AttnArgs& a, int n_cu);
 hipError_t launch_decode_stream(const AttnArgs& a, float* ws, int n_splits, hipStream_t s);
-// MFMA flash prefill (F16 / BF16 caches).  Row tiles (256 query rows of
+// MFMA flash prefill (F16 / BF16 caches; BF16 K also beside F16 V).  Row tiles (256 query rows of
 // one kv group) rt >= R have their key range split over n workgroups (all
 // row tiles over `forced` when forced > 0); split rows leave partials in ws
 // (prefill_ws_bytes) that the last split of the row tile merges inside the
