@@ -350,6 +350,71 @@ def test_4096_token_projection_with_split_tail(ctx, torch_gpu, wt):
     print(f"  q max {mq[0]:.2e}; k max {mk[0]:.2e}")
 
 
+TILE_CASES = [
+    # hidden, Hq, Hkv, d, weights, cache, T, B: the tile and pieces of k that the call takes
+    (64, 2, 2, 64, vva.F16, vva.F16, 9, 1),          # 64 x 64, one k step (fewer than loads in flight), 9 rows
+    (384, 14, 2, 64, vva.Q8_0, vva.Q8_0, 65, 1),     # 64 x 64, a second token tile of one row
+    (448, 2, 1, 128, vva.Q8_0, vva.Q8_0, 33, 2),     # 64 features of a 128-dim head, Q8_0 cache (pair epilogue)
+    (832, 2, 1, 128, vva.F16, vva.BF16, 63, 1),      # the same, vector epilogue, 13 steps
+    (1536, 12, 2, 128, vva.Q8_0, vva.F32, 20, 1),    # 64 x 64 in pieces of k
+    (3584, 28, 4, 128, vva.F16, vva.Q8_0, 31, 2),    # the same, pair epilogue
+    (320, 14, 2, 64, vva.Q8_0, vva.F16, 1400, 1),    # 64 x 128
+    (640, 28, 4, 128, vva.F16, vva.Q8_0, 385, 1),    # 64 x 128 or 64 x 64, ragged token tile, pair epilogue
+    (3584, 28, 4, 128, vva.Q8_0, vva.Q8_0, 513, 1),  # 128 x 128 in pieces
+    (192, 28, 4, 128, vva.Q8_0, vva.BF16, 500, 1),   # 128 x 128 or 64 x 64, 3 steps
+    (192, 12, 2, 128, vva.Q8_0, vva.Q8_0, 4001, 1),  # 256 x 128, 3 steps, pair epilogue
+    (1536, 12, 2, 128, vva.F16, vva.F16, 1500, 2),   # 256 x 128, two sequences
+    (3584, 28, 4, 128, vva.F16, vva.Q8_0, 3001, 1),  # 256 x 256, pair epilogue, ragged
+    (3584, 28, 4, 128, vva.Q8_0, vva.F16, 1501, 2),  # 256 x 256 on dequantized weights, two sequences
+]
+
+
+@pytest.mark.parametrize("hidden,Hq,Hkv,d,wt,ct,T,B", TILE_CASES)
+def test_gemm_tiles_match_oracle(ctx, torch_gpu, hidden, Hq, Hkv, d, wt, ct, T, B):
+    """Every tile of the GEMM at its edges: k shorter than the loads in flight,
+    remainders of k and of the token rows, heads cut in two, pieces of k.  The
+    first and last 96 token rows of every sequence match the oracle, q_out's
+    other rows are finite, and the output projection of the same rows does."""
+    torch = torch_gpu
+    print(f"gemm tiles hidden={hidden} Hq={Hq} Hkv={Hkv} d={d} w={wt} cache={ct} T={T} B={B}", flush=True)
+    rng = np.random.default_rng(hidden + T + wt)
+    kv = vva.KVCache(ctx, 1, Hkv, d, T + 8, B, ct)
+    x = rng.standard_normal((B, T, hidden)).astype(np.float32)
+    raws, ws = zip(*[_weight(torch, rng, n * d, hidden, wt) for n in (Hq, Hkv, Hkv)])
+    bias = [(rng.standard_normal(n * d) * 0.5).astype(np.float32) for n in (Hq, Hkv, Hkv)]
+    pos = np.tile(np.arange(3, 3 + T, dtype=np.int32), (B, 1))
+    q_out = torch.full((B, T, Hq, d), float("nan"), dtype=torch.float32, device="cuda")
+    gb = [torch.from_numpy(b).cuda() for b in bias]
+    ctx.qkv_rope_append(kv, 0, torch.from_numpy(x).cuda(), *ws, torch.from_numpy(pos).cuda(), q_out,
+                        bq=gb[0], bk=gb[1], bv=gb[2])
+    torch.cuda.synchronize()
+    got = as_f32(torch, q_out)
+    assert np.isfinite(got).all()
+    rows = np.unique(np.r_[0:min(T, 96), max(0, T - 96):T])
+    for b in range(B):
+        y = [vvo.linear(x[b][rows], raws[i], wt, n * d, bias[i]).reshape(len(rows), n, d)
+             for i, n in enumerate((Hq, Hkv, Hkv))]
+        _check(got[b][rows], vvo.rope(y[0][None], pos[b][rows])[0], vva.F32, f"q (b={b})")
+        kraw, vraw = kv.download(0, b, T + 1)
+        for raw, ref, what in ((kraw, vvo.rope(y[1][None], pos[b][rows])[0], "k"), (vraw, y[2], "v")):
+            dec = vvo.to_f32(raw[rows].reshape(-1), ct, len(rows) * Hkv * d).reshape(len(rows), Hkv, d)
+            _check(dec, ref, ct, f"{what} cache (b={b})")
+            assert not raw[T:].any()
+    kv.free()
+    # the output projection: in = Hq d, out a multiple of 128
+    hid = (hidden + 127) // 128 * 128
+    wo_raw, wo = _weight(torch, rng, hid, Hq * d, wt)
+    o = rng.standard_normal((B, T, Hq * d)).astype(np.float32)
+    res = rng.standard_normal((B, T, hid)).astype(np.float32)
+    h = torch.full((B, T, hid), float("nan"), dtype=torch.float32, device="cuda")
+    ctx.out_proj_residual(torch.from_numpy(o).cuda(), wo, torch.from_numpy(res).cuda(), h)
+    torch.cuda.synchronize()
+    got = as_f32(torch, h)
+    assert np.isfinite(got).all()
+    for b in range(B):
+        _check(got[b][rows], vvo.linear(o[b][rows], wo_raw, wt, hid) + res[b][rows], vva.F32, f"h (b={b})")
+
+
 def test_projection_argument_errors(ctx, torch_gpu):
     torch = torch_gpu
     rng = np.random.default_rng(0)

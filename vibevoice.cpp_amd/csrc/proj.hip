@@ -15,19 +15,24 @@
 // ggml's integer block sums; each is below 2^-12 relative.)
 //
 // GEMM.  D[m][n] = sum_k W[m][k] X[n][k]: m = output feature, n = token row
-// (b * T + t), k = input feature.  A workgroup computes a 128 x 128 tile
-// over k in steps of 64 with 4 waves, each a 64 x 64 quadrant of 2 x 2
-// v_mfma_f32_32x32x16_f16 blocks.  Both operands are k-contiguous rows, so
-// every MFMA fragment is one 16-byte LDS read; rows are padded to 144 bytes
-// (16 mod 256: conflict-free fragment reads).  Tiles are staged through
-// registers into two LDS stages (the loads of tile j + 1 fly while tile j is
-// computed); the compiler tracks every load.  Workgroups are ordered so that
-// each XCD (workgroups are dealt to the 8 XCDs round-robin) walks a
-// contiguous run of tiles: the 36 weight tiles of one token tile share its
-// X tile in that XCD's L2.
+// (b * T + t), k = input feature.  Two kernels, chosen by gemm_plan: tiles of
+// 64 x 64 to 256 x 128 over either weight type (proj_gemm_kernel),
+// and 256 x 256 tiles over F16 weights for calls that fill the chip with them
+// (proj_gemm_big_kernel).  Both operands are k-contiguous rows, so every
+// v_mfma_f32_32x32x16_f16 fragment is one 16-byte LDS read.
 //
-// Few token rows (a decode step: B * T <= 8).  The GEMM's 128-row token tile
-// would be almost empty and its 36 workgroups too few to stream the weights,
+// proj_gemm_kernel: 4 or 8 waves, each a share of 32 x 32 blocks, k in steps of
+// 64.  Tiles are staged through registers into two LDS stages of rows padded
+// to 144 bytes (16 mod 256: conflict-free fragment reads; unpadded rows with
+// swizzled 16-byte slots measured the same); the compiler tracks every load.
+// Before this kernel, calls below 1024 rows ran 256 x 128 tiles
+// through an LDS ring (F16) or 128 x 128 tiles with one step's loads in flight
+// (Q8_0), three or four pieces of k each; us of a call, then and now: q/k/v
+// F16 0.5B 257 rows 31.2 -> 13.8, 1.5B 257 rows 35.9 -> 17.6, 7B 64 rows 32.5
+// -> 19.1; Q8_0 0.5B 64 rows 20.9 -> 14.0, 7B 16 rows 30.4 -> 20.1.
+//
+// Few token rows (a decode step: B * T <= 8).  The GEMM's token tile
+// would be almost empty and its workgroups too few to stream the weights,
 // so proj_gemv_kernel reads each weight row once, one wave of 4 rows per
 // workgroup (1152 workgroups for the 7B q/k/v stack, evenly spread over the
 // CUs), all of a lane's weight loads in flight before any is used: F16
@@ -44,6 +49,9 @@
 // q_out / cache types (Q8_0 rows quantized per 32-dim block).
 #include "vva_internal.hpp"
 
+#include <algorithm>
+#include <cmath>
+
 namespace vva {
 
 namespace {
@@ -53,14 +61,8 @@ namespace {
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-constexpr int kTM = 128;                    // output features per tile
-constexpr int kTN = 128;                    // token rows per tile
 constexpr int kTK = 64;                     // inputs per k step
 constexpr int kPitch = kTK * 2 + 16;        // LDS bytes per operand row
-constexpr int kOpBytes = 128 * kPitch;      // one operand tile: 18,432
-constexpr int kStage = 2 * kOpBytes;        // A (weights) then B (x)
-constexpr int kCPitch = kTM + 4;            // floats per token row of the epilogue tile
-static_assert(2 * kStage >= kTN * kCPitch * 4 + 16, "the epilogue tile (and the split ticket flag) reuse the two stages");
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void* base, uint32_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, 0x00020000);
@@ -73,23 +75,28 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void* base, uint32_
 // stores the 8 results as one 16-byte (f16 / bf16) or two (f32) stores.
 // One element per lane and store instruction would issue one lane per cycle.
 // The arithmetic per element is the pair epilogue's.
+// A tile of 64 features of a d = 128 head holds dims [c, c + 32) and [64 + c,
+// 96 + c) (c = `c0`): dl, Pl are the head's dims and pairs within the tile.
 template <int TM, int TN, int NTH>
-__device__ __forceinline__ void qkv_epilogue_vec(const ProjArgs& a, const float* C, int cpitch, int m0, int n0, int tid) {
+__device__ __forceinline__ void qkv_epilogue_vec(const ProjArgs& a, const float* C, int cpitch, int m0, int n0, int tid,
+                                                 int c0 = 0) {
     constexpr int CPT = TM / 8;                        // chunks per token row of the tile
     static_assert(NTH % CPT == 0, "a thread keeps its chunk");
     constexpr int TPP = NTH / CPT;                     // tokens per pass
     constexpr int EB = 4;                              // passes whose RoPE loads go out together
     const int d = a.d, P = d >> 1;
+    const int dl = min(d, TM), Pl = dl >> 1;
     const int c = tid % CPT, f = c * 8;
-    const int hl = f / d, i0 = f - hl * d;             // head within the tile, its first dim
-    const int f0 = m0 + hl * d;
+    const int hl = f / dl, il = f - hl * dl;           // head within the tile, its first dim there
+    const int f0 = m0 + hl * dl;
     if (f0 >= a.M) return;                             // past the last matrix
     const int mat = f0 < a.m_end[0] ? 0 : (f0 < a.m_end[1] ? 1 : 2);
     const int mrow = f0 - (mat == 0 ? 0 : mat == 1 ? a.m_end[0] : a.m_end[1]);
     const int head = mrow / d;
-    const bool lo = i0 < P;                            // first halves of the rotation pairs
-    const int ip = lo ? i0 + P : i0 - P;               // the partners' first dim
-    const int j0 = lo ? i0 : ip;                       // pair index of the first dim
+    const bool lo = il < Pl;                           // first halves of the rotation pairs
+    const int ilp = lo ? il + Pl : il - Pl;            // the partners' first dim in the tile
+    const int j0 = c0 + (lo ? il : ilp);               // pair index of the first dim
+    const int i0 = lo ? j0 : j0 + P, ip = lo ? j0 + P : j0;   // the dims of the head
     const float* bias = mat == 0 ? a.bias[0] : mat == 1 ? a.bias[1] : a.bias[2];
     float bs[8], bp[8];
 #pragma unroll
@@ -112,15 +119,15 @@ __device__ __forceinline__ void qkv_epilogue_vec(const ProjArgs& a, const float*
         for (int e = 0; e < EB; ++e) {
             const int nl = nb + TPP * e, n = n0 + nl;
             if (nl >= TN || n >= a.N) break;
-            const float* cr = C + nl * cpitch + hl * d;
+            const float* cr = C + nl * cpitch + hl * dl;
             // the chunk and its partners' chunk as 16-byte reads (the row
-            // pitch, d and i0 keep them 16-byte aligned): 8 scalar reads at a
+            // pitch, dl and il keep them 16-byte aligned): 8 scalar reads at a
             // 32-byte lane stride would meet on the same banks
             float yv[8], qv[8];
-            *(float4*)&yv[0] = *(const float4*)(cr + i0);
-            *(float4*)&yv[4] = *(const float4*)(cr + i0 + 4);
-            *(float4*)&qv[0] = *(const float4*)(cr + ip);
-            *(float4*)&qv[4] = *(const float4*)(cr + ip + 4);
+            *(float4*)&yv[0] = *(const float4*)(cr + il);
+            *(float4*)&yv[4] = *(const float4*)(cr + il + 4);
+            *(float4*)&qv[0] = *(const float4*)(cr + ilp);
+            *(float4*)&qv[4] = *(const float4*)(cr + ilp + 4);
             float out[8];
 #pragma unroll
             for (int k = 0; k < 8; ++k) {
@@ -158,7 +165,7 @@ __device__ __forceinline__ void qkv_epilogue_vec(const ProjArgs& a, const float*
 }
 
 // ---- split along K.  Each piece of a tile stores its accumulators (NW
-// compute waves x 2 x 2 blocks of v_mfma_f32_32x32x16) as one block of the
+// waves x BI x BJ blocks of v_mfma_f32_32x32x16) as one block of the
 // partial area, in the accumulators' own order [wave][block][4-register
 // group][lane] so that every store instruction writes 1 KB of whole lines,
 // with agent-scope (sc1) buffer stores: coherent across the XCDs' L2 caches
@@ -171,18 +178,19 @@ constexpr int kSc1 = 16;                               // buffer cache policy: a
 // vmcnt counts stores too, so a load waited for after a store waits for
 // that store as well (a batch of 8 keeps the unrolled code small)
 constexpr int kEpiQkv = 8, kEpiRes = 8;
-template <int NW>
-__device__ __forceinline__ void splitk_store(const f32x16 (&acc)[2][2], char* piece, int w, int lane) {
-    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(piece, (short)0, NW * 4096 * 4, 0x00020000);
+template <int NW, int BI, int BJ>
+__device__ __forceinline__ void splitk_store(const f32x16 (&acc)[BI][BJ], char* piece, int w, int lane) {
+    constexpr int NB = BI * BJ;
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(piece, (short)0, NW * NB * 4096, 0x00020000);
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < BI; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < BJ; ++j)
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 const u32x4 v = {__float_as_uint(acc[i][j][4 * g]), __float_as_uint(acc[i][j][4 * g + 1]),
                                  __float_as_uint(acc[i][j][4 * g + 2]), __float_as_uint(acc[i][j][4 * g + 3])};
-                __builtin_amdgcn_raw_buffer_store_b128(v, rs, (w * 16 + (i * 2 + j) * 4 + g) * 1024 + lane * 16, 0, kSc1);
+                __builtin_amdgcn_raw_buffer_store_b128(v, rs, ((w * NB + i * BJ + j) * 4 + g) * 1024 + lane * 16, 0, kSc1);
             }
 }
 // Thread 0 takes the ticket (after every piece store of the workgroup has
@@ -203,10 +211,11 @@ __device__ __forceinline__ bool splitk_ticket(unsigned* tk, int ksplit, int* fla
 // the tile, in split order; every thread of the workgroup (NT) takes part,
 // FB float4s at a time with all their loads in flight.  WM: compute waves
 // along the features (the wave's quadrant is wm = w % WM, wn = w / WM).
-template <int NW, int NT, int WM, int FB>
+template <int NW, int NT, int WM, int BI, int BJ, int FB>
 __device__ __forceinline__ void splitk_sum(const char* piece0, int ksplit, float* C, int cpitch) {
-    constexpr int PIECE = NW * 4096 * 4;
-    constexpr int NF = NW * 1024 / NT;                 // float4s per thread
+    constexpr int NB = BI * BJ;
+    constexpr int PIECE = NW * NB * 4096;
+    constexpr int NF = NW * NB * 256 / NT;             // float4s per thread
     static_assert(NF % FB == 0, "whole batches");
 #pragma unroll
     for (int f0 = 0; f0 < NF; f0 += FB) {
@@ -234,10 +243,10 @@ __device__ __forceinline__ void splitk_sum(const char* piece0, int ksplit, float
                 s.z += __uint_as_float(v[e][k].z);
                 s.w += __uint_as_float(v[e][k].w);
             }
-            const int w = f >> 10, gi = (f >> 6) & 15, lane = f & 63;
-            const int i = gi >> 3, j = (gi >> 2) & 1, g = gi & 3;
+            const int w = f / (NB * 256), blk = (f >> 8) % NB, g = (f >> 6) & 3, lane = f & 63;
+            const int i = blk / BJ, j = blk % BJ;
             const int wm = w % WM, wn = w / WM, l32 = lane & 31, half = lane >> 5;
-            *(float4*)(C + (wn * 64 + 32 * j + l32) * cpitch + wm * 64 + 32 * i + 4 * half + 8 * g) = s;
+            *(float4*)(C + ((wn * BJ + j) * 32 + l32) * cpitch + (wm * BI + i) * 32 + 4 * half + 8 * g) = s;
         }
     }
 }
@@ -316,113 +325,153 @@ __global__ void __launch_bounds__(256) proj_prep_kernel(ProjPrepArgs a) {
 
 // ------------------------------------------------------------ GEMM
 
+// TM x TN output tile per workgroup of 4 waves (2 x 2), 8 (4 x 2) at TM = 256,
+// k in steps of 64 through two LDS stages.  What bounds it is the way of the
+// operands: a call this short has few tiles, each of which walks all of k, and
+// a step's MFMAs (128 to 512 cycles) are far shorter than the ~1 us a load
+// takes.  So the loads of PF steps are in flight at once, in a ring of
+// registers (no address or count of loads depends on the step: a step past the
+// last one reads past the buffer, zeros without memory traffic).
 // WQ8: Q8_0 weights (else F16).  MODE: kProjQKV or kProjResidual.
-template <bool WQ8, int MODE>
-__global__ void __launch_bounds__(256) proj_gemm_kernel(ProjArgs a) {
+template <bool WQ8, int MODE, int TM, int TN, int PF>
+__global__ void __launch_bounds__(TM == 256 ? 512 : 256, 2) proj_gemm_kernel(ProjArgs a) {
+    static_assert(PF % 2 == 0, "a step's LDS stage is its place in the ring modulo 2");
+    constexpr int NT = TM == 256 ? 512 : 256;
+    constexpr int WM = NT / 128;                       // waves along the features (two along the tokens)
+    constexpr int BI = TM / 32 / WM, BJ = TN / 64;     // 32 x 32 blocks per wave
+    constexpr int CP = TM + 4;                         // floats per token row of the epilogue tile
+    constexpr int OPA = TM * kPitch, STAGE = (TM + TN) * kPitch;
+    constexpr int NA = TM * 8 / NT, NB = TN * 8 / NT;         // 16-byte chunks of a step per thread
+    constexpr int RING = 2 * STAGE > TN * CP * 4 + 16 ? 2 * STAGE : TN * CP * 4 + 16;
     prefetch_kernargs<sizeof(ProjArgs)>();
-    __shared__ __attribute__((aligned(16))) char lds[2 * kStage];
+    __shared__ __attribute__((aligned(16))) char lds[RING];
 
     const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, l32 = lane & 31;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = w & 1, wn = w >> 1;             // the wave's 64 x 64 quadrant
+    const int wm = w % WM, wn = w / WM;
 
-    // Workgroup i runs on XCD i % 8; XCD x takes the contiguous run of tiles
-    // [x * q + min(x, r), ...) of its c_x = q + (x < r) workgroups.
-    const int n_mt = a.M / kTM, n_nt = (a.N + kTN - 1) / kTN;
-    const int ksplit = a.ksplit, tail0 = a.tail0;
-    int mt, nt, ks = 0, tile = 0;                             // tile: its ticket and partials
-    if (ksplit > 1 && tail0 == 0) {
-        // every tile split along K: the order walks (k piece, weight tile,
-        // token tile), token tiles innermost, so that the workgroups an XCD
-        // runs together share one weight slice in its L2
-        const int q = gridDim.x / 8, r = gridDim.x % 8, x = blockIdx.x % 8;
-        const int wo = x * q + min(x, r) + (int)blockIdx.x / 8;
-        ks = wo / (n_nt * n_mt);
-        mt = (wo / n_nt) % n_mt;
-        nt = wo % n_nt;
-        tile = mt * n_nt + nt;
-    } else if (ksplit > 1 && (int)blockIdx.x >= tail0) {
-        // the last round's tiles, split along K (after the unsplit ones)
-        const int qq = (int)blockIdx.x - tail0, wo = tail0 + qq / ksplit;
-        ks = qq % ksplit;
-        tile = qq / ksplit;
-        mt = wo % n_mt;
-        nt = wo / n_mt;
-    } else {
-        const int hp = ksplit > 1 ? tail0 : (int)gridDim.x;
-        const int q = hp / 8, r = hp % 8, x = blockIdx.x % 8;
-        const int wo = x * q + min(x, r) + (int)blockIdx.x / 8;   // the XCD's contiguous run of the order
-        mt = wo % n_mt;
-        nt = wo / n_mt;
-    }
-    const bool split = ksplit > 1 && (tail0 == 0 || (int)blockIdx.x >= tail0);
-    const int m0 = mt * kTM, n0 = nt * kTN;
+    // Workgroup i runs on XCD i % 8; XCD x takes a contiguous run of the
+    // order (k piece, weight tile, token tile), token tiles innermost: the
+    // weights, the larger operand of a call this short, go to one L2 each.
+    const int n_mt = a.M / TM, n_nt = (a.N + TN - 1) / TN, ksplit = a.ksplit;
+    const int gq = gridDim.x / 8, gr = gridDim.x % 8, gx = blockIdx.x % 8;
+    const int wo = gx * gq + min(gx, gr) + (int)blockIdx.x / 8;
+    const int ks = wo / (n_nt * n_mt), tile = wo - ks * n_nt * n_mt;
+    const int mt = tile / n_nt, nt = tile - mt * n_nt;
+    // 64 features of a 128-dim head are two runs of 32, whose dims rotate together
+    const bool halves = MODE == kProjQKV && TM < a.d;
+    const int m0 = halves ? (mt >> 1) * 128 : mt * TM, n0 = nt * TN;
+    const int c0 = halves ? (mt & 1) * 32 : 0;
     const int mat = m0 < a.m_end[0] ? 0 : (m0 < a.m_end[1] ? 1 : 2);
     const int mrow0 = m0 - (mat ? a.m_end[mat - 1] : 0);     // first row in its matrix
-    const char* wbase = a.w[mat] + (int64_t)mrow0 * a.w_nb[mat];
     const int64_t wnb = a.w_nb[mat];
 
     // x rows past N read as zeros through the buffer range
-    const __amdgpu_buffer_rsrc_t xrs = rsrc(a.xh + (int64_t)n0 * a.K, (uint32_t)(min(a.N - n0, kTN) * a.K * 2));
-    const __amdgpu_buffer_rsrc_t wrs = rsrc(wbase, (uint32_t)(kTM * wnb));
+    const __amdgpu_buffer_rsrc_t xrs = rsrc(a.xh + (int64_t)n0 * a.K, (uint32_t)(min(a.N - n0, TN) * a.K * 2));
+    const __amdgpu_buffer_rsrc_t wrs = rsrc(a.w[mat] + (int64_t)mrow0 * wnb, (uint32_t)((halves ? 128 : TM) * wnb));
     const int nk_all = a.K / kTK;
-    const int nsp = split ? ksplit : 1;
-    const int k_lo = ks * nk_all / nsp;
-    const int nk = (ks + 1) * nk_all / nsp - k_lo;
+    const int k_lo = ks * nk_all / ksplit;
+    const int nk = (ks + 1) * nk_all / ksplit - k_lo;
+    constexpr uint32_t kPast = 0x80000000u;                  // past every range (they stay below 2 GiB)
+    auto slot = [](int row, int c) { return row * kPitch + c * 16; };
+    auto wrow = [&](int r) { return halves ? c0 + r + (r & 32) : r; };
 
-    // per thread and k step: 4 x 16 bytes of B (and of an F16 A): chunk c =
-    // tid + 256 i is row c / 8, 16-byte column c % 8
-    u32x4 breg[4], areg[4];
-    uint32_t qreg[9];
-    auto load = [&](int kt) {
+    // per thread and step: 16-byte chunks c = tid + NT i of B (and of an F16
+    // A), row c / 8, column c % 8.  Q8_0 A, 128 or 256 rows: block tid % 2 of row
+    // tid / 2, 9 dwords from the 4-byte boundary at or below it (the block of
+    // an odd index starts 2 bytes in; an even one's 9th dword is the next
+    // block's scale, always inside the row).  64 rows: 16 codes, half tid % 2
+    // of block tid / 2 % 2 of row tid / 4: 4 dwords from the boundary below
+    // them, a fifth where they start 2 bytes in, and the scale's.
+    uint32_t aoff[WQ8 ? 1 : NA], boff[NB];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int c = tid + 256 * i, row = c >> 3, col = c & 7;
-            breg[i] = __builtin_amdgcn_raw_buffer_load_b128(xrs, (row * a.K + (k_lo + kt) * kTK) * 2 + col * 16, 0, 0);
+    for (int i = 0; i < NB; ++i) {
+        const int c = tid + NT * i;
+        boff[i] = (uint32_t)((c >> 3) * a.K + k_lo * kTK) * 2 + (c & 7) * 16;
+    }
+    if constexpr (!WQ8) {
+#pragma unroll
+        for (int i = 0; i < NA; ++i) {
+            const int c = tid + NT * i;
+            aoff[i] = (uint32_t)(wrow(c >> 3) * wnb) + k_lo * kTK * 2 + (c & 7) * 16;
         }
+    } else {
+        const int row = TM >= 128 ? tid >> 1 : tid >> 2, blk = TM >= 128 ? tid & 1 : (tid >> 1) & 1;
+        aoff[0] = (uint32_t)(wrow(row) * wnb) + (uint32_t)(k_lo * 2 + blk) * kQ8Bytes;
+    }
+    struct Step {
+        u32x4 b[NB];
+        u32x4 a[WQ8 ? (TM >= 128 ? 2 : 1) : NA];
+        uint32_t q, sc;                                // Q8_0: the last dword; (64 rows) the scale's
+    } ring[PF];
+    auto load = [&](Step& s, int kt) {
+        const bool live = kt < nk;
+#pragma unroll
+        for (int i = 0; i < NB; ++i)
+            s.b[i] = __builtin_amdgcn_raw_buffer_load_b128(xrs, live ? boff[i] + kt * kTK * 2 : kPast, 0, 0);
         if constexpr (!WQ8) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int c = tid + 256 * i, row = c >> 3, col = c & 7;
-                areg[i] = __builtin_amdgcn_raw_buffer_load_b128(wrs, (uint32_t)(row * wnb) + (k_lo + kt) * kTK * 2 + col * 16, 0, 0);
-            }
+            for (int i = 0; i < NA; ++i)
+                s.a[i] = __builtin_amdgcn_raw_buffer_load_b128(wrs, live ? aoff[i] + kt * kTK * 2 : kPast, 0, 0);
         } else {
-            // block kt * 2 + (tid & 1) of row tid / 2: 34 bytes from the
-            // 4-byte boundary at or below it (9 dwords; the block of an odd
-            // index starts 2 bytes in, an even one's 9th dword is the next
-            // block's scale, always inside the row)
-            const uint32_t off = (uint32_t)((tid >> 1) * wnb) + (uint32_t)((k_lo + kt) * 2 + (tid & 1)) * kQ8Bytes;
-#pragma unroll
-            for (int i = 0; i < 9; ++i) qreg[i] = __builtin_amdgcn_raw_buffer_load_b32(wrs, (off & ~3u) + 4 * i, 0, 0);
+            const uint32_t off = live ? aoff[0] + kt * 2 * kQ8Bytes : kPast;
+            if constexpr (TM >= 128) {
+                s.a[0] = __builtin_amdgcn_raw_buffer_load_b128(wrs, off & ~3u, 0, 0);
+                s.a[1] = __builtin_amdgcn_raw_buffer_load_b128(wrs, (off & ~3u) + 16, 0, 0);
+                s.q = __builtin_amdgcn_raw_buffer_load_b32(wrs, (off & ~3u) + 32, 0, 0);
+            } else {
+                const uint32_t co = off + 2 + (tid & 1) * 16;
+                s.a[0] = __builtin_amdgcn_raw_buffer_load_b128(wrs, co & ~3u, 0, 0);
+                s.q = __builtin_amdgcn_raw_buffer_load_b32(wrs, co & 2 ? (co & ~3u) + 16 : co, 0, 0);
+                s.sc = __builtin_amdgcn_raw_buffer_load_b32(wrs, off & ~3u, 0, 0);
+            }
         }
     };
-    auto store = [&](int st) {
-        char* sa = lds + st * kStage;
-        char* sb = sa + kOpBytes;
+    auto store = [&](Step& s, int st) {
+        // (nothing of a step's values is computed before this: it would wait for the load)
+        if constexpr (WQ8) asm("" : "+v"(s.q), "+v"(s.sc));
+        char* sa = lds + st * STAGE;
+        char* sb = sa + OPA;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int c = tid + 256 * i, row = c >> 3, col = c & 7;
-            *(u32x4*)(sb + row * kPitch + col * 16) = breg[i];
+        for (int i = 0; i < NB; ++i) {
+            const int c = tid + NT * i;
+            *(u32x4*)(sb + slot(c >> 3, c & 7)) = s.b[i];
         }
         if constexpr (!WQ8) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int c = tid + 256 * i, row = c >> 3, col = c & 7;
-                *(u32x4*)(sa + row * kPitch + col * 16) = areg[i];
+            for (int i = 0; i < NA; ++i) {
+                const int c = tid + NT * i;
+                *(u32x4*)(sa + slot(c >> 3, c & 7)) = s.a[i];
             }
         } else {
-            const bool odd = tid & 1;                  // the block starts 2 bytes into dword 0
-            const uint32_t dbits = odd ? (qreg[0] >> 16) : (qreg[0] & 0xffffu);
+            // block index odd: it starts 2 bytes into its dword, its codes on
+            // a dword; even: the other way round
+            constexpr int NC = TM >= 128 ? 8 : 4;      // dwords of codes per thread
+            const bool odd = TM >= 128 ? tid & 1 : tid & 2;
+            uint32_t qr[NC + 1], codes[NC];
+            uint32_t dbits;
+            if constexpr (TM >= 128) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) qr[i] = s.a[i / 4][i % 4];
+                qr[8] = s.q;
+                dbits = odd ? (qr[0] >> 16) : (qr[0] & 0xffffu);
+#pragma unroll
+                for (int i = 0; i < 8; ++i) codes[i] = odd ? qr[i + 1] : __builtin_amdgcn_alignbyte(qr[i + 1], qr[i], 2);
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) qr[i] = s.a[0][i];
+                qr[4] = s.q;
+                dbits = odd ? (s.sc >> 16) : (s.sc & 0xffffu);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) codes[i] = odd ? qr[i] : __builtin_amdgcn_alignbyte(qr[i + 1], qr[i], 2);
+            }
             _Float16 dh;
             const uint16_t d16 = (uint16_t)dbits;
             __builtin_memcpy(&dh, &d16, 2);
             const h2 dd = {dh, dh};
-            uint32_t codes[8];                         // the 32 codes, 4 per dword
+            uint32_t outw[2 * NC];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) codes[i] = odd ? qreg[i + 1] : __builtin_amdgcn_alignbyte(qreg[i + 1], qreg[i], 2);
-            uint32_t outw[16];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
+            for (int i = 0; i < NC; ++i) {
                 const uint32_t c = codes[i];
                 const h2 lo = {(_Float16)(int8_t)(c & 0xff), (_Float16)(int8_t)((c >> 8) & 0xff)};
                 const h2 hi = {(_Float16)(int8_t)((c >> 16) & 0xff), (_Float16)(int8_t)(c >> 24)};
@@ -430,67 +479,85 @@ __global__ void __launch_bounds__(256) proj_gemm_kernel(ProjArgs a) {
                 __builtin_memcpy(&outw[2 * i], &plo, 4);
                 __builtin_memcpy(&outw[2 * i + 1], &phi, 4);
             }
-            char* dst = sa + (tid >> 1) * kPitch + (tid & 1) * 64;
+            const int row = TM >= 128 ? tid >> 1 : tid >> 2, sl = TM >= 128 ? (tid & 1) * 4 : (tid & 3) * 2;
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-                *(u32x4*)(dst + 16 * i) = u32x4{outw[4 * i], outw[4 * i + 1], outw[4 * i + 2], outw[4 * i + 3]};
+            for (int i = 0; i < NC / 2; ++i)
+                *(u32x4*)(sa + slot(row, sl + i)) = u32x4{outw[4 * i], outw[4 * i + 1], outw[4 * i + 2], outw[4 * i + 3]};
         }
     };
 
-    f32x16 acc[2][2];
+    f32x16 acc[BI][BJ];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < BI; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = f32x16{};
-
-    load(0);
-    store(0);
-    if (nk > 1) load(1);
-    __syncthreads();
+        for (int j = 0; j < BJ; ++j) acc[i][j] = f32x16{};
     // fragment offsets within a stage: row l32 of each 32-row block, the
     // lane's 8-element k group
-    const int a_rd = (wm * 64 + l32) * kPitch + half * 16;
-    const int b_rd = kOpBytes + (wn * 64 + l32) * kPitch + half * 16;
-    for (int kt = 0; kt < nk; ++kt) {
-        const char* st = lds + (kt & 1) * kStage;
+    const int a_rd = slot(wm * BI * 32 + l32, half), b_rd = OPA + slot(wn * BJ * 32 + l32, half);
+
+    // (in this order: the waits of the loop count the loads that came later)
 #pragma unroll
-        for (int ks = 0; ks < kTK / 16; ++ks) {
-            h8 af[2], bf[2];
+    for (int u = 0; u < PF; ++u) {
+        load(ring[u], u);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    store(ring[0], 0);
+    __builtin_amdgcn_sched_barrier(0);
+    load(ring[0], PF);
+    __syncthreads();
+    // step kt of place u in the ring
+    auto step = [&](int kt, int u, bool more) {
+        const char* st = lds + (u & 1) * STAGE;
 #pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const u32x4 ua = *(const u32x4*)(st + a_rd + i * 32 * kPitch + ks * 32);
-                const u32x4 ub = *(const u32x4*)(st + b_rd + i * 32 * kPitch + ks * 32);
+        for (int kk = 0; kk < kTK / 16; ++kk) {
+            h8 af[BI], bf[BJ];
+#pragma unroll
+            for (int i = 0; i < BI; ++i) {
+                const u32x4 ua = *(const u32x4*)(st + a_rd + i * 32 * kPitch + kk * 32);
                 __builtin_memcpy(&af[i], &ua, 16);
-                __builtin_memcpy(&bf[i], &ub, 16);
             }
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
+            for (int j = 0; j < BJ; ++j) {
+                const u32x4 ub = *(const u32x4*)(st + b_rd + j * 32 * kPitch + kk * 32);
+                __builtin_memcpy(&bf[j], &ub, 16);
+            }
 #pragma unroll
-                for (int j = 0; j < 2; ++j)
+            for (int i = 0; i < BI; ++i)
+#pragma unroll
+                for (int j = 0; j < BJ; ++j)
                     acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i], bf[j], acc[i][j], 0, 0, 0);
         }
-        if (kt + 1 < nk) {
-            store((kt + 1) & 1);      // that stage held tile kt - 1: every wave is past it
-            if (kt + 2 < nk) load(kt + 2);
-        }
+        // the other stage held step kt - 1: every wave is past it
+        store(ring[(u + 1) % PF], (u + 1) & 1);
+        if (more) load(ring[(u + 1) % PF], kt + 1 + PF);
         __syncthreads();
+    };
+    // whole turns of the ring without a branch, then the rest (an exit within
+    // a turn would make every wait of the next one count for the worst case)
+    int kt = 0;
+    for (; kt + PF <= nk; kt += PF) {
+#pragma unroll
+        for (int u = 0; u < PF; ++u) step(kt + u, u, true);
     }
+#pragma unroll
+    for (int u = 0; u < PF - 1; ++u)
+        if (kt + u < nk) step(kt + u, u, false);       // uniform; every step's loads are out
 
     // ---- accumulators to LDS as C[token][feature]: lane (half, l32) of
     // block (i, j) holds features 8 (r / 4) + 4 half + r % 4 of token l32
     // (split along K: the tile's last piece sums every piece's partial there)
     float* C = (float*)lds;
-    if (split) {
-        constexpr int PIECE = 4 * 4096 * 4;
-        splitk_store<4>(acc, a.part + ((int64_t)tile * ksplit + ks) * PIECE, w, lane);
-        if (!splitk_ticket(a.tickets + tile, ksplit, (int*)(lds + 2 * kStage - 16))) return;
-        splitk_sum<4, 256, 2, 8>(a.part + (int64_t)tile * ksplit * PIECE, ksplit, C, kCPitch);
+    if (ksplit > 1) {
+        constexpr int PIECE = TM * TN * 4, NF = TM * TN / 4 / NT;
+        splitk_store<NT / 64>(acc, a.part + ((int64_t)tile * ksplit + ks) * PIECE, w, lane);
+        if (!splitk_ticket(a.tickets + tile, ksplit, (int*)(lds + RING - 16))) return;
+        splitk_sum<NT / 64, NT, WM, BI, BJ, NF < 8 ? NF : 8>(a.part + (int64_t)tile * ksplit * PIECE, ksplit, C, CP);
     } else {
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < BI; ++i)
 #pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                float* crow = C + (wn * 64 + 32 * j + l32) * kCPitch + wm * 64 + 32 * i + 4 * half;
+            for (int j = 0; j < BJ; ++j) {
+                float* crow = C + ((wn * BJ + j) * 32 + l32) * CP + (wm * BI + i) * 32 + 4 * half;
 #pragma unroll
                 for (int g = 0; g < 4; ++g)
                     *(float4*)(crow + 8 * g) = make_float4(acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2],
@@ -501,112 +568,87 @@ __global__ void __launch_bounds__(256) proj_gemm_kernel(ProjArgs a) {
 
     if constexpr (MODE == kProjQKV) {
         if (a.vec_store) {
-            qkv_epilogue_vec<kTM, kTN, 256>(a, C, kCPitch, m0, n0, tid);
+            qkv_epilogue_vec<TM, TN, NT>(a, C, CP, m0, n0, tid, c0);
             return;
         }
-        // 64 rotation pairs per token (one head of d = 128, two of d = 64):
-        // thread (token tid / 64 + 4 pass, pair tid % 64)
-        const int d = a.d, P = d >> 1;
-        const int pi = tid & 63, hl = pi / P, i = pi - hl * P;
-        const int head = (mrow0 + hl * d) / d;
+        // TM / 2 rotation pairs per token: pair tid % (TM / 2) of the tile is
+        // pair i of its head; 32 consecutive threads hold the pairs of two
+        // whole 32-dim blocks of one token
+        constexpr int NP = TM / 2, TPP = NT / NP;      // tokens per pass
+        const int d = a.d, P = d >> 1, dl = min(d, TM), Pl = dl >> 1;
+        const int pi = tid % NP, hl = pi / Pl, li = pi - hl * Pl, i = c0 + li;
+        const int head = (mrow0 + hl * dl) / d;
         const float* bias = a.bias[mat];
-        const float b0 = bias ? bias[mrow0 + hl * d + i] : 0.0f;
-        const float b1 = bias ? bias[mrow0 + hl * d + i + P] : 0.0f;
+        const float b0 = bias ? bias[head * d + i] : 0.0f;
+        const float b1 = bias ? bias[head * d + i + P] : 0.0f;
         // the batch's RoPE pairs loaded first (one memory round trip per batch)
-        for (int nb = tid >> 6; nb < kTN; nb += 4 * kEpiQkv) {
+        for (int nb = tid / NP; nb < TN; nb += TPP * kEpiQkv) {
             float2 csb[kEpiQkv];
 #pragma unroll
             for (int e = 0; e < kEpiQkv; ++e)
-                csb[e] = a.rope[(int64_t)min(n0 + nb + 4 * e, a.N - 1) * P + i];      // used for q and k only
+                csb[e] = a.rope[(int64_t)min(n0 + nb + TPP * e, a.N - 1) * P + i];    // used for q and k only
 #pragma unroll
             for (int e = 0; e < kEpiQkv; ++e) {
-            const int nl = nb + 4 * e;
-            const int n = n0 + nl;
-            if (nl >= kTN || n >= a.N) break;              // wave-uniform
-            float y0 = C[nl * kCPitch + hl * d + i] + b0;
-            float y1 = C[nl * kCPitch + hl * d + i + P] + b1;
-            if (mat < 2) {
-                const float2 cs = csb[e];
-                const float r0 = fmaf(y0, cs.x, -(y1 * cs.y));
-                const float r1 = fmaf(y0, cs.y, y1 * cs.x);
-                y0 = r0;
-                y1 = r1;
-            }
-            const int b = a.N == a.T ? 0 : n / a.T, t = n - b * a.T;
-            if (mat == 0) {
-                const int64_t eo = type_elem_bytes(a.q_out_type);
-                char* dst = a.q_out + b * a.qo_nb_b + t * a.qo_nb_t + head * a.qo_nb_h;
-                store_elem(dst + i * eo, a.q_out_type, y0);
-                store_elem(dst + (i + P) * eo, a.q_out_type, y1);
-            } else {
-                // (one sequence: constant indices, no indexed kernel-argument load per pass)
-                char* const kd = a.N == a.T ? a.k_dst[0] : a.k_dst[b];
-                char* const vd = a.N == a.T ? a.v_dst[0] : a.v_dst[b];
-                char* row = (mat == 1 ? kd : vd) + t * a.cache_row_bytes + head * a.cache_head_bytes;
-                if (a.cache_type == VVA_TYPE_Q8_0) {
-                    store_q8_pair(row, i, P, y0, y1);
-                } else {
-                    const int64_t ec = type_elem_bytes(a.cache_type);
-                    store_elem(row + i * ec, a.cache_type, y0);
-                    store_elem(row + (i + P) * ec, a.cache_type, y1);
+                const int nl = nb + TPP * e;
+                const int n = n0 + nl;
+                if (nl >= TN || n >= a.N) break;       // uniform per 32 lanes
+                float y0 = C[nl * CP + hl * dl + li] + b0;
+                float y1 = C[nl * CP + hl * dl + li + Pl] + b1;
+                if (mat < 2) {
+                    const float2 cs = csb[e];
+                    const float r0 = fmaf(y0, cs.x, -(y1 * cs.y));
+                    const float r1 = fmaf(y0, cs.y, y1 * cs.x);
+                    y0 = r0;
+                    y1 = r1;
                 }
-            }
+                const int b = a.N == a.T ? 0 : n / a.T, t = n - b * a.T;
+                if (mat == 0) {
+                    const int64_t eo = type_elem_bytes(a.q_out_type);
+                    char* dst = a.q_out + b * a.qo_nb_b + t * a.qo_nb_t + head * a.qo_nb_h;
+                    store_elem(dst + i * eo, a.q_out_type, y0);
+                    store_elem(dst + (i + P) * eo, a.q_out_type, y1);
+                } else {
+                    // (one sequence: constant indices, no indexed kernel-argument load per pass)
+                    char* const kd = a.N == a.T ? a.k_dst[0] : a.k_dst[b];
+                    char* const vd = a.N == a.T ? a.v_dst[0] : a.v_dst[b];
+                    char* row = (mat == 1 ? kd : vd) + t * a.cache_row_bytes + head * a.cache_head_bytes;
+                    if (a.cache_type == VVA_TYPE_Q8_0) {
+                        store_q8_pair(row, i, P, y0, y1);
+                    } else {
+                        const int64_t ec = type_elem_bytes(a.cache_type);
+                        store_elem(row + i * ec, a.cache_type, y0);
+                        store_elem(row + (i + P) * ec, a.cache_type, y1);
+                    }
+                }
             }
         }
     } else {
-        // h = y + x, 4 features per thread: thread (token tid / 32 + 8 pass,
-        // features 4 (tid % 32) ..)
-        const int c4 = (tid & 31) * 4;
+        // h = y + x, 4 features per thread
+        constexpr int TPP = NT / (TM / 4);             // tokens per pass
+        const int c4 = tid % (TM / 4) * 4;
         // the batch's residual rows loaded first (one memory round trip per batch)
-        for (int nb = tid >> 5; nb < kTN; nb += 8 * kEpiRes) {
+        for (int nb = tid / (TM / 4); nb < TN; nb += TPP * kEpiRes) {
             float4 xrb[kEpiRes];
 #pragma unroll
             for (int e = 0; e < kEpiRes; ++e) {
-                const int n = min(n0 + nb + 8 * e, a.N - 1);
+                const int n = min(n0 + nb + TPP * e, a.N - 1);
                 const int b = a.N == a.T ? 0 : n / a.T, t = n - b * a.T;
                 xrb[e] = *(const float4*)(a.res + b * a.res_nb_b + t * a.res_nb_t + (int64_t)(m0 + c4) * 4);
             }
 #pragma unroll
             for (int e = 0; e < kEpiRes; ++e) {
-                const int nl = nb + 8 * e;
+                const int nl = nb + TPP * e;
                 const int n = n0 + nl;
-                if (nl >= kTN || n >= a.N) break;
+                if (nl >= TN || n >= a.N) break;
                 const int b = a.N == a.T ? 0 : n / a.T, t = n - b * a.T;
                 const float4 xr = xrb[e];
-                const float* cr = C + nl * kCPitch + c4;
+                const float* cr = C + nl * CP + c4;
                 *(float4*)(a.h + b * a.h_nb_b + t * a.h_nb_t + (int64_t)(m0 + c4) * 4) =
                     make_float4(cr[0] + xr.x, cr[1] + xr.y, cr[2] + xr.z, cr[3] + xr.w);
             }
         }
     }
 }
-
-// ------------------------------------------------------------ wide GEMM (F16 weights)
-
-// 256 output features x 128 token rows per workgroup, k in steps of 64.
-// Eight producer waves DMA the tiles straight into a 3-stage LDS ring
-// (buffer_load_dwordx4 ... lds).  From L2 one wave's LDS loads stream at
-// ~20 GB/s whatever their number in flight, so eight issuing waves are what
-// a CU needs to feed its matrix cores (~110 GB/s at this tile shape); the
-// compute waves issue none, so they never wait behind a full load queue.
-// Eight compute waves, two per SIMD, each own a 64 x 64 quadrant of 2 x 2
-// v_mfma_f32_32x32x16_f16 blocks.  Rows are 128 bytes (64 f16 of k) in LDS;
-// a DMA instruction fills 8 rows, and its lane l writes LDS 16-byte slot
-// l % 8 of row l / 8 with the row's 16-byte k chunk (l % 8) ^ sw(row),
-// sw(row) = (row / 2) % 8: a fragment read (16 lanes x 16 bytes per LDS
-// cycle, rows r .. r + 15 at one k chunk) then touches every bank once.
-constexpr int kWM = 256, kWN = 128, kWK = 64;
-constexpr int kWStages = 3;
-constexpr int kWA = kWM * kWK * 2;             // 32 KB of weights per stage
-constexpr int kWB = kWN * kWK * 2;             // 16 KB of token rows per stage
-constexpr int kWStage = kWA + kWB;
-constexpr int kWCompute = 8, kWProd = 8;
-constexpr int kWLoadsA = kWA / 1024 / kWProd;  // DMA loads per producer and stage
-constexpr int kWLoadsB = kWB / 1024 / kWProd;
-constexpr int kWLoads = kWLoadsA + kWLoadsB;
-constexpr int kWCPitch = kWM + 4;              // floats per token row of the epilogue tile
-static_assert(2 * kWLoads <= 63, "two stages of a producer's loads fit its 6-bit vmcnt");
-static_assert(kWN * kWCPitch * 4 + 16 <= kWStages * kWStage, "the epilogue tile (and the split ticket flag) reuse the ring");
 
 __device__ __forceinline__ void wdma16(i32x4 rsrc, uint32_t lds_addr, int voffset) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
@@ -618,257 +660,6 @@ template <int N>
 __device__ __forceinline__ void wwait_barrier() {
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(N) : "memory");
 }
-__device__ __forceinline__ void wlds_barrier() {
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : : : "memory");
-}
-
-template <int MODE>
-__global__ void __launch_bounds__((kWCompute + kWProd) * 64) proj_gemm_wide_kernel(ProjArgs a) {
-    prefetch_kernargs<sizeof(ProjArgs)>();
-    __shared__ __attribute__((aligned(16))) char lds[kWStages * kWStage];
-    const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, l32 = lane & 31;
-    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-
-    // Workgroup i runs on XCD i % 8; XCD x takes the contiguous run of tiles
-    // [x * q + min(x, r), ...) of an order that walks groups of 4 token
-    // tiles, the 4 token tiles of every weight tile in turn: the tiles an
-    // XCD runs at one time share few weight and token rows in its L2.
-    const int n_mt = (a.M + kWM - 1) / kWM, n_nt = (a.N + kWN - 1) / kWN;
-    const int ksplit = a.ksplit, tail0 = a.tail0;
-    int mt, nt, ks = 0, tile = 0;                             // tile: its ticket and partials
-    auto order = [&](int wo) {
-        const int grp = wo / (n_mt * 4), gn = min(4, n_nt - grp * 4), j = wo - grp * n_mt * 4;
-        mt = j / gn;
-        nt = grp * 4 + j % gn;
-    };
-    if (ksplit > 1 && tail0 == 0) {
-        // every tile split along K: the order walks (k piece, weight tile,
-        // token tile), token tiles innermost, so that the workgroups an XCD
-        // runs together share one weight slice in its L2
-        const int q = gridDim.x / 8, r = gridDim.x % 8, x = blockIdx.x % 8;
-        const int wo = x * q + min(x, r) + (int)blockIdx.x / 8;
-        nt = wo % n_nt;
-        mt = (wo / n_nt) % n_mt;
-        ks = wo / (n_nt * n_mt);
-        tile = mt * n_nt + nt;
-    } else if (ksplit > 1 && (int)blockIdx.x >= tail0) {
-        // the last round's tiles, split along K (after the unsplit ones)
-        const int qq = (int)blockIdx.x - tail0;
-        order(tail0 + qq / ksplit);
-        ks = qq % ksplit;
-        tile = qq / ksplit;
-    } else {
-        const int hp = ksplit > 1 ? tail0 : (int)gridDim.x;
-        const int q = hp / 8, r = hp % 8, x = blockIdx.x % 8;
-        order(x * q + min(x, r) + (int)blockIdx.x / 8);      // the XCD's contiguous run of the order
-    }
-    const bool split = ksplit > 1 && (tail0 == 0 || (int)blockIdx.x >= tail0);
-    const int m0 = mt * kWM, n0 = nt * kWN;
-    const int nk_all = a.K / kWK;
-    const int nsp = split ? ksplit : 1;
-    const int k_lo = ks * nk_all / nsp;
-    const int nk = (ks + 1) * nk_all / nsp - k_lo;
-    constexpr int PIECE = kWCompute * 4096 * 4;
-    int* const split_flag = (int*)(lds + kWStages * kWStage - 16);
-    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
-
-    if (w >= kWCompute) {
-        // ---- producers: chunks p, p + 2, ... of each operand's stage
-        const int pw = w - kWCompute;
-        const int sub = lane >> 3, slot = lane & 7;
-        int aoff[kWLoadsA], boff[kWLoadsB];
-        i32x4 ars[kWLoadsA];
-#pragma unroll
-        for (int i = 0; i < kWLoadsA; ++i) {
-            const int row = (pw + kWProd * i) * 8 + sub;            // tile row of this lane
-            const int g = m0 + (pw + kWProd * i) * 8;               // its 8-row group (one matrix)
-            const int mat = g < a.m_end[0] ? 0 : (g < a.m_end[1] ? 1 : (g < a.m_end[2] ? 2 : 3));
-            const int mbeg = mat == 0 ? 0 : a.m_end[mat - 1];
-            const int mrows = mat < 3 ? a.m_end[mat] - mbeg : 0;
-            ars[i] = make_rsrc_sgpr(mat < 3 ? a.w[mat] : a.w[0], (uint32_t)(mrows * a.w_nb[mat < 3 ? mat : 0]));
-            const int mr = m0 + row - mbeg;
-            aoff[i] = mr * (int)a.w_nb[mat < 3 ? mat : 0] + (((slot ^ ((row >> 1) & 7))) << 4);
-        }
-        const int nrows = min(a.N - n0, kWN);
-        const i32x4 brs = make_rsrc_sgpr((const char*)(a.xh + (int64_t)n0 * a.K), (uint32_t)(nrows * a.K * 2));
-#pragma unroll
-        for (int i = 0; i < kWLoadsB; ++i) {
-            const int row = (pw + kWProd * i) * 8 + sub;
-            boff[i] = row * a.K * 2 + (((slot ^ ((row >> 1) & 7))) << 4);
-        }
-        // a stage past the last loads zeros (offsets past every range)
-        auto issue = [&](int kt) {
-            const uint32_t st = lds0 + (uint32_t)(kt % kWStages) * kWStage;
-            const bool live = kt < nk;
-            const int ko = (k_lo + kt) * kWK * 2;
-#pragma unroll
-            for (int i = 0; i < kWLoadsA; ++i)
-                wdma16(ars[i], st + (pw + kWProd * i) * 1024, live ? aoff[i] + ko : 0x40000000);
-#pragma unroll
-            for (int i = 0; i < kWLoadsB; ++i)
-                wdma16(brs, st + kWA + (pw + kWProd * i) * 1024, live ? boff[i] + ko : 0x40000000);
-        };
-        issue(0);
-        issue(1);
-        for (int kt = 0; kt < nk; ++kt) {
-            wwait_barrier<kWLoads>();                      // T_kt: stage kt landed
-            issue(kt + 2);                                 // into the stage of kt - 1
-        }
-        asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
-        __syncthreads();                                   // every wave is done with the ring
-        if (split) {
-            if (!splitk_ticket(a.tickets + tile, ksplit, split_flag)) return;
-            splitk_sum<kWCompute, (kWCompute + kWProd) * 64, 4, 4>(a.part + (int64_t)tile * ksplit * PIECE, ksplit,
-                                                                 (float*)lds, kWCPitch);
-        }
-        __syncthreads();                                   // the epilogue tile is written
-        return;
-    }
-
-    // ---- compute waves: quadrant (wm, wn) of 64 features x 64 tokens
-    const int wm = w & 3, wn = w >> 2;
-    const int sw = (l32 >> 1) & 7;
-    const int a_rd = (wm * 64 + l32) * 128;
-    const int b_rd = kWA + (wn * 64 + l32) * 128;
-    f32x16 acc[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = f32x16{};
-    for (int kt = 0; kt < nk; ++kt) {
-        wlds_barrier();                                    // T_kt
-        const char* st = lds + (kt % kWStages) * kWStage;
-#pragma unroll
-        for (int ks = 0; ks < kWK / 16; ++ks) {
-            const int ch = ((2 * ks + half) ^ sw) << 4;
-            h8 af[2], bf[2];
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const u32x4 ua = *(const u32x4*)(st + a_rd + i * 32 * 128 + ch);
-                const u32x4 ub = *(const u32x4*)(st + b_rd + i * 32 * 128 + ch);
-                __builtin_memcpy(&af[i], &ua, 16);
-                __builtin_memcpy(&bf[i], &ub, 16);
-            }
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i], bf[j], acc[i][j], 0, 0, 0);
-        }
-    }
-    __syncthreads();                                       // every wave is done with the ring
-
-    // ---- accumulators to LDS as C[token][feature]: lane (half, l32) of
-    // block (i, j) holds features 8 (r / 4) + 4 half + r % 4 of token l32
-    // (split along K: the tile's last piece sums every piece's partial there,
-    // with the producer waves)
-    float* C = (float*)lds;
-    if (split) {
-        splitk_store<kWCompute>(acc, a.part + ((int64_t)tile * ksplit + ks) * PIECE, w, lane);
-        if (!splitk_ticket(a.tickets + tile, ksplit, split_flag)) return;
-        splitk_sum<kWCompute, (kWCompute + kWProd) * 64, 4, 4>(a.part + (int64_t)tile * ksplit * PIECE, ksplit, C,
-                                                             kWCPitch);
-    } else {
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                float* crow = C + (wn * 64 + 32 * j + l32) * kWCPitch + wm * 64 + 32 * i + 4 * half;
-#pragma unroll
-                for (int g = 0; g < 4; ++g)
-                    *(float4*)(crow + 8 * g) = make_float4(acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2],
-                                                           acc[i][j][4 * g + 3]);
-            }
-    }
-    __syncthreads();
-
-    if constexpr (MODE == kProjQKV) {
-        if (a.vec_store) {
-            if (tid < kWCompute * 64) qkv_epilogue_vec<kWM, kWN, kWCompute * 64>(a, C, kWCPitch, m0, n0, tid);
-            return;
-        }
-        // 128 rotation pairs per token (two heads of d = 128, four of d = 64):
-        // thread (token tid / 128 + 4 pass, pair tid % 128)
-        const int d = a.d, P = d >> 1;
-        const int pi = tid & 127, hl = pi / P, i = pi - hl * P;
-        const int f0 = m0 + hl * d;                        // first feature of the head
-        if (f0 >= a.M) return;                             // past the last matrix (uniform per half-wave)
-        const int mat = f0 < a.m_end[0] ? 0 : (f0 < a.m_end[1] ? 1 : 2);
-        const int mrow = f0 - (mat ? a.m_end[mat - 1] : 0);
-        const int head = mrow / d;
-        const float* bias = a.bias[mat];
-        const float b0 = bias ? bias[mrow + i] : 0.0f;
-        const float b1 = bias ? bias[mrow + i + P] : 0.0f;
-        // the batch's RoPE pairs loaded first (one memory round trip per batch)
-        constexpr int PS = kWCompute * 64 / 128;          // token stride between passes
-        for (int nb = tid >> 7; nb < kWN; nb += PS * kEpiQkv) {
-            float2 csb[kEpiQkv];
-#pragma unroll
-            for (int e = 0; e < kEpiQkv; ++e)
-                csb[e] = a.rope[(int64_t)min(n0 + nb + PS * e, a.N - 1) * P + i];     // used for q and k only
-#pragma unroll
-            for (int e = 0; e < kEpiQkv; ++e) {
-            const int nl = nb + PS * e;
-            const int n = n0 + nl;
-            if (nl >= kWN || n >= a.N) break;              // uniform per wave
-            float y0 = C[nl * kWCPitch + hl * d + i] + b0;
-            float y1 = C[nl * kWCPitch + hl * d + i + P] + b1;
-            if (mat < 2) {
-                const float2 cs = csb[e];
-                const float r0 = fmaf(y0, cs.x, -(y1 * cs.y));
-                const float r1 = fmaf(y0, cs.y, y1 * cs.x);
-                y0 = r0;
-                y1 = r1;
-            }
-            const int b = a.N == a.T ? 0 : n / a.T, t = n - b * a.T;
-            if (mat == 0) {
-                const int64_t eo = type_elem_bytes(a.q_out_type);
-                char* dst = a.q_out + b * a.qo_nb_b + t * a.qo_nb_t + head * a.qo_nb_h;
-                store_elem(dst + i * eo, a.q_out_type, y0);
-                store_elem(dst + (i + P) * eo, a.q_out_type, y1);
-            } else {
-                // (one sequence: constant indices, no indexed kernel-argument load per pass)
-                char* const kd = a.N == a.T ? a.k_dst[0] : a.k_dst[b];
-                char* const vd = a.N == a.T ? a.v_dst[0] : a.v_dst[b];
-                char* row = (mat == 1 ? kd : vd) + t * a.cache_row_bytes + head * a.cache_head_bytes;
-                if (a.cache_type == VVA_TYPE_Q8_0) {
-                    store_q8_pair(row, i, P, y0, y1);
-                } else {
-                    const int64_t ec = type_elem_bytes(a.cache_type);
-                    store_elem(row + i * ec, a.cache_type, y0);
-                    store_elem(row + (i + P) * ec, a.cache_type, y1);
-                }
-            }
-            }
-        }
-    } else {
-        // h = y + x, 4 features per thread: thread (token tid / 64 + 8 pass,
-        // features 4 (tid % 64) ..)
-        const int c4 = (tid & 63) * 4;
-        if (m0 + c4 >= a.M) return;
-        // the batch's residual rows loaded first (one memory round trip per batch)
-        for (int nb = tid >> 6; nb < kWN; nb += kWCompute * kEpiRes) {
-            float4 xrb[kEpiRes];
-#pragma unroll
-            for (int e = 0; e < kEpiRes; ++e) {
-                const int n = min(n0 + nb + kWCompute * e, a.N - 1);
-                const int b = a.N == a.T ? 0 : n / a.T, t = n - b * a.T;
-                xrb[e] = *(const float4*)(a.res + b * a.res_nb_b + t * a.res_nb_t + (int64_t)(m0 + c4) * 4);
-            }
-#pragma unroll
-            for (int e = 0; e < kEpiRes; ++e) {
-                const int nl = nb + kWCompute * e;
-                const int n = n0 + nl;
-                if (nl >= kWN || n >= a.N) break;
-                const int b = a.N == a.T ? 0 : n / a.T, t = n - b * a.T;
-                const float4 xr = xrb[e];
-                const float* cr = C + nl * kWCPitch + c4;
-                *(float4*)(a.h + b * a.h_nb_b + t * a.h_nb_t + (int64_t)(m0 + c4) * 4) =
-                    make_float4(cr[0] + xr.x, cr[1] + xr.y, cr[2] + xr.z, cr[3] + xr.w);
-            }
-        }
-    }
-}
 
 // ------------------------------------------------------------ big GEMM (F16 weights, long calls)
 
@@ -876,12 +667,12 @@ __global__ void __launch_bounds__((kWCompute + kWProd) * 64) proj_gemm_wide_kern
 // waves (two per SIMD), each a 128 x 64 block of 4 x 2
 // v_mfma_f32_32x32x16_f16 blocks whose 128 accumulators live in AGPRs: per
 // k16 step a wave reads 6 fragments (6 KB of LDS) for 8 MFMAs, 3/4 of the LDS
-// reads per MFMA of the wide kernel's 64 x 64 quadrants, whose fragment
+// reads per MFMA of 64 x 64 quadrants, whose fragment
 // reads and DMA writes kept LDS saturated.  The waves DMA the tiles into a
 // 2-stage LDS ring themselves (buffer_load_dwordx4 ... lds, 8 loads per wave
 // and stage): eight issuing waves, since one wave's LDS loads stream at
-// ~20 GB/s.  Rows are 128 bytes (64 f16 of k) in LDS, laid out as the
-// wide kernel's: a DMA instruction fills 8 rows, lane l writing 16-byte slot
+// ~20 GB/s.  Rows are 128 bytes (64 f16 of k) in LDS: a DMA
+// instruction fills 8 rows, lane l writing 16-byte slot
 // l % 8 of row l / 8 with the row's k chunk (l % 8) ^ ((row / 2) % 8), so a
 // fragment read (16 lanes, rows r .. r + 15 at one k chunk) touches every
 // bank once.  Step kt: the MFMAs of each k16 quarter run while the next
@@ -908,7 +699,7 @@ constexpr int kBCBytes = kBHalf * kBCPitch * 4;
 constexpr int kBLds = kBRing > kBCBytes ? kBRing : kBCBytes;
 constexpr int kBPiece = kBWaves * 8 * 4096;     // bytes of one K piece's accumulators (256 x 256 f32)
 constexpr int kBMaxSplit = 8;
-constexpr int kBigMinRows = 1024;             // token rows from which the big GEMM runs (shorter: the wide one measured faster)
+constexpr int kBigMinRows = 1024;             // fewest token rows of a big GEMM (gemm_plan)
 static_assert(kBStages == 2 && kBStages * kBLoads <= 63, "two stages of a wave's loads fit its 6-bit vmcnt");
 static_assert(kBLds <= 160 * 1024, "LDS");
 
@@ -1028,7 +819,7 @@ proj_gemm_big_kernel(ProjArgs a) {
     const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, l32 = lane & 31;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
 
-    // Tile order as in the wide kernel: XCD x (workgroup i runs on XCD i % 8)
+    // Tile order: XCD x (workgroup i runs on XCD i % 8)
     // takes a contiguous run of an order that walks groups of 4 token tiles,
     // the 4 token tiles of every weight tile in turn.
     const int n_mt = (a.M + kBM - 1) / kBM, n_nt = (a.N + kBN - 1) / kBN;
@@ -2402,55 +2193,85 @@ hipError_t launch_proj_gemv(ProjArgs& a, float* y_ws, int n_cu, hipStream_t s) {
     return hipGetLastError();
 }
 
-// The GEMM's tiles against the workgroups resident at once (one wide F16
-// workgroup per CU, two of the 128 x 128 kernel): a call whose tiles fill
-// at most half of them (short chunks, e.g. 512 tokens) is split along K, at
-// least 4 k steps per piece, up to 4 pieces, one round.
 namespace {
-// F16 weights over at least kBigMinRows token rows take the big kernel (256 x 256
-// tiles); shorter calls the wide one (256 x 128), whose split pieces are half
-// the size
-bool proj_big(const ProjArgs& a) { return a.w_type != VVA_TYPE_Q8_0 && a.N >= kBigMinRows; }
+constexpr int kDqMaxK = 8192;                  // inputs of a Q8_0 row that proj_dequant_q8_kernel holds
+// Kernel, tile and K pieces of a call: the least of the estimates (us)
+//   steps x workgroups per CU x time of a step + cost of exchanging the pieces.
+// The times of a step are measured ones (0.5B, 1.5B and 7B shapes, 16 to 4096
+// token rows), of a workgroup that has its CU to itself and of one of several
+// on it; between one and 1.6 workgroups per CU the fuller CUs set the time.
+// Pieces are for calls whose workgroups are all resident at once.  At the
+// choices that fall out (us of the whole call, prep included; the kernel that
+// runs against the next best one): q/k/v 0.5B, 257 rows 13.8 (64 x 64) against
+// 17.3 (64 x 128); 7B, 64 rows 18.8 (3 pieces) against 25.3 (one); 7B, 512 rows
+// 45.6 (128 x 128, 3 pieces) against 50.4 (64 x 64); 7B output, 1024 rows 48.1
+// (128 x 128) against 53.4 (the big kernel); 7B q/k/v, 1024 rows 69.5 (256 x
+// 128) against 80.7 (64 x 128) and 112 (the big kernel); 7B q/k/v, 3000 rows
+// 132 (the big kernel) against 151 (256 x 128); 1.5B q/k/v, 4096 rows 57.5
+// (256 x 128) against 76.1 (the big kernel, whose 128 tiles leave half the CUs
+// idle).  What sets the larger tiles' steps is the operands' way from L2:
+// ~9 TB/s over the chip, at every tile size.
+struct GemmPlan { int tm, tn, ks; };
+GemmPlan gemm_plan(const ProjArgs& a, int n_cu, bool allow_big) {
+    struct Tile { int tm, tn; double lone, shared, merge; };
+    static const Tile kF16[] = {{64, 64, 0.27, 0.33, 2.5}, {64, 128, 0.45, 0.55, 4.0}, {128, 128, 0.85, 0.85, 9.0},
+                                {256, 128, 1.20, 1.20, 0.0}};
+    static const Tile kQ8[] = {{64, 64, 0.33, 0.40, 2.5}, {64, 128, 0.50, 0.62, 4.0}, {128, 128, 0.95, 0.95, 9.0},
+                               {256, 128, 1.35, 1.35, 0.0}};
+    const bool q8 = a.w_type == VVA_TYPE_Q8_0;
+    const int nk = a.K / kTK;
+    GemmPlan best{64, 64, 1};
+    double best_us = 1e30;
+    // a tile lies in one matrix (every matrix has a multiple of 128 rows); 256
+    // rows never came first below kBigMinRows token rows, nor in pieces
+    const bool m256 = a.N >= kBigMinRows && a.M % 256 == 0 && a.m_end[0] % 256 == 0 && a.m_end[1] % 256 == 0;
+    for (const Tile& t : q8 ? kQ8 : kF16) {
+        if (t.tm == 256 && !m256) continue;
+        const int64_t tiles = (int64_t)(a.M / t.tm) * ((a.N + t.tn - 1) / t.tn);
+        for (int ks = 1; ks <= 4; ++ks) {
+            if (ks > 1 && (t.tm == 256 || tiles > kMaxProjTickets || tiles * ks > 2 * n_cu || nk < 4 * ks)) break;
+            double x = (double)(tiles * ks) / n_cu;
+            if (t.tm == 256) x = std::ceil(x);                 // one workgroup per CU
+            const double us = (double)nk / ks * (x <= 1.0 ? t.lone : std::max(1.6, x) * t.shared) + (ks > 1 ? t.merge : 0.0);
+            if (us < best_us) {
+                best_us = us;
+                best = GemmPlan{t.tm, t.tn, ks};
+            }
+        }
+    }
+    // the big kernel: 1.45 us a step and 25 us around them, whatever the share
+    // of the CUs that its tiles fill; Q8_0 weights are dequantized for it first
+    if (allow_big && a.N >= kBigMinRows && !(q8 && a.K > kDqMaxK)) {
+        const int64_t tiles = (int64_t)((a.M + kBM - 1) / kBM) * ((a.N + kBN - 1) / kBN);
+        const int64_t tail = tiles % n_cu;
+        const double rounds = (double)(tiles / n_cu) + (tail == 0 ? 0.0 : (tiles > n_cu && 4 * tail <= n_cu) ? 0.6 : 1.0);
+        const double us = rounds * (25.0 + 1.45 * nk) + (q8 ? 2.0 + (double)a.M * a.K * 6.4e-7 : 0.0);
+        if (us < best_us) best = GemmPlan{kBM, kBN, 1};
+    }
+    return best;
+}
+bool proj_big(const ProjArgs& a, int n_cu) { return gemm_plan(a, n_cu, true).tn == kBN; }
 }  // namespace
 
 int proj_ksplit(const ProjArgs& a, int n_cu, int* tail0) {
-    const bool q8 = a.w_type == VVA_TYPE_Q8_0;
-    if (proj_big(a)) {
-        // the last round's tiles, when they fill at most a quarter of the CUs,
-        // split along K (at most kBMaxSplit pieces of at least 8 k steps)
-        const int tiles = ((a.M + kBM - 1) / kBM) * ((a.N + kBN - 1) / kBN);
-        const int nk = a.K / kBK, r = tiles % n_cu;
-        *tail0 = 0;
-        if (r == 0 || 4 * r > n_cu || r > kMaxProjTickets || nk < 16) return 1;
-        *tail0 = tiles - r;
-        return max(1, min(min(kBMaxSplit, n_cu / r), nk / 8));
-    }
-    const int tiles = q8 ? (a.M / kTM) * ((a.N + kTN - 1) / kTN) : ((a.M + kWM - 1) / kWM) * ((a.N + kWN - 1) / kWN);
-    const int slots = q8 ? 2 * n_cu : n_cu;
-    const int nk = a.K / (q8 ? kTK : kWK);
     *tail0 = 0;
-    if (tiles < 1 || nk < 8) return 1;
-    if (2 * tiles <= slots) {                          // every tile: one round
-        if (tiles > kMaxProjTickets) return 1;
-        return max(1, min(min(4, slots / tiles), nk / 4));
-    }
-    // the last round's tiles when they fill at most a quarter of the slots
-    const int r = tiles % slots;
-    if (r == 0 || 4 * r > slots || r > kMaxProjTickets) return 1;
+    if (!proj_big(a, n_cu)) return gemm_plan(a, n_cu, false).ks;
+    // the last round's tiles, when they fill at most a quarter of the CUs,
+    // split along K (at most kBMaxSplit pieces of at least 8 k steps)
+    const int tiles = ((a.M + kBM - 1) / kBM) * ((a.N + kBN - 1) / kBN);
+    const int nk = a.K / kBK, r = tiles % n_cu;
+    if (r == 0 || 4 * r > n_cu || r > kMaxProjTickets || nk < 16) return 1;
     *tail0 = tiles - r;
-    return max(1, min(min(4, slots / r), nk / 4));
+    return max(1, min(min(kBMaxSplit, n_cu / r), nk / 8));
 }
-size_t proj_part_bytes(const ProjArgs& a) {
+size_t proj_part_bytes(const ProjArgs& a, int n_cu) {
     if (a.ksplit <= 1) return 0;
-    if (proj_big(a)) {
+    if (proj_big(a, n_cu)) {
         const size_t tiles = (size_t)((a.M + kBM - 1) / kBM) * ((a.N + kBN - 1) / kBN);
         return (tiles - a.tail0) * a.ksplit * kBPiece;
     }
-    const bool q8 = a.w_type == VVA_TYPE_Q8_0;
-    const size_t tiles = q8 ? (size_t)(a.M / kTM) * ((a.N + kTN - 1) / kTN)
-                            : (size_t)((a.M + kWM - 1) / kWM) * ((a.N + kWN - 1) / kWN);
-    const size_t split = a.tail0 > 0 ? tiles - a.tail0 : tiles;
-    return split * a.ksplit * (q8 ? 4 : kWCompute) * 4096 * sizeof(float);
+    const GemmPlan t = gemm_plan(a, n_cu, false);
+    return (size_t)(a.M / t.tm) * ((a.N + t.tn - 1) / t.tn) * a.ksplit * t.tm * t.tn * sizeof(float);
 }
 
 // Q8_0 weight rows dequantized to f16 rows of d * q: the products the Q8_0
@@ -2461,7 +2282,6 @@ size_t proj_part_bytes(const ProjArgs& a) {
 // row, so a dword past it reads as zero), then thread t converts the 8
 // codes t % 4 of block t / 4 and stores their 16 bytes, so that every store
 // instruction writes 1 KB of the row contiguously.
-constexpr int kDqMaxK = 8192;
 constexpr int kDqThreads = 256;
 __global__ void __launch_bounds__(kDqThreads) proj_dequant_q8_kernel(ProjArgs a, uint16_t* dst) {
     __shared__ uint32_t rowbuf[kDqMaxK / 32 * kQ8Bytes / 4 + 4];
@@ -2504,7 +2324,7 @@ __global__ void __launch_bounds__(kDqThreads) proj_dequant_q8_kernel(ProjArgs a,
     }
 }
 
-bool proj_dequant_q8(const ProjArgs& a) { return a.w_type == VVA_TYPE_Q8_0 && a.N >= kBigMinRows && a.K <= kDqMaxK; }
+bool proj_dequant_q8(const ProjArgs& a, int n_cu) { return a.w_type == VVA_TYPE_Q8_0 && proj_big(a, n_cu); }
 
 hipError_t launch_proj_dequant_q8(const ProjArgs& a, uint16_t* dst, hipStream_t s) {
     hipLaunchKernelGGL(proj_dequant_q8_kernel, dim3((unsigned)a.M), dim3(kDqThreads), 0, s, a, dst);
@@ -2516,7 +2336,23 @@ size_t proj_ws_bytes(int N, int K, int P) {
     return xh + (size_t)N * P * sizeof(float2);
 }
 
-hipError_t launch_proj(ProjPrepArgs& p, ProjArgs& a, void* ws, hipStream_t s) {
+namespace {
+template <int MODE>
+void launch_gemm(const ProjArgs& a, const GemmPlan& t, dim3 g, hipStream_t s) {
+    const bool q8 = a.w_type == VVA_TYPE_Q8_0;
+    const dim3 b(t.tm == 256 ? 512 : 256);
+#define VVA_GEMM(TM, TN, PF)                                                                                   \
+    if (q8) hipLaunchKernelGGL((proj_gemm_kernel<true, MODE, TM, TN, PF>), g, b, 0, s, a);                     \
+    else    hipLaunchKernelGGL((proj_gemm_kernel<false, MODE, TM, TN, PF>), g, b, 0, s, a)
+    if (t.tm == 64 && t.tn == 64) { VVA_GEMM(64, 64, 6); }
+    else if (t.tm == 64) { VVA_GEMM(64, 128, 4); }
+    else if (t.tm == 128) { VVA_GEMM(128, 128, 4); }
+    else { VVA_GEMM(256, 128, 4); }
+#undef VVA_GEMM
+}
+}  // namespace
+
+hipError_t launch_proj(ProjPrepArgs& p, ProjArgs& a, void* ws, int n_cu, hipStream_t s) {
     p.xh = (uint16_t*)ws;
     p.rope = p.P > 0 ? (float2*)((char*)ws + ((size_t)p.N * p.K * 2 + 255) / 256 * 256) : nullptr;
     a.xh = p.xh;
@@ -2524,14 +2360,13 @@ hipError_t launch_proj(ProjPrepArgs& p, ProjArgs& a, void* ws, hipStream_t s) {
     hipLaunchKernelGGL(proj_prep_kernel, dim3(p.N), dim3(256), 0, s, p);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    const bool q8 = a.w_type == VVA_TYPE_Q8_0;
     if (a.ksplit < 1 || !a.part || !a.tickets) {
         a.ksplit = 1;
         a.tail0 = 0;
     }
     // every tile's pieces, or the unsplit tiles then the split tail's pieces
     auto grid = [&](int tiles) { return a.tail0 > 0 ? a.tail0 + (tiles - a.tail0) * a.ksplit : tiles * a.ksplit; };
-    if (proj_big(a)) {
+    if (proj_big(a, n_cu)) {
         const int tiles = ((a.M + kBM - 1) / kBM) * ((a.N + kBN - 1) / kBN);
         const dim3 g(grid(tiles)), b(kBWaves * 64);
         if (a.mode == kProjQKV) hipLaunchKernelGGL((proj_gemm_big_kernel<kProjQKV>), g, b, 0, s, a);
@@ -2542,18 +2377,10 @@ hipError_t launch_proj(ProjPrepArgs& p, ProjArgs& a, void* ws, hipStream_t s) {
         else                    hipLaunchKernelGGL((proj_big_merge_kernel<kProjResidual>), gm, dim3(256), 0, s, a);
         return hipGetLastError();
     }
-    if (!q8) {
-        const int wtiles = grid(((a.M + kWM - 1) / kWM) * ((a.N + kWN - 1) / kWN));
-        const dim3 block((kWCompute + kWProd) * 64);
-        if (a.mode == kProjQKV) hipLaunchKernelGGL((proj_gemm_wide_kernel<kProjQKV>), dim3(wtiles), block, 0, s, a);
-        else                    hipLaunchKernelGGL((proj_gemm_wide_kernel<kProjResidual>), dim3(wtiles), block, 0, s, a);
-        return hipGetLastError();
-    }
-    // Q8_0 weights below the big-kernel threshold (F16 ones took the wide
-    // kernel above; the 128 x 128 kernel on F16 weights measured no faster)
-    const int tiles = grid((a.M / kTM) * ((a.N + kTN - 1) / kTN));
-    if (a.mode == kProjQKV) hipLaunchKernelGGL((proj_gemm_kernel<true, kProjQKV>), dim3(tiles), dim3(256), 0, s, a);
-    else                    hipLaunchKernelGGL((proj_gemm_kernel<true, kProjResidual>), dim3(tiles), dim3(256), 0, s, a);
+    const GemmPlan t = gemm_plan(a, n_cu, false);
+    const dim3 g((a.M / t.tm) * ((a.N + t.tn - 1) / t.tn) * a.ksplit);
+    if (a.mode == kProjQKV) launch_gemm<kProjQKV>(a, t, g, s);
+    else                    launch_gemm<kProjResidual>(a, t, g, s);
     return hipGetLastError();
 }
 

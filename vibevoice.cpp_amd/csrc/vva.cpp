@@ -1015,14 +1015,14 @@ bool rows16(const vva_tensor* x) {
 // when the GEMM is split along K, the pieces' partials; the split tickets
 // follow the decode step's and the prefill's in the context's ticket buffer.
 static vva_status run_proj_gemm(vva_context* ctx, ProjPrepArgs& p, ProjArgs& a, int N, int K, int P) {
-    const bool dq = proj_dequant_q8(a);
+    const bool dq = proj_dequant_q8(a, ctx->n_cu);
     ProjArgs g = a;                                    // the GEMM's view of the weights
     if (dq) g.w_type = VVA_TYPE_F16;
     g.ksplit = proj_ksplit(g, ctx->n_cu, &g.tail0);
     g.tickets = ctx->tickets + kMaxStepTickets + kMaxPrefillTickets;
     const size_t base = (proj_ws_bytes(N, K, P) + 255) / 256 * 256;
     const size_t wbytes = dq ? ((size_t)a.M * K * 2 + 255) / 256 * 256 : 0;
-    vva_status st = ensure_ws(ctx, base + wbytes + proj_part_bytes(g));
+    vva_status st = ensure_ws(ctx, base + wbytes + proj_part_bytes(g, ctx->n_cu));
     if (st != VVA_OK) return st;
     if (dq) {
         uint16_t* wd = (uint16_t*)((char*)ctx->ws + base);
@@ -1034,7 +1034,7 @@ static vva_status run_proj_gemm(vva_context* ctx, ProjPrepArgs& p, ProjArgs& a, 
         }
     }
     g.part = g.ksplit > 1 ? (char*)ctx->ws + base + wbytes : nullptr;
-    const hipError_t e = launch_proj(p, g, ctx->ws, ctx->stream);
+    const hipError_t e = launch_proj(p, g, ctx->ws, ctx->n_cu, ctx->stream);
     return e == hipSuccess ? VVA_OK : hip_fail(ctx, e, "projection launch");
 }
 

@@ -179,7 +179,7 @@ constexpr int kMaxProjTickets = 1024;
 // K split of the GEMM of a call (1: none; *tail0 > 0: only the last round's
 // tiles) and the bytes of its partials
 int proj_ksplit(const ProjArgs& a, int n_cu, int* tail0);
-size_t proj_part_bytes(const ProjArgs& a);
+size_t proj_part_bytes(const ProjArgs& a, int n_cu);
 
 // --------------------------------------------------------- host launchers
 
@@ -243,11 +243,11 @@ PrefillPlan prefill_plan(const AttnArgs& a, int n_cu, int forced, size_t ws_cap,
 size_t prefill_ws_bytes(const AttnArgs& a, const PrefillPlan& p);
 // Prep + GEMM of a linear layer; ws holds proj_ws_bytes(N, K, P) bytes.
 size_t proj_ws_bytes(int N, int K, int P);
-// Q8_0 weights over a long call (>= 1024 token rows): the rows are
-// dequantized to f16 d * q (M x K) for the F16 GEMM
-bool proj_dequant_q8(const ProjArgs& a);
+// Q8_0 weights over a call that the big F16 GEMM runs: the rows are
+// dequantized to f16 d * q (M x K) for it
+bool proj_dequant_q8(const ProjArgs& a, int n_cu);
 hipError_t launch_proj_dequant_q8(const ProjArgs& a, uint16_t* dst, hipStream_t s);
-hipError_t launch_proj(ProjPrepArgs& p, ProjArgs& a, void* ws, hipStream_t s);
+hipError_t launch_proj(ProjPrepArgs& p, ProjArgs& a, void* ws, int n_cu, hipStream_t s);
 // Few token rows (decode steps): one weight-streaming GEMV launch that
 // converts the rows itself.  kProjQKV writes y = x w^T + bias (F32 [N][M],
 // at `ws`) for the caller's RoPE + append; kProjResidual writes h.
