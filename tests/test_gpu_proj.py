@@ -357,6 +357,9 @@ TILE_CASES = [
     (448, 2, 1, 128, vva.Q8_0, vva.Q8_0, 33, 2),     # 64 features of a 128-dim head, Q8_0 cache (pair epilogue)
     (832, 2, 1, 128, vva.F16, vva.BF16, 63, 1),      # the same, vector epilogue, 13 steps
     (1536, 12, 2, 128, vva.Q8_0, vva.F32, 20, 1),    # 64 x 64 in pieces of k
+    (896, 14, 2, 64, vva.F16, vva.Q8_0, 130, 1),     # two token rows past the second tile
+    (1536, 12, 2, 128, vva.F16, vva.F16, 37, 3),     # pieces of k, three sequences
+    (64, 2, 2, 64, vva.F16, vva.F32, 10, 1),         # F16 x
     (3584, 28, 4, 128, vva.F16, vva.Q8_0, 31, 2),    # the same, pair epilogue
     (320, 14, 2, 64, vva.Q8_0, vva.F16, 1400, 1),    # 64 x 128
     (640, 28, 4, 128, vva.F16, vva.Q8_0, 385, 1),    # 64 x 128 or 64 x 64, ragged token tile, pair epilogue
@@ -374,18 +377,26 @@ def test_gemm_tiles_match_oracle(ctx, torch_gpu, hidden, Hq, Hkv, d, wt, ct, T, 
     """Every tile of the GEMM at its edges: k shorter than the loads in flight,
     remainders of k and of the token rows, heads cut in two, pieces of k.  The
     first and last 96 token rows of every sequence match the oracle, q_out's
-    other rows are finite, and the output projection of the same rows does."""
+    other rows are finite, and the output projection of the same rows does.
+    x comes as F32, F16 or BF16 (the 64 x 64 tiles of F16 weights read it
+    themselves), and once with rows at odd strides."""
     torch = torch_gpu
     print(f"gemm tiles hidden={hidden} Hq={Hq} Hkv={Hkv} d={d} w={wt} cache={ct} T={T} B={B}", flush=True)
     rng = np.random.default_rng(hidden + T + wt)
     kv = vva.KVCache(ctx, 1, Hkv, d, T + 8, B, ct)
-    x = rng.standard_normal((B, T, hidden)).astype(np.float32)
+    xt = (vva.F32, vva.F16, vva.BF16)[T % 3]
+    pad = 8 if T % 2 else 2                             # row strides of whole and of broken 16-byte units
+
+    def rows_of(a):
+        g = to_gpu(torch, np.concatenate([a, np.zeros((B, T, pad), np.float32)], -1), xt)[..., :a.shape[-1]]
+        return g, as_f32(torch, g.contiguous())        # on the device, and the values there
+    xg, x = rows_of(rng.standard_normal((B, T, hidden)).astype(np.float32))
     raws, ws = zip(*[_weight(torch, rng, n * d, hidden, wt) for n in (Hq, Hkv, Hkv)])
     bias = [(rng.standard_normal(n * d) * 0.5).astype(np.float32) for n in (Hq, Hkv, Hkv)]
     pos = np.tile(np.arange(3, 3 + T, dtype=np.int32), (B, 1))
     q_out = torch.full((B, T, Hq, d), float("nan"), dtype=torch.float32, device="cuda")
     gb = [torch.from_numpy(b).cuda() for b in bias]
-    ctx.qkv_rope_append(kv, 0, torch.from_numpy(x).cuda(), *ws, torch.from_numpy(pos).cuda(), q_out,
+    ctx.qkv_rope_append(kv, 0, xg, *ws, torch.from_numpy(pos).cuda(), q_out,
                         bq=gb[0], bk=gb[1], bv=gb[2])
     torch.cuda.synchronize()
     got = as_f32(torch, q_out)
@@ -404,10 +415,10 @@ def test_gemm_tiles_match_oracle(ctx, torch_gpu, hidden, Hq, Hkv, d, wt, ct, T, 
     # the output projection: in = Hq d, out a multiple of 128
     hid = (hidden + 127) // 128 * 128
     wo_raw, wo = _weight(torch, rng, hid, Hq * d, wt)
-    o = rng.standard_normal((B, T, Hq * d)).astype(np.float32)
+    og, o = rows_of(rng.standard_normal((B, T, Hq * d)).astype(np.float32))
     res = rng.standard_normal((B, T, hid)).astype(np.float32)
     h = torch.full((B, T, hid), float("nan"), dtype=torch.float32, device="cuda")
-    ctx.out_proj_residual(torch.from_numpy(o).cuda(), wo, torch.from_numpy(res).cuda(), h)
+    ctx.out_proj_residual(og, wo, torch.from_numpy(res).cuda(), h)
     torch.cuda.synchronize()
     got = as_f32(torch, h)
     assert np.isfinite(got).all()

@@ -333,8 +333,15 @@ __global__ void __launch_bounds__(256) proj_prep_kernel(ProjPrepArgs a) {
 // registers (no address or count of loads depends on the step: a step past the
 // last one reads past the buffer, zeros without memory traffic).
 // WQ8: Q8_0 weights (else F16).  MODE: kProjQKV or kProjResidual.
-template <bool WQ8, int MODE, int TM, int TN, int PF>
+// XB: 0, the prep kernel's f16 rows; 2 or 4 (output projection, F16 weights),
+// the token rows themselves (F16 / BF16 or F32), rounded to f16 as they are
+// staged: no prep launch, 3 of the 10 us of a short call (0.5B, 64 rows 9.0 ->
+// 7.0; 1.5B, 257 rows 12.0 -> 10.5).  The q/k/v call keeps it: its RoPE pairs,
+// computed in each of its weight tiles, took longer than the launch (0.5B, 257
+// rows 13.8 -> 19.3), and so would quantizing a row in each for Q8_0 weights.
+template <bool WQ8, int MODE, int TM, int TN, int PF, int XB>
 __global__ void __launch_bounds__(TM == 256 ? 512 : 256, 2) proj_gemm_kernel(ProjArgs a) {
+    static_assert(XB == 0 || (!WQ8 && MODE == kProjResidual && TM == 64 && TN == 64), "see XB");
     static_assert(PF % 2 == 0, "a step's LDS stage is its place in the ring modulo 2");
     constexpr int NT = TM == 256 ? 512 : 256;
     constexpr int WM = NT / 128;                       // waves along the features (two along the tokens)
@@ -366,8 +373,10 @@ __global__ void __launch_bounds__(TM == 256 ? 512 : 256, 2) proj_gemm_kernel(Pro
     const int mrow0 = m0 - (mat ? a.m_end[mat - 1] : 0);     // first row in its matrix
     const int64_t wnb = a.w_nb[mat];
 
-    // x rows past N read as zeros through the buffer range
-    const __amdgpu_buffer_rsrc_t xrs = rsrc(a.xh + (int64_t)n0 * a.K, (uint32_t)(min(a.N - n0, TN) * a.K * 2));
+    // x rows past N read as zeros: past the buffer range
+    const __amdgpu_buffer_rsrc_t xrs =
+        XB ? rsrc(a.x, (uint32_t)((a.N / a.T - 1) * a.x_nb_b + (a.T - 1) * a.x_nb_t) + (uint32_t)a.K * XB)
+           : rsrc(a.xh + (int64_t)n0 * a.K, (uint32_t)(min(a.N - n0, TN) * a.K * 2));
     const __amdgpu_buffer_rsrc_t wrs = rsrc(a.w[mat] + (int64_t)mrow0 * wnb, (uint32_t)((halves ? 128 : TM) * wnb));
     const int nk_all = a.K / kTK;
     const int k_lo = ks * nk_all / ksplit;
@@ -387,7 +396,13 @@ __global__ void __launch_bounds__(TM == 256 ? 512 : 256, 2) proj_gemm_kernel(Pro
 #pragma unroll
     for (int i = 0; i < NB; ++i) {
         const int c = tid + NT * i;
-        boff[i] = (uint32_t)((c >> 3) * a.K + k_lo * kTK) * 2 + (c & 7) * 16;
+        if constexpr (XB) {
+            const int n = n0 + (c >> 3), b = n / a.T;
+            boff[i] = n < a.N ? (uint32_t)(b * a.x_nb_b + (n - b * a.T) * a.x_nb_t) + (uint32_t)(k_lo * kTK + (c & 7) * 8) * XB
+                              : kPast;
+        } else {
+            boff[i] = (uint32_t)((c >> 3) * a.K + k_lo * kTK) * 2 + (c & 7) * 16;
+        }
     }
     if constexpr (!WQ8) {
 #pragma unroll
@@ -400,15 +415,18 @@ __global__ void __launch_bounds__(TM == 256 ? 512 : 256, 2) proj_gemm_kernel(Pro
         aoff[0] = (uint32_t)(wrow(row) * wnb) + (uint32_t)(k_lo * 2 + blk) * kQ8Bytes;
     }
     struct Step {
-        u32x4 b[NB];
+        u32x4 b[XB == 4 ? 2 * NB : NB];
         u32x4 a[WQ8 ? (TM >= 128 ? 2 : 1) : NA];
         uint32_t q, sc;                                // Q8_0: the last dword; (64 rows) the scale's
     } ring[PF];
     auto load = [&](Step& s, int kt) {
         const bool live = kt < nk;
 #pragma unroll
-        for (int i = 0; i < NB; ++i)
-            s.b[i] = __builtin_amdgcn_raw_buffer_load_b128(xrs, live ? boff[i] + kt * kTK * 2 : kPast, 0, 0);
+        for (int i = 0; i < NB; ++i) {
+            const uint32_t off = live ? boff[i] + kt * kTK * (XB ? XB : 2) : kPast;
+            s.b[i] = __builtin_amdgcn_raw_buffer_load_b128(xrs, off, 0, 0);
+            if constexpr (XB == 4) s.b[NB + i] = __builtin_amdgcn_raw_buffer_load_b128(xrs, off + 16, 0, 0);
+        }
         if constexpr (!WQ8) {
 #pragma unroll
             for (int i = 0; i < NA; ++i)
@@ -435,7 +453,21 @@ __global__ void __launch_bounds__(TM == 256 ? 512 : 256, 2) proj_gemm_kernel(Pro
 #pragma unroll
         for (int i = 0; i < NB; ++i) {
             const int c = tid + NT * i;
-            *(u32x4*)(sb + slot(c >> 3, c & 7)) = s.b[i];
+            u32x4 v = s.b[i];
+            if constexpr (XB == 4) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const u32x4 f = e < 2 ? s.b[i] : s.b[NB + i];
+                    v[e] = (uint32_t)f32_to_f16(__uint_as_float(f[2 * e & 3])) |
+                           ((uint32_t)f32_to_f16(__uint_as_float(f[(2 * e & 3) + 1])) << 16);
+                }
+            } else if (XB == 2 && a.x_type == VVA_TYPE_BF16) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    v[e] = (uint32_t)f32_to_f16(__uint_as_float(v[e] << 16)) |
+                           ((uint32_t)f32_to_f16(__uint_as_float(v[e] & 0xffff0000u)) << 16);
+            }
+            *(u32x4*)(sb + slot(c >> 3, c & 7)) = v;
         }
         if constexpr (!WQ8) {
 #pragma unroll
@@ -2232,7 +2264,8 @@ GemmPlan gemm_plan(const ProjArgs& a, int n_cu, bool allow_big) {
             if (ks > 1 && (t.tm == 256 || tiles > kMaxProjTickets || tiles * ks > 2 * n_cu || nk < 4 * ks)) break;
             double x = (double)(tiles * ks) / n_cu;
             if (t.tm == 256) x = std::ceil(x);                 // one workgroup per CU
-            const double us = (double)nk / ks * (x <= 1.0 ? t.lone : std::max(1.6, x) * t.shared) + (ks > 1 ? t.merge : 0.0);
+            double us = (double)nk / ks * (x <= 1.0 ? t.lone : std::max(1.6, x) * t.shared) + (ks > 1 ? t.merge : 0.0);
+            if (t.tn == 64 && a.direct) us -= 3.5;    // no prep launch
             if (us < best_us) {
                 best_us = us;
                 best = GemmPlan{t.tm, t.tn, ks};
@@ -2250,8 +2283,20 @@ GemmPlan gemm_plan(const ProjArgs& a, int n_cu, bool allow_big) {
     }
     return best;
 }
+bool proj_direct(const ProjArgs& a, int n_cu) {
+    const GemmPlan t = gemm_plan(a, n_cu, true);
+    return t.tm == 64 && t.tn == 64 && a.direct;
+}
 bool proj_big(const ProjArgs& a, int n_cu) { return gemm_plan(a, n_cu, true).tn == kBN; }
 }  // namespace
+
+// the output projection, F16 weights, 16-byte aligned rows within 32-bit offsets
+bool proj_direct_ok(const ProjArgs& a) {
+    return a.mode == kProjResidual && a.w_type == VVA_TYPE_F16 && (uintptr_t)a.x % 16 == 0 && a.x_nb_t % 16 == 0 && a.x_nb_b % 16 == 0 &&
+           a.x_nb_t >= 0 && a.x_nb_b >= 0 &&
+           (a.N / a.T - 1) * a.x_nb_b + (a.T - 1) * a.x_nb_t + (int64_t)a.K * 4 < ((int64_t)1 << 31);
+}
+bool proj_needs_prep(const ProjArgs& a, int n_cu) { return !proj_direct(a, n_cu); }
 
 int proj_ksplit(const ProjArgs& a, int n_cu, int* tail0) {
     *tail0 = 0;
@@ -2342,8 +2387,15 @@ void launch_gemm(const ProjArgs& a, const GemmPlan& t, dim3 g, hipStream_t s) {
     const bool q8 = a.w_type == VVA_TYPE_Q8_0;
     const dim3 b(t.tm == 256 ? 512 : 256);
 #define VVA_GEMM(TM, TN, PF)                                                                                   \
-    if (q8) hipLaunchKernelGGL((proj_gemm_kernel<true, MODE, TM, TN, PF>), g, b, 0, s, a);                     \
-    else    hipLaunchKernelGGL((proj_gemm_kernel<false, MODE, TM, TN, PF>), g, b, 0, s, a)
+    if (q8) hipLaunchKernelGGL((proj_gemm_kernel<true, MODE, TM, TN, PF, 0>), g, b, 0, s, a);                  \
+    else    hipLaunchKernelGGL((proj_gemm_kernel<false, MODE, TM, TN, PF, 0>), g, b, 0, s, a)
+    if constexpr (MODE == kProjResidual) {
+        if (t.tn == 64 && a.direct) {
+            if (a.x_type == VVA_TYPE_F32) hipLaunchKernelGGL((proj_gemm_kernel<false, MODE, 64, 64, 4, 4>), g, b, 0, s, a);
+            else                          hipLaunchKernelGGL((proj_gemm_kernel<false, MODE, 64, 64, 6, 2>), g, b, 0, s, a);
+            return;
+        }
+    }
     if (t.tm == 64 && t.tn == 64) { VVA_GEMM(64, 64, 6); }
     else if (t.tm == 64) { VVA_GEMM(64, 128, 4); }
     else if (t.tm == 128) { VVA_GEMM(128, 128, 4); }
@@ -2353,13 +2405,15 @@ void launch_gemm(const ProjArgs& a, const GemmPlan& t, dim3 g, hipStream_t s) {
 }  // namespace
 
 hipError_t launch_proj(ProjPrepArgs& p, ProjArgs& a, void* ws, int n_cu, hipStream_t s) {
-    p.xh = (uint16_t*)ws;
-    p.rope = p.P > 0 ? (float2*)((char*)ws + ((size_t)p.N * p.K * 2 + 255) / 256 * 256) : nullptr;
-    a.xh = p.xh;
-    a.rope = p.rope;
-    hipLaunchKernelGGL(proj_prep_kernel, dim3(p.N), dim3(256), 0, s, p);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
+    hipError_t e = hipSuccess;
+    if (!proj_direct(a, n_cu)) {
+        p.xh = (uint16_t*)ws;
+        p.rope = p.P > 0 ? (float2*)((char*)ws + ((size_t)p.N * p.K * 2 + 255) / 256 * 256) : nullptr;
+        a.xh = p.xh;
+        a.rope = p.rope;
+        hipLaunchKernelGGL(proj_prep_kernel, dim3(p.N), dim3(256), 0, s, p);
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+    }
     if (a.ksplit < 1 || !a.part || !a.tickets) {
         a.ksplit = 1;
         a.tail0 = 0;

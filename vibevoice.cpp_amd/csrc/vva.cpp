@@ -1017,10 +1017,13 @@ bool rows16(const vva_tensor* x) {
 static vva_status run_proj_gemm(vva_context* ctx, ProjPrepArgs& p, ProjArgs& a, int N, int K, int P) {
     const bool dq = proj_dequant_q8(a, ctx->n_cu);
     ProjArgs g = a;                                    // the GEMM's view of the weights
+    g.x = p.x; g.x_type = p.x_type; g.x_nb_t = p.x_nb_t; g.x_nb_b = p.x_nb_b;
     if (dq) g.w_type = VVA_TYPE_F16;
+    // (dequantized weights meet x in its Q8_0 round trip: the prep's rows)
+    g.direct = !dq && proj_direct_ok(g);
     g.ksplit = proj_ksplit(g, ctx->n_cu, &g.tail0);
     g.tickets = ctx->tickets + kMaxStepTickets + kMaxPrefillTickets;
-    const size_t base = (proj_ws_bytes(N, K, P) + 255) / 256 * 256;
+    const size_t base = proj_needs_prep(g, ctx->n_cu) ? (proj_ws_bytes(N, K, P) + 255) / 256 * 256 : 0;
     const size_t wbytes = dq ? ((size_t)a.M * K * 2 + 255) / 256 * 256 : 0;
     vva_status st = ensure_ws(ctx, base + wbytes + proj_part_bytes(g, ctx->n_cu));
     if (st != VVA_OK) return st;
@@ -1160,8 +1163,7 @@ extern "C" vva_status vva_qkv_rope_append(vva_context* ctx, vva_kv* kv, int laye
         const vva_tensor tq = proj_view(0, Hq), tk = proj_view(Hq * d, Hkv), tv = proj_view((Hq + Hkv) * d, Hkv);
         return vva_rope_append(ctx, kv, layer, &tq, &tk, &tv, pos, seq_ids, freq_base, q_out);
     }
-    if ((st = run_proj_gemm(ctx, p, a, (int)N, (int)K, p.P)) != VVA_OK) return st;
-    return VVA_OK;
+    return run_proj_gemm(ctx, p, a, (int)N, (int)K, p.P);
 }
 
 extern "C" vva_status vva_qkv_proj(vva_context* ctx, const vva_tensor* x, const vva_tensor* wq, const vva_tensor* wk,
