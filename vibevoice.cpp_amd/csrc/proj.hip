@@ -1590,14 +1590,28 @@ hipError_t launch_gemv_f16(const ProjArgs& a, hipStream_t s) {
 // the workgroup goes out first, then its 256 threads quantize the token rows
 // once into LDS (ggml's quantize_row_q8_0, as proj_gemv_kernel does per
 // lane: the same codes and fp16-rounded scales), and each wave takes its 4
-// rows' integer block dots against them.
+// rows' integer block dots against them.  NIT: blocks per lane and row (a
+// lane past the row's blocks would load for nothing).  HALF (rows of at most
+// 32 blocks, which would leave half the lanes idle): lanes 0 .. 31 take the
+// wave's rows 0 and 1, lanes 32 .. 63 its rows 2 and 3.
+// Sum over each half of the wave, in every lane of the half.
+__device__ __forceinline__ float half_sum(float x) {
+    x += dpp<kDppXor1>(x);
+    x += dpp<kDppXor2>(x);
+    x += dpp<kDppHalfMirror>(x);
+    x += dpp<kDppMirror>(x);
+    return add_swap16(x);
+}
 constexpr int kGv8Waves = 4;
 constexpr int kGv8Rows = kGvRows * kGv8Waves;
-template <int MODE>
+template <int MODE, int NIT, bool HALF>
 __global__ void __launch_bounds__(64 * kGv8Waves) proj_gemv_q8_kernel(ProjArgs a) {
     prefetch_kernargs<sizeof(ProjArgs)>();
     __shared__ __attribute__((aligned(16))) uint32_t xq[kGvMaxN][kGvMaxK / 32][8];   // codes of row n, block j
     __shared__ float xd[kGvMaxN][kGvMaxK / 32];         // their fp16-rounded scales
+    constexpr int RL = HALF ? kGvRows / 2 : kGvRows;     // rows per lane
+    constexpr int LPR = HALF ? 32 : 64;                  // lanes per row
+    static_assert(!HALF || NIT == 1, "at most 32 blocks");
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int N = a.N, K = a.K, nbk = K / 32;
     const int m0 = blockIdx.x * kGv8Rows + wv * kGvRows; // matrix boundaries are multiples of 16
@@ -1634,14 +1648,15 @@ __global__ void __launch_bounds__(64 * kGv8Waves) proj_gemv_q8_kernel(ProjArgs a
     }
     // weight block j of each row: 34 bytes from the 4-byte boundary at or
     // below it (rows are 4-byte aligned: K is a multiple of 64)
-    uint32_t qw[kGvQ8It][kGvRows][9];
+    uint32_t qw[NIT][RL][9];
 #pragma unroll
-    for (int it = 0; it < kGvQ8It; ++it) {
-        const int j = lane + 64 * it;
+    for (int it = 0; it < NIT; ++it) {
+        const int j = (lane & (LPR - 1)) + LPR * it;
         const int jj = j < nbk ? j : 0;
 #pragma unroll
-        for (int r = 0; r < kGvRows; ++r) {
-            const uint32_t* p = (const uint32_t*)(wb + ro[r] * wnb + (((int64_t)jj * kQ8Bytes) & ~(int64_t)3));
+        for (int r = 0; r < RL; ++r) {
+            const int row = HALF && lane >= 32 ? ro[(r + 2) % kGvRows] : ro[r];
+            const uint32_t* p = (const uint32_t*)(wb + row * wnb + (((int64_t)jj * kQ8Bytes) & ~(int64_t)3));
 #pragma unroll
             for (int i = 0; i < 9; ++i) qw[it][r][i] = p[i];
         }
@@ -1673,22 +1688,21 @@ __global__ void __launch_bounds__(64 * kGv8Waves) proj_gemv_q8_kernel(ProjArgs a
     }
     __syncthreads();
 
-    float acc[kGvRows][kGvMaxN];
+    float acc[RL][kGvMaxN];
 #pragma unroll
-    for (int r = 0; r < kGvRows; ++r)
+    for (int r = 0; r < RL; ++r)
 #pragma unroll
         for (int n = 0; n < kGvMaxN; ++n) acc[r][n] = 0.0f;
 #pragma unroll
-    for (int it = 0; it < kGvQ8It; ++it) {
-        if (64 * it >= nbk) break;                                   // uniform
-        const int j = lane + 64 * it;
+    for (int it = 0; it < NIT; ++it) {
+        const int j = (lane & (LPR - 1)) + LPR * it;
         const bool live = j < nbk;
         const int jj = live ? j : 0;
         const bool odd = jj & 1;                                     // the block starts 2 bytes into dword 0
-        float dw[kGvRows];
-        uint32_t codes[kGvRows][8];
+        float dw[RL];
+        uint32_t codes[RL][8];
 #pragma unroll
-        for (int r = 0; r < kGvRows; ++r) {
+        for (int r = 0; r < RL; ++r) {
             const uint32_t* q = qw[it][r];
             dw[r] = live ? f16_to_f32((uint16_t)(odd ? q[0] >> 16 : q[0] & 0xffffu)) : 0.0f;
 #pragma unroll
@@ -1701,7 +1715,7 @@ __global__ void __launch_bounds__(64 * kGv8Waves) proj_gemv_q8_kernel(ProjArgs a
             const uint32_t xc[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
             const float dx = xd[n][jj];
 #pragma unroll
-            for (int r = 0; r < kGvRows; ++r) {
+            for (int r = 0; r < RL; ++r) {
                 int s = 0;
 #pragma unroll
                 for (int i = 0; i < 8; ++i) s = __builtin_amdgcn_sdot4((int)codes[r][i], (int)xc[i], s, false);
@@ -1713,15 +1727,39 @@ __global__ void __launch_bounds__(64 * kGv8Waves) proj_gemv_q8_kernel(ProjArgs a
     // sums over the lanes; lane r * N + n keeps (row r, token n)
     float outv = 0.0f;
 #pragma unroll
-    for (int r = 0; r < kGvRows; ++r)
+    for (int r = 0; r < RL; ++r)
 #pragma unroll
         for (int n = 0; n < kGvMaxN; ++n) {
             if (n >= N) break;                                       // uniform
-            const float sum = wave_sum(acc[r][n]);
-            if (lane == r * N + n) outv = sum;
+            if constexpr (HALF) {
+                const float sum = half_sum(acc[r][n]);
+                const float lo = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(sum), 0));
+                const float hi = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(sum), 32));
+                if (lane == r * N + n) outv = lo;
+                if (lane == (r + 2) * N + n) outv = hi;
+            } else {
+                const float sum = wave_sum(acc[r][n]);
+                if (lane == r * N + n) outv = sum;
+            }
         }
     if constexpr (MODE == kProjQKVRope) gemv_rope_store(a, lane, N, mat, rl, outv + addend);
     else gemv_store<MODE>(a, lane, N, m0, outv + addend);
+}
+
+template <int MODE>
+hipError_t launch_gemv_q8(const ProjArgs& a, hipStream_t s) {
+    const dim3 g(a.M / kGv8Rows), b(64 * kGv8Waves);
+    // (the output projection measured slower with half waves: 0.5B, 5 rows 9.3
+    // us against 6.3)
+    if constexpr (MODE != kProjResidual) {
+        if (a.K <= 32 * 32) {
+            hipLaunchKernelGGL((proj_gemv_q8_kernel<MODE, 1, true>), g, b, 0, s, a);
+            return hipGetLastError();
+        }
+    }
+    if (a.K <= 32 * 64) hipLaunchKernelGGL((proj_gemv_q8_kernel<MODE, 1, false>), g, b, 0, s, a);
+    else                hipLaunchKernelGGL((proj_gemv_q8_kernel<MODE, kGvQ8It, false>), g, b, 0, s, a);
+    return hipGetLastError();
 }
 
 }  // namespace
@@ -2203,11 +2241,8 @@ hipError_t launch_proj_gemv(ProjArgs& a, float* y_ws, int n_cu, hipStream_t s) {
         return launch_gemv_lds<false, kProjResidual>(a, sw, s);
     }
     if (gemv_q8_ok(a)) {
-        const dim3 g8(a.M / kGv8Rows), b8(64 * kGv8Waves);
-        if (a.mode == kProjQKVRope)  hipLaunchKernelGGL((proj_gemv_q8_kernel<kProjQKVRope>), g8, b8, 0, s, a);
-        else if (a.mode == kProjQKV) hipLaunchKernelGGL((proj_gemv_q8_kernel<kProjQKV>), g8, b8, 0, s, a);
-        else                         hipLaunchKernelGGL((proj_gemv_q8_kernel<kProjResidual>), g8, b8, 0, s, a);
-        return hipGetLastError();
+        if (a.mode == kProjQKVRope) return launch_gemv_q8<kProjQKVRope>(a, s);
+        return a.mode == kProjQKV ? launch_gemv_q8<kProjQKV>(a, s) : launch_gemv_q8<kProjResidual>(a, s);
     }
     if (gemv_f16_ok(a))
         return a.mode == kProjQKVRope ? launch_gemv_f16<kProjQKVRope>(a, s)
