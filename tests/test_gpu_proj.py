@@ -352,6 +352,11 @@ def test_4096_token_projection_with_split_tail(ctx, torch_gpu, wt):
 
 TILE_CASES = [
     # hidden, Hq, Hkv, d, weights, cache, T, B: the tile and pieces of k that the call takes
+    (896, 14, 2, 64, vva.F16, vva.F16, 7, 1),        # 64 x 64 for 7 rows of F16 weights
+    (3584, 28, 4, 128, vva.F16, vva.Q8_0, 1, 4),     # and for 4 rows of the largest ones
+    (1024, 14, 2, 64, vva.Q8_0, vva.F32, 3, 1),      # GEMV, half waves, all 32 blocks
+    (1088, 12, 2, 128, vva.Q8_0, vva.F16, 3, 2),     # GEMV, one round of blocks
+    (2112, 12, 2, 128, vva.Q8_0, vva.Q8_0, 4, 1),    # GEMV, two rounds of blocks
     (64, 2, 2, 64, vva.F16, vva.F16, 9, 1),          # 64 x 64, one k step (fewer than loads in flight), 9 rows
     (384, 14, 2, 64, vva.Q8_0, vva.Q8_0, 65, 1),     # 64 x 64, a second token tile of one row
     (448, 2, 1, 128, vva.Q8_0, vva.Q8_0, 33, 2),     # 64 features of a 128-dim head, Q8_0 cache (pair epilogue)

@@ -1768,6 +1768,17 @@ bool proj_gemv_supported(int N, int K, int M) {
     return N >= 1 && N <= kGvMaxN && K <= kGvMaxK && K % 64 == 0 && M % kGvRows == 0;
 }
 
+// F16 weights: the GEMV's dot products grow with the token rows, the GEMM's
+// cost does not.  us of the q/k/v and output calls, GEMV against GEMM: 7B, 3
+// rows 16.0 + 9.7 against 17.1 + 11.0, 5 rows 21.6 + 13.8, 8 rows 30.1 + 20.0
+// (GEMM the same 17.1 + 11.0); 1.5B, 5 rows 11.5 + 7.6, 8 rows 14.4 + 10.4,
+// against 13.7 + 7.8; 0.5B, 8 rows 12.4 + 7.8 against 11.6 + 6.7.  (Q8_0
+// weights: 7B, 8 rows 17.7 + 12.1 against 20.0 + 15.4, the GEMV throughout.)
+bool proj_few_rows_gemm(const ProjArgs& a) {
+    return a.w_type == VVA_TYPE_F16 && a.M % 128 == 0 &&
+           (a.N >= 7 || (a.N >= 4 && (int64_t)a.M * a.K >= (int64_t)8 << 20));
+}
+
 // Sums over the wave of 4 values per lane at once, value k ending in every
 // lane of 16 k .. 16 k + 15: lane halves exchanged by permlane32 swaps
 // (values k and k + 2 meet), rows of 16 by a permlane16 swap, then a row

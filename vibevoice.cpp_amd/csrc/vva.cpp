@@ -1014,18 +1014,38 @@ bool rows16(const vva_tensor* x) {
 // call, the weights dequantized to f16 (the GEMM then runs on those), then,
 // when the GEMM is split along K, the pieces' partials; the split tickets
 // follow the decode step's and the prefill's in the context's ticket buffer.
-static vva_status run_proj_gemm(vva_context* ctx, ProjPrepArgs& p, ProjArgs& a, int N, int K, int P) {
-    const bool dq = proj_dequant_q8(a, ctx->n_cu);
-    ProjArgs g = a;                                    // the GEMM's view of the weights
+struct ProjGemmPlan {
+    ProjArgs g;                                        // the GEMM's view of the call
+    bool dq;
+    size_t base, wbytes, total;                        // workspace: prep rows, dequantized weights, all
+};
+static ProjGemmPlan plan_proj_gemm(vva_context* ctx, const ProjPrepArgs& p, const ProjArgs& a, int N, int K, int P) {
+    ProjGemmPlan r{a, proj_dequant_q8(a, ctx->n_cu), 0, 0, 0};
+    ProjArgs& g = r.g;
     g.x = p.x; g.x_type = p.x_type; g.x_nb_t = p.x_nb_t; g.x_nb_b = p.x_nb_b;
-    if (dq) g.w_type = VVA_TYPE_F16;
+    if (r.dq) g.w_type = VVA_TYPE_F16;
     // (dequantized weights meet x in its Q8_0 round trip: the prep's rows)
-    g.direct = !dq && proj_direct_ok(g);
+    g.direct = !r.dq && proj_direct_ok(g);
     g.ksplit = proj_ksplit(g, ctx->n_cu, &g.tail0);
     g.tickets = ctx->tickets + kMaxStepTickets + kMaxPrefillTickets;
-    const size_t base = proj_needs_prep(g, ctx->n_cu) ? (proj_ws_bytes(N, K, P) + 255) / 256 * 256 : 0;
-    const size_t wbytes = dq ? ((size_t)a.M * K * 2 + 255) / 256 * 256 : 0;
-    vva_status st = ensure_ws(ctx, base + wbytes + proj_part_bytes(g, ctx->n_cu));
+    r.base = proj_needs_prep(g, ctx->n_cu) ? (proj_ws_bytes(N, K, P) + 255) / 256 * 256 : 0;
+    r.wbytes = r.dq ? ((size_t)a.M * K * 2 + 255) / 256 * 256 : 0;
+    r.total = r.base + r.wbytes + proj_part_bytes(g, ctx->n_cu);
+    return r;
+}
+// Whether a call of few token rows takes the GEMV: the rows are 16-byte
+// aligned, and the GEMM is not the faster one (or would have to grow the
+// workspace where that cannot be done: under capture).
+static bool takes_gemv(vva_context* ctx, const vva_tensor* x, const ProjPrepArgs& p, const ProjArgs& a, int N, int K, int P) {
+    if (!proj_gemv_supported(N, K, a.M) || !rows16(x)) return false;
+    return !proj_few_rows_gemm(a) || !ws_can_hold(ctx, plan_proj_gemm(ctx, p, a, N, K, P).total);
+}
+static vva_status run_proj_gemm(vva_context* ctx, ProjPrepArgs& p, ProjArgs& a, int N, int K, int P) {
+    ProjGemmPlan pl = plan_proj_gemm(ctx, p, a, N, K, P);
+    ProjArgs& g = pl.g;
+    const bool dq = pl.dq;
+    const size_t base = pl.base, wbytes = pl.wbytes;
+    vva_status st = ensure_ws(ctx, pl.total);
     if (st != VVA_OK) return st;
     if (dq) {
         uint16_t* wd = (uint16_t*)((char*)ctx->ws + base);
@@ -1135,7 +1155,7 @@ extern "C" vva_status vva_qkv_rope_append(vva_context* ctx, vva_kv* kv, int laye
     p.P = (int)(d / 2);
     p.theta_scale = powf(freq_base, -2.0f / (float)d);
     DeviceGuard g(ctx->device);
-    if (proj_gemv_supported((int)N, (int)K, a.M) && rows16(x)) {
+    if (takes_gemv(ctx, x, p, a, (int)N, (int)K, p.P)) {
         // a decode step: the weight-streaming GEMV.  F32 / F16 / BF16 caches:
         // it rotates q and k and stores q_out and the cache rows itself (each
         // wave computes two whole rotation pairs), one launch.  Q8_0 caches
@@ -1272,7 +1292,7 @@ extern "C" vva_status vva_out_proj_residual(vva_context* ctx, const vva_tensor* 
     p.P = 0;
     DeviceGuard g(ctx->device);
     hipError_t e;
-    if (proj_gemv_supported((int)N, (int)K, (int)M) && rows16(o)) {
+    if (takes_gemv(ctx, o, p, a, (int)N, (int)K, 0)) {
         a.x = p.x; a.x_type = p.x_type; a.x_nb_t = p.x_nb_t; a.x_nb_b = p.x_nb_b;
         e = launch_proj_gemv(a, nullptr, ctx->n_cu, ctx->stream);
         return e == hipSuccess ? VVA_OK : hip_fail(ctx, e, "out_proj_residual launch");

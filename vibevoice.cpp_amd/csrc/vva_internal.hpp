@@ -257,6 +257,8 @@ hipError_t launch_proj(ProjPrepArgs& p, ProjArgs& a, void* ws, int n_cu, hipStre
 // converts the rows itself.  kProjQKV writes y = x w^T + bias (F32 [N][M],
 // at `ws`) for the caller's RoPE + append; kProjResidual writes h.
 bool proj_gemv_supported(int N, int K, int M);
+// whether such a call runs faster as a GEMM all the same
+bool proj_few_rows_gemm(const ProjArgs& a);
 hipError_t launch_proj_gemv(ProjArgs& a, float* y_ws, int n_cu, hipStream_t s);
 // Whether launch_proj_gemv can run a kProjQKV call as kProjQKVRope (one
 // launch: projections, bias, RoPE and the append of F32 / F16 / BF16 rows).
