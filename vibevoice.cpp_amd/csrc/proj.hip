@@ -2291,11 +2291,11 @@ constexpr int kDqMaxK = 8192;                  // inputs of a Q8_0 row that proj
 // ~9 TB/s over the chip, at every tile size.
 struct GemmPlan { int tm, tn, ks; };
 GemmPlan gemm_plan(const ProjArgs& a, int n_cu, bool allow_big) {
-    struct Tile { int tm, tn; double lone, shared, merge; };
-    static const Tile kF16[] = {{64, 64, 0.27, 0.33, 2.5}, {64, 128, 0.45, 0.55, 4.0}, {128, 128, 0.85, 0.85, 9.0},
-                                {256, 128, 1.20, 1.20, 0.0}};
-    static const Tile kQ8[] = {{64, 64, 0.33, 0.40, 2.5}, {64, 128, 0.50, 0.62, 4.0}, {128, 128, 0.95, 0.95, 9.0},
-                               {256, 128, 1.35, 1.35, 0.0}};
+    struct Tile { int tm, tn; double lone, shared, merge, merge_x; };   // merge_x: per workgroup and CU
+    static const Tile kF16[] = {{64, 64, 0.28, 0.33, 2.3, 0.5}, {64, 128, 0.45, 0.55, 4.0, 0.0}, {128, 128, 0.85, 0.85, 9.0, 0.0},
+                                {256, 128, 1.20, 1.20, 0.0, 0.0}};
+    static const Tile kQ8[] = {{64, 64, 0.33, 0.40, 2.3, 0.5}, {64, 128, 0.50, 0.62, 4.0, 0.0}, {128, 128, 0.95, 0.95, 9.0, 0.0},
+                               {256, 128, 1.35, 1.35, 0.0, 0.0}};
     const bool q8 = a.w_type == VVA_TYPE_Q8_0;
     const int nk = a.K / kTK;
     GemmPlan best{64, 64, 1};
@@ -2310,7 +2310,8 @@ GemmPlan gemm_plan(const ProjArgs& a, int n_cu, bool allow_big) {
             if (ks > 1 && (t.tm == 256 || tiles > kMaxProjTickets || tiles * ks > 2 * n_cu || nk < 4 * ks)) break;
             double x = (double)(tiles * ks) / n_cu;
             if (t.tm == 256) x = std::ceil(x);                 // one workgroup per CU
-            double us = (double)nk / ks * (x <= 1.0 ? t.lone : std::max(1.6, x) * t.shared) + (ks > 1 ? t.merge : 0.0);
+            double us = (double)nk / ks * (x <= 1.0 ? t.lone : std::max(1.6, x) * t.shared) +
+                        (ks > 1 ? t.merge + t.merge_x * x : 0.0);
             if (t.tn == 64 && a.direct) us -= 3.5;    // no prep launch
             if (us < best_us) {
                 best_us = us;
