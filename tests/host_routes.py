@@ -1,0 +1,98 @@
+"""Routes of the C ABI on the CPU (a child program of test_host_routes.py, not
+a test module): libvva.so over a stand-in of the HIP runtime
+(tests/cpp/fake_hip.cpp) that records kernel launches and allocations instead
+of making them.  `python host_routes.py NAME` runs the scenario NAME; its
+assertions set the exit status.  Device pointers are made up: the host code
+never reads them."""
+import ctypes
+import os
+import sys
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+sys.path.insert(0, os.path.join(os.path.dirname(HERE), "vibevoice.cpp_amd"))
+FAKE = ctypes.CDLL(os.path.join(HERE, "cpp", "bin", "libfakehip.so"), mode=ctypes.RTLD_GLOBAL)
+FAKE.fake_take_log.restype = ctypes.c_char_p
+FAKE.fake_set.argtypes = [ctypes.c_int, ctypes.c_size_t]
+
+import vva  # noqa: E402 — after the stand-in
+
+LIB = vva.load_library()
+ES = {vva.F32: 4, vva.F16: 2, vva.BF16: 2, vva.I32: 4, vva.Q8_0: 34}
+NO_LIMIT = 1 << 40
+ref = ctypes.byref
+
+
+def row_bytes(t, n):
+    return n // 32 * 34 if t == vva.Q8_0 else n * ES[t]
+
+
+class Host:
+    """A fresh context over the stand-in; tensors at made-up addresses."""
+
+    def __init__(self):
+        self.h = ctypes.c_void_p()
+        FAKE.fake_set(0, NO_LIMIT)
+        assert LIB.vva_create(0, None, ref(self.h)) == vva.OK
+        self.next = 1 << 45
+        FAKE.fake_take_log()
+
+    def kv(self, Hkv, d, max_seq, n_seq, t, lens):
+        h = ctypes.c_void_p()
+        assert LIB.vva_kv_create(self.h, ref(vva.KVDesc(1, Hkv, d, max_seq, n_seq, t)), ref(h)) == vva.OK
+        for s, n in enumerate(lens):
+            assert LIB.vva_kv_set_len(h, s, n) == vva.OK
+        FAKE.fake_take_log()
+        return h
+
+    def tensor(self, t, ne, nb=None, data=None, off=0):
+        """ne as ggml's; dense unless nb; at a fresh 4 KiB boundary + off unless data."""
+        ne = list(ne) + [1] * (4 - len(ne))
+        if nb is None:
+            nb = [ES[t], row_bytes(t, ne[0])]
+            nb += [nb[1] * ne[1], nb[1] * ne[1] * ne[2]]
+        if data is None:
+            data = self.next
+            self.next += (sum(n * b for n, b in zip(ne[1:], nb[1:])) + 8191) // 4096 * 4096
+        x = vva.Tensor()
+        x.data, x.type = data + off, t
+        for i in range(4):
+            x.ne[i], x.nb[i] = ne[i], nb[i]
+        return x
+
+    def call(self, fn, *args, capturing=False, malloc_max=NO_LIMIT):
+        """Status, names of the kernels launched, allocations made."""
+        FAKE.fake_set(int(capturing), malloc_max)
+        st = getattr(LIB, fn)(self.h, *args)
+        FAKE.fake_set(0, NO_LIMIT)
+        log = FAKE.fake_take_log().decode().splitlines()
+        self.grids = [ln.split(" grid ")[1] for ln in log if ln.startswith("kernel ")]
+        return (st, [ln.split(" grid ")[0][len("kernel "):] for ln in log if ln.startswith("kernel ")],
+                [int(ln.split()[1]) for ln in log if ln.startswith("malloc ")])
+
+    def err(self):
+        return LIB.vva_last_error(self.h).decode()
+
+
+def bf16_v_window():
+    """A BF16 V window whose f16 copy [L][Hkv][d] would leave the prefill
+    kernel's 32-bit range (2^30 bytes) although the caller's head-major rows,
+    2 d bytes apart, do not: the kernel then converts as it reads."""
+    d, T = 128, 2000
+    for Hkv, L, converts in ((4, 4000, True), (64, 65536 - 65, True), (64, 65536 - 64, False), (64, 262145, False)):
+        c = Host()
+        nb = [2, 2 * d, 2 * d * L, 2 * d * L * Hkv]                   # ne = [d, L, Hkv, 1]
+        k, v = c.tensor(vva.BF16, [d, L, Hkv], nb), c.tensor(vva.BF16, [d, L, Hkv], nb)
+        q = c.tensor(vva.F32, [d, T, Hkv])
+        out = c.tensor(vva.F32, [d, Hkv, T])
+        st, kernels, _ = c.call("vva_flash_attn_ext", ref(q), ref(k), ref(v), None, d ** -0.5, 0.0, 0.0, ref(out))
+        assert st == vva.OK, c.err()
+        print(Hkv, L, kernels)
+        assert ("window_bf16_v_kernel" in kernels) == converts
+        want = f"prefill_kernel<{d}, {vva.BF16}, {vva.F16 if converts else vva.BF16}, false>"
+        assert want in kernels, want
+
+
+SCENARIOS = [bf16_v_window]
+
+if __name__ == "__main__":
+    {f.__name__: f for f in SCENARIOS}[sys.argv[1]]()

@@ -929,7 +929,7 @@ size_t window_f16_bytes(const AttnArgs& a) {
     return (n + 255) / 256 * 256;
 }
 
-// Whether converting the BF16 V window once pays.  It costs a launch (3.5 us)
+// Whether converting the BF16 V window once pays (and can be done).  It costs a launch (3.5 us)
 // and the window's bytes (4 TB/s); it saves the conversions of every 32 query
 // rows' V^T fragments, 25 us of a 1.5B prefill of 4096 tokens (1e8 visible
 // (row, key) pairs at d = 128).
@@ -938,6 +938,9 @@ size_t window_bf16_v_bytes(const AttnArgs& a) {
     double pairs = 0.0, bytes = 0.0;
     size_t n = 0;
     for (int b = 0; b < a.B; ++b) {
+        // the copy's rows within the kernel's 32-bit offsets, as prefill_supported
+        // asks of the caller's (head-major rows are Hkv times closer together)
+        if ((int64_t)(a.L[b] + kBN) * a.Hkv * a.d * 2 >= ((int64_t)1 << 30)) return 0;
         const double keys = a.mask_mode == kMaskCausal ? a.past[b] + 0.5 * a.T : a.L[b];
         pairs += keys * a.T * a.Hq;
         n += (size_t)a.L[b] * a.Hkv * a.d * 2;

@@ -95,7 +95,8 @@ hipError_t launch_window_to_f16(const AttnArgs& a, void* dst, unsigned long long
 
 // BF16 V rows [0, L_b) of each sequence converted to f16 ([L_b][Hkv][d], one
 // after the other) for the MFMA prefill, which otherwise converts per 32 query
-// rows: the bytes, or 0 where the conversion does not pay.
+// rows: the bytes, or 0 where the conversion does not pay or its rows would
+// leave the kernel's 32-bit offsets.
 size_t window_bf16_v_bytes(const AttnArgs& a);
 hipError_t launch_window_bf16_v(const AttnArgs& a, void* dst, hipStream_t s);
 
