@@ -212,13 +212,14 @@ VVA_API vva_status vva_attn(vva_context* ctx, const vva_kv* kv, int layer,
  * q, k, v ne = [d, H, 1, B]; pos I32 ne = [1] or [1, B]; q_out receives
  * RoPE(q); out F32 ne = [d, Hq, 1, B].  Unless q_out aliases q: F32 / F16 /
  * BF16 caches run as one kernel (RoPE, append, split attention and, up to 16
- * key splits, their merge; longer windows add a merge kernel); dense Q8_0
- * caches run the streamed decode kernel in step mode (RoPE of q, the new row
- * appended by the split that holds it) and its merge kernel, with q_out rows
- * 16-byte
- * aligned.  Other cases run the two calls.  Results equal the two calls'
- * (bit for bit on Q8_0 caches).  Does not advance len.  No counterpart of
- * its own in the reference: it fuses three of its ops per decode step. */
+ * key splits, their merge; longer windows add a merge kernel), 16-bit ones
+ * beyond 8192 keys where the kv head count divides 8 and the rows of q_out
+ * and out are 16-byte aligned; dense Q8_0 caches run the streamed decode
+ * kernel in step mode (RoPE of q, the new row appended by the split that
+ * holds it) and its merge kernel, with q_out rows 16-byte aligned.  Other
+ * cases run the two calls.  Results equal the two calls' (bit for bit on
+ * Q8_0 caches).  Does not advance len.  No counterpart of its own in the
+ * reference: it fuses three of its ops per decode step. */
 VVA_API vva_status vva_decode_step(vva_context* ctx, vva_kv* kv, int layer,
                                    const vva_tensor* q, const vva_tensor* k, const vva_tensor* v,
                                    const vva_tensor* pos, const int32_t* seq_ids, float freq_base,

@@ -92,7 +92,64 @@ def bf16_v_window():
         assert want in kernels, want
 
 
-SCENARIOS = [bf16_v_window]
+def one_token_call(t, Hkv, Hq, d, L, q_off=0, out_off=0, B=1):
+    """vva_attn of one token over L keys: the kernels it takes."""
+    c = Host()
+    kv = c.kv(Hkv, d, L, B, t, [L - 1] * B)
+    q, out = c.tensor(vva.F32, [d, Hq, 1, B], off=q_off), c.tensor(vva.F32, [d, Hq, 1, B], off=out_off)
+    st, kernels, _ = c.call("vva_attn", kv, 0, ref(q), None, None, d ** -0.5, ref(out))
+    assert st == vva.OK, c.err()
+    return kernels
+
+
+def step_call(t, Hkv, Hq, d, L, qo_off=0, out_off=0, B=1, q_out=None, out=None, host=None, **kw):
+    """vva_decode_step to L keys: status and the kernels it takes.  q_out and
+    out: functions of (host, q, k, v) giving other tensors."""
+    c = host or Host()
+    kv = c.kv(Hkv, d, L, B, t, [L - 1] * B)
+    q, k, v = (c.tensor(vva.F32, [d, h, 1, B]) for h in (Hq, Hkv, Hkv))
+    pos = c.tensor(vva.I32, [1])
+    qo = q_out(c, q, k, v) if q_out else c.tensor(vva.F32, [d, Hq, 1, B], off=qo_off)
+    o = out(c, q, k, v, qo) if out else c.tensor(vva.F32, [d, Hq, 1, B], off=out_off)
+    st, kernels, mallocs = c.call("vva_decode_step", kv, 0, ref(q), ref(k), ref(v), ref(pos), None, 1e6, d ** -0.5,
+                                  ref(qo), ref(o), **kw)
+    return st, kernels, mallocs
+
+
+def one_token_precision():
+    """One-token attention over 16-bit caches: f16 probabilities (and f16 V for
+    BF16 caches) only for the calls that decode_kernel has always taken with
+    them; other head counts and unaligned rows keep the fp32 row kernel, in
+    vva_attn and in steps beyond 8192 keys.  F32 caches are fp32 throughout."""
+    def name(kernels):
+        assert len(kernels) == 1 or kernels[1].startswith("decode_merge_kernel"), kernels
+        return kernels[0].split("<")[0]
+    for d in (64, 128):
+        for t in (vva.F16, vva.BF16, vva.F32):
+            for Hkv, G in ((1, 8), (2, 7), (3, 2), (4, 1), (5, 1), (6, 4), (7, 1), (8, 2), (12, 2), (16, 1)):
+                fp16 = t != vva.F32 and 8 % Hkv == 0
+                want = "decode_step_kernel" if fp16 or t == vva.F32 else "attn_rows_kernel"
+                got = name(one_token_call(t, Hkv, Hkv * G, d, 300))
+                assert got == want, (d, t, Hkv, G, got)
+                for L in (300, 8192):                             # short steps: every head count, as ever
+                    st, kernels, _ = step_call(t, Hkv, Hkv * G, d, L)
+                    assert st == vva.OK and name(kernels) == "decode_step_kernel", (d, t, Hkv, G, L, kernels)
+                st, kernels, _ = step_call(t, Hkv, Hkv * G, d, 8193)
+                assert st == vva.OK
+                if want == "decode_step_kernel":
+                    assert name(kernels) == want, (d, t, Hkv, G, kernels)
+                else:
+                    assert [k.split("<")[0] for k in kernels] == ["rope_append_vec_kernel", want], (d, t, Hkv, kernels)
+            if t == vva.F32:
+                continue
+            # rows of q or out that are not 16-byte aligned
+            for off in ((4, 0), (8, 0), (0, 4)):
+                assert name(one_token_call(t, 2, 14, d, 300, *off)) == "attn_rows_kernel", (d, t, off)
+            st, kernels, _ = step_call(t, 2, 14, d, 9000, qo_off=8)
+            assert st == vva.OK and kernels[1].split("<")[0] == "attn_rows_kernel", kernels
+
+
+SCENARIOS = [bf16_v_window, one_token_precision]
 
 if __name__ == "__main__":
     {f.__name__: f for f in SCENARIOS}[sys.argv[1]]()

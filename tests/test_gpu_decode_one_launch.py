@@ -103,3 +103,42 @@ def test_one_token_flash_on_strided_rows(ctx, torch_gpu, dt):
     ref = torch.matmul(torch.softmax(s, -1), v.double().contiguous()).view(B, 1, Hq, d)
     tol = 1e-4 if dt == "float32" else 2e-3
     assert (outs[0].double() - ref).abs().max().item() <= tol
+
+
+@pytest.mark.parametrize("t", [vva.F16, vva.BF16])
+@pytest.mark.parametrize("d,Hkv", [(64, 3), (128, 6)])
+def test_other_head_counts_keep_fp32_probabilities(ctx, torch_gpu, d, Hkv, t):
+    """kv head counts that do not divide 8, 16-bit caches: one-token attention
+    and steps beyond 8192 keys keep the row kernel (fp32 probabilities and V):
+    bit for bit, and a BF16 V beyond the f16 range stays finite."""
+    torch = torch_gpu
+    Hq, L = 2 * Hkv, 8300
+    print(f"fp32 one-token d={d} Hkv={Hkv} type={t}", flush=True)
+    a = vva.KVCache(ctx, 1, Hkv, d, L, 1, t)
+    u = vva.KVCache(ctx, 1, Hkv, d, L, 1, t)
+    rng = np.random.default_rng(d)
+    k, v = (rng.standard_normal((L, Hkv, d)).astype(np.float32) for _ in range(2))
+    if t == vva.BF16:
+        v[L // 2] = 1e5                                     # 65504 is the largest finite f16
+    for kv in (a, u):
+        kv.upload(0, 0, 0, k, v)
+    qkv = [to_gpu(torch, rng.standard_normal((1, 1, n, d)), vva.F32) for n in (Hq, Hkv, Hkv)]
+    pos = torch.tensor([L - 1], dtype=torch.int32, device="cuda")
+    qa, qu = torch.empty_like(qkv[0]), torch.empty_like(qkv[0])
+    outs = [torch.full((1, 1, Hq, d), float("nan"), device="cuda") for _ in range(3)]
+    for kv in (a, u):
+        kv.set_len(0, L - 1)
+    ctx.decode_step(a, 0, *qkv, pos, qa, outs[0], d ** -0.5)
+    ctx.rope_append(u, 0, *qkv, pos, qu)
+    ctx.attn(u, 0, qu, outs[1], d ** -0.5)
+    ctx.set_attn_path(1)
+    try:
+        ctx.attn(u, 0, qu, outs[2], d ** -0.5)
+    finally:
+        ctx.set_attn_path(0)
+    torch.cuda.synchronize()
+    assert torch.equal(qa, qu)
+    assert torch.isfinite(outs[2]).all()
+    assert torch.equal(outs[0], outs[2]) and torch.equal(outs[1], outs[2])
+    a.free()
+    u.free()

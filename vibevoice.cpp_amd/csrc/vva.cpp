@@ -263,8 +263,11 @@ vva_status run_attention(vva_context* ctx, AttnArgs& a, bool fixed = false) {
         ctx->last_splits = ctx->logged_splits = n_splits;
         return VVA_OK;
     }
-    if (ctx->attn_path != 1 && a.T == 1 && a.k_type == a.v_type && a.mask_mode != kMaskExplicit) {
-        // F32 / F16 / BF16 rows without an explicit mask: every key is visible to the one token
+    if (ctx->attn_path != 1 && a.T == 1 && a.k_type == a.v_type && a.mask_mode != kMaskExplicit &&
+        (a.k_type == VVA_TYPE_F32 || decode_supported(a))) {
+        // F32 / F16 / BF16 rows without an explicit mask: every key is visible to the one token.
+        // 16-bit rows: the kernel rounds the probabilities (and BF16 V) to f16, as decode_kernel
+        // does, so it takes that kernel's calls; the others keep the row kernel's fp32
         StepArgs sa{};
         sa.q = a.q; sa.q_type = a.q_type; sa.q_nb_h = a.q_nb_h; sa.q_nb_b = a.q_nb_b;
         for (int b = 0; b < a.B; ++b) {
@@ -1353,9 +1356,8 @@ extern "C" vva_status vva_decode_step(vva_context* ctx, vva_kv* kv, int layer, c
     DeviceGuard g(ctx->device);
     // q_out aliasing q: every split reads q while split 0 writes q_out
     const bool alias = q_out->data == q->data;
-    if (!alias && kv->desc.type == VVA_TYPE_Q8_0 && ctx->attn_path == 0) {
-        // dense Q8_0 caches: the streamed decode kernel in step mode (RoPE of q,
-        // the new row appended by the split that holds it), then its merge
+    // the step's attention as vva_attn's arguments, with the query rows of `rows`
+    auto attn_args = [&](const vva_tensor* rows) {
         AttnArgs c{};
         for (int b = 0; b < B; ++b) {
             c.k[b] = a.kc[b];
@@ -1363,15 +1365,21 @@ extern "C" vva_status vva_decode_step(vva_context* ctx, vva_kv* kv, int layer, c
             c.past[b] = a.past[b];
             c.L[b] = a.past[b] + 1;
         }
-        c.q = a.q; c.q_type = a.q_type;
-        c.q_nb_h = q->nb[1]; c.q_nb_t = q->nb[2]; c.q_nb_b = q->nb[3];
+        c.q = (const char*)rows->data; c.q_type = rows->type;
+        c.q_nb_h = rows->nb[1]; c.q_nb_t = rows->nb[2]; c.q_nb_b = rows->nb[3];
         c.k_nb_tok = c.v_nb_tok = kv->row_bytes;
         c.k_nb_head = c.v_nb_head = kv->head_bytes;
-        c.k_type = c.v_type = VVA_TYPE_Q8_0;
+        c.k_type = c.v_type = kv->desc.type;
         c.mask_mode = kMaskCausal;
         c.scale = scale;
         c.out = a.out; c.o_nb_h = out->nb[1]; c.o_nb_t = out->nb[2]; c.o_nb_b = out->nb[3];
         c.d = (int)d; c.Hq = (int)Hq; c.Hkv = (int)Hkv; c.T = 1; c.B = (int)B;
+        return c;
+    };
+    if (!alias && kv->desc.type == VVA_TYPE_Q8_0 && ctx->attn_path == 0) {
+        // dense Q8_0 caches: the streamed decode kernel in step mode (RoPE of q,
+        // the new row appended by the split that holds it), then its merge
+        const AttnArgs c = attn_args(q);
         // q_out rows are written 16 bytes at a time
         const bool qo_aligned = (uintptr_t)q_out->data % 16 == 0 && q_out->nb[1] % 16 == 0 && q_out->nb[3] % 16 == 0 &&
                                 (int64_t)q_out->nb[0] == type_elem_bytes(q_out->type);
@@ -1396,8 +1404,11 @@ extern "C" vva_status vva_decode_step(vva_context* ctx, vva_kv* kv, int layer, c
             return VVA_OK;
         }
     }
-    if (alias || !decode_step_supported(a)) {
-        // the unfused path: RoPE + append, then attention (other cache types, longer windows)
+    bool one_launch = !alias && decode_step_supported(a);
+    if (one_launch && kv->desc.type != VVA_TYPE_F32 && *std::max_element(a.past, a.past + B) >= kStepAnyHeads)
+        one_launch = decode_supported(attn_args(q_out));
+    if (!one_launch) {
+        // the two calls: RoPE + append, then attention
         if ((st = vva_rope_append(ctx, kv, layer, q, k, v, pos, seq_ids, freq_base, q_out)) != VVA_OK) return st;
         return vva_attn(ctx, kv, layer, q_out, seq_ids, nullptr, scale, out);
     }

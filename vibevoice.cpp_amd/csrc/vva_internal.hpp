@@ -122,6 +122,10 @@ struct StepArgs {
     int G;                                                 // Hq / Hkv
 };
 bool decode_step_supported(const StepArgs& a);
+// 16-bit caches: windows up to which vva_decode_step takes every head count.
+// Longer ones go there only where vva_attn's probabilities are f16 too
+// (decode_supported); the rest keep the two calls, whose attention is fp32.
+constexpr int kStepAnyHeads = 8192;
 // Key splits per (sequence, kv head); wgs > 0: workgroups to plan for
 int decode_step_splits(const StepArgs& a, int n_cu, int wgs);
 size_t decode_step_ws_bytes(const StepArgs& a, int n_splits);
