@@ -149,7 +149,63 @@ def one_token_precision():
             assert st == vva.OK and kernels[1].split("<")[0] == "attn_rows_kernel", kernels
 
 
-SCENARIOS = [bf16_v_window, one_token_precision]
+def proj_call(mode, wt, heads, N, T=None, xt=vva.F32, cache=vva.F16, host=None, **kw):
+    """vva_qkv_rope_append ("qkv") or vva_out_proj_residual ("out") of N token
+    rows: status, kernels, allocations."""
+    c = host or Host()
+    d, Hq, Hkv, hidden = heads
+    T = T or N
+    B = N // T
+    def weight(M, K):
+        return c.tensor(wt, [K, M])
+    if mode == "out":
+        o, x, h = c.tensor(xt, [Hq * d, T, B]), c.tensor(vva.F32, [hidden, T, B]), c.tensor(vva.F32, [hidden, T, B])
+        return c.call("vva_out_proj_residual", ref(o), ref(weight(hidden, Hq * d)), ref(x), ref(h), **kw)
+    kv = c.kv(Hkv, d, T, B, cache, [0] * B)
+    x, q = c.tensor(xt, [hidden, T, B]), c.tensor(vva.F32, [d, Hq, T, B])
+    pos = c.tensor(vva.I32, [T])
+    return c.call("vva_qkv_rope_append", kv, 0, ref(x), *(ref(weight(n * d, hidden)) for n in (Hq, Hkv, Hkv)), None,
+                  None, None, ref(pos), None, 1e6, ref(q), **kw)
+
+
+H05, H15, H7 = (64, 14, 2, 896), (128, 12, 2, 1536), (128, 28, 4, 3584)      # d, Hq, Hkv, hidden
+
+
+def workspace_one_can_do_without():
+    """Calls that use the workspace only to be faster run without it where it
+    cannot grow: under capture on a fresh context, or on a full device."""
+    for kw in ({"capturing": True}, {"malloc_max": 1 << 19}):
+        # a BF16 prefill converts V as it reads
+        c = Host()
+        kv = c.kv(4, 128, 16384, 1, vva.BF16, [0])
+        q, out = c.tensor(vva.BF16, [128, 28, 16384]), c.tensor(vva.F32, [128, 28, 16384])
+        args = (kv, 0, ref(q), None, None, 0.1, ref(out))
+        st, kernels, mallocs = c.call("vva_attn", *args, **kw)
+        assert st == vva.OK and not mallocs, c.err()
+        assert kernels == [f"prefill_kernel<128, {vva.BF16}, {vva.BF16}, false>"], kernels
+        st, kernels, mallocs = c.call("vva_attn", *args)
+        assert st == vva.OK and kernels[0] == "window_bf16_v_kernel" and mallocs, kernels
+        # 4 to 8 rows of F16 weights: the GEMV instead of the GEMM (the q/k/v
+        # call's GEMV itself needs the first megabyte)
+        for mode in ("qkv", "out"):
+            for N in (4, 8):
+                c = Host()
+                if mode == "qkv":
+                    assert proj_call(mode, vva.F16, H7, 3, host=c)[2] == [1 << 20]
+                st, kernels, mallocs = proj_call(mode, vva.F16, H7, N, host=c, **kw)
+                assert st == vva.OK and not mallocs and kernels[0].startswith("proj_gemv_"), (kernels, mallocs, c.err())
+                st, kernels, _ = proj_call(mode, vva.F16, H7, N, host=c)
+                assert st == vva.OK and kernels[-1].startswith("proj_gemm_kernel"), kernels
+    # what cannot do without says so, and the next call is none the worse
+    c = Host()
+    kv = c.kv(4, 128, 2048, 1, vva.F16, [2047])
+    q, out = c.tensor(vva.F32, [128, 28]), c.tensor(vva.F32, [128, 28])
+    for kw, want in (({"malloc_max": 1 << 19}, vva.ERR_OOM), ({"capturing": True}, vva.ERR_INVALID_ARG), ({}, vva.OK)):
+        st, kernels, _ = c.call("vva_attn", kv, 0, ref(q), None, None, 0.1, ref(out), **kw)
+        assert st == want and bool(kernels) == (want == vva.OK), (st, want, c.err())
+
+
+SCENARIOS = [bf16_v_window, one_token_precision, workspace_one_can_do_without]
 
 if __name__ == "__main__":
     {f.__name__: f for f in SCENARIOS}[sys.argv[1]]()

@@ -199,30 +199,36 @@ vva_status check_tensor(vva_context* ctx, const vva_tensor* t, const char* name)
 // power of two, 1 MiB at least), so the retired buffers together never
 // exceed the live one: a chunked prefill whose window grows by one chunk per
 // call retires O(log n) buffers, not one per chunk.
-vva_status ensure_ws(vva_context* ctx, size_t bytes) {
-    if (bytes <= ctx->ws_bytes) return VVA_OK;
+hipError_t grow_ws(vva_context* ctx, size_t bytes) {
+    if (bytes <= ctx->ws_bytes) return hipSuccess;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(ctx->stream, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone)
-        return fail(ctx, VVA_ERR_INVALID_ARG,
-                    "split workspace must grow to %zu bytes during stream capture; run one call of this "
-                    "shape before capturing", bytes);
+        return hipErrorStreamCaptureUnsupported;
     size_t sz = (size_t)1 << 20;
     while (sz < bytes) sz <<= 1;
     float* p = nullptr;
-    hipError_t e = hipMalloc(&p, sz);
-    if (e != hipSuccess) return hip_fail(ctx, e, "hipMalloc(split workspace)");
+    const hipError_t e = hipMalloc(&p, sz);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();                       // not the next launch's error
+        return e;
+    }
     if (ctx->ws) ctx->ws_retired.push_back(ctx->ws);
     ctx->ws = p;
     ctx->ws_bytes = sz;
-    return VVA_OK;
+    return hipSuccess;
+}
+vva_status ensure_ws(vva_context* ctx, size_t bytes) {
+    const hipError_t e = grow_ws(ctx, bytes);
+    if (e == hipErrorStreamCaptureUnsupported)
+        return fail(ctx, VVA_ERR_INVALID_ARG,
+                    "split workspace must grow to %zu bytes during stream capture; run one call of this "
+                    "shape before capturing", bytes);
+    return e == hipSuccess ? VVA_OK : hip_fail(ctx, e, "hipMalloc(split workspace)");
 }
 
-// Whether ensure_ws(bytes) would not have to grow during a capture.
-bool ws_can_hold(vva_context* ctx, size_t bytes) {
-    if (bytes <= ctx->ws_bytes) return true;
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    return hipStreamIsCapturing(ctx->stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone;
-}
+// For a call that has a way without it: whether the workspace holds `bytes`,
+// grown if need be (not under capture, nor on a device without the memory).
+bool try_ws(vva_context* ctx, size_t bytes) { return grow_ws(ctx, bytes) == hipSuccess; }
 
 // Split workspace of one call: the context's, grown on demand, or (fixed)
 // the device's static scratch, which never allocates and refuses sizes
@@ -409,10 +415,10 @@ vva_status run_attention(vva_context* ctx, AttnArgs& a, bool fixed = false) {
         const PrefillPlan plan = plan_for(a, fixed ? kScratchBytes : ((size_t)1 << 34));
         // BF16 V converted to f16 ahead of the kernel where that pays and the
         // workspace can hold it beside the partials (the static scratch is
-        // what it is, and a stream under capture cannot grow the context's:
-        // the kernel then converts as it reads, with the same result)
+        // what it is, and the context's cannot grow under capture or on a full
+        // device: the kernel then converts as it reads, with the same result)
         const size_t pb = prefill_ws_bytes(a, plan), vb = window_bf16_v_bytes(a);
-        const bool conv_v = vb > 0 && (fixed ? pb + vb <= kScratchBytes : ws_can_hold(ctx, pb + vb));
+        const bool conv_v = vb > 0 && (fixed ? pb + vb <= kScratchBytes : try_ws(ctx, pb + vb));
         if (conv_v || plan.max_ks > 1) {
             vva_status st = get_ws(ctx, fixed, pb + (conv_v ? vb : 0), &ws);
             if (st != VVA_OK) return st;
@@ -1037,11 +1043,11 @@ static ProjGemmPlan plan_proj_gemm(vva_context* ctx, const ProjPrepArgs& p, cons
     return r;
 }
 // Whether a call of few token rows takes the GEMV: the rows are 16-byte
-// aligned, and the GEMM is not the faster one (or would have to grow the
-// workspace where that cannot be done: under capture).
+// aligned, and the GEMM is not the faster one (or its workspace cannot be
+// had: under capture, or on a full device).
 static bool takes_gemv(vva_context* ctx, const vva_tensor* x, const ProjPrepArgs& p, const ProjArgs& a, int N, int K, int P) {
     if (!proj_gemv_supported(N, K, a.M) || !rows16(x)) return false;
-    return !proj_few_rows_gemm(a) || !ws_can_hold(ctx, plan_proj_gemm(ctx, p, a, N, K, P).total);
+    return !proj_few_rows_gemm(a) || !try_ws(ctx, plan_proj_gemm(ctx, p, a, N, K, P).total);
 }
 static vva_status run_proj_gemm(vva_context* ctx, ProjPrepArgs& p, ProjArgs& a, int N, int K, int P) {
     ProjGemmPlan pl = plan_proj_gemm(ctx, p, a, N, K, P);
