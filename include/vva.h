@@ -217,8 +217,10 @@ VVA_API vva_status vva_attn(vva_context* ctx, const vva_kv* kv, int layer,
  * and out are 16-byte aligned; dense Q8_0 caches run the streamed decode
  * kernel in step mode (RoPE of q, the new row appended by the split that
  * holds it) and its merge kernel, with q_out rows 16-byte aligned.  Other
- * cases run the two calls.  Results equal the two calls' (bit for bit on
- * Q8_0 caches).  Does not advance len.  No counterpart of its own in the
+ * cases run the two calls.  Where an F32 cache's split partials cannot be
+ * held (under HIP graph capture, on a full device) its window is split less,
+ * so such a step needs no workspace.  Results equal the two calls' (bit for
+ * bit on Q8_0 caches).  Does not advance len.  No counterpart of its own in the
  * reference: it fuses three of its ops per decode step. */
 VVA_API vva_status vva_decode_step(vva_context* ctx, vva_kv* kv, int layer,
                                    const vva_tensor* q, const vva_tensor* k, const vva_tensor* v,

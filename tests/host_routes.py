@@ -205,7 +205,49 @@ def workspace_one_can_do_without():
         assert st == want and bool(kernels) == (want == vva.OK), (st, want, c.err())
 
 
-SCENARIOS = [bf16_v_window, one_token_precision, workspace_one_can_do_without]
+def f32_step_without_workspace():
+    """One-token calls on an F32 cache are accepted wherever their split
+    partials cannot be held, with fewer splits; a 16-bit cache's are refused
+    there, as they always were."""
+    d, Hq, Hkv, B = 128, 28, 4, 2
+    per_split = B * Hq * (d + 2) * 4
+    for kw, refusal in (({"capturing": True}, vva.ERR_INVALID_ARG), ({"malloc_max": 1 << 21}, vva.ERR_OOM)):
+        for warm in (0, 300):                                     # keys of an earlier call: 0, none
+            for L in (64, 65, 4097, 32768):
+                c = Host()
+                if warm:
+                    assert step_call(vva.F32, Hkv, Hq, d, warm, B=B, host=c)[2] == [1 << 20]
+                st, kernels, mallocs = step_call(vva.F32, Hkv, Hq, d, L, B=B, host=c, **kw)
+                assert st == vva.OK, (kw, L, c.err())
+                n = LIB.vva_last_decode_splits(c.h)
+                assert kernels[0].startswith("decode_step_kernel") and c.grids[0] == f"{n},{Hkv},{B}"
+                have = max([1 << 20 if warm else 0] + mallocs)
+                chunks, most = -(-L // 64), 512 // (Hkv * B)      # 64 keys a chunk, 512 workgroups
+                want = -(-chunks // -(-chunks // most))
+                assert n == max(1, min(want, have // per_split)), (n, want, have)
+                # vva_attn alone, the same workspace
+                c = Host()
+                if warm:
+                    step_call(vva.F32, Hkv, Hq, d, warm, B=B, host=c)
+                kv = c.kv(Hkv, d, L, B, vva.F32, [L - 1] * B)
+                q, out = c.tensor(vva.F32, [d, Hq, 1, B]), c.tensor(vva.F32, [d, Hq, 1, B])
+                assert c.call("vva_attn", kv, 0, ref(q), None, None, 0.1, ref(out), **kw)[0] == vva.OK, c.err()
+                assert LIB.vva_last_decode_splits(c.h) == n
+        assert step_call(vva.F16, Hkv, Hq, d, 8192, B=B, **kw)[0] == (refusal if "capturing" in kw else vva.OK)
+    # the static scratch: splits forced beyond it
+    for t, want in ((vva.F32, vva.OK), (vva.F16, vva.ERR_INVALID_ARG)):
+        c = Host()
+        assert LIB.vva_set_schedule(c.h, 1 << 20, 0, 0) == vva.OK
+        kv = c.kv(Hkv, d, 65536, 16, t, [65535] * 16)
+        q, out = c.tensor(vva.F32, [d, Hq, 1, 16]), c.tensor(vva.F32, [d, Hq, 1, 16])
+        st, kernels, _ = c.call("vva_attn_noalloc", kv, 0, ref(q), None, None, 0.1, ref(out))
+        assert st == want and bool(kernels) == (want == vva.OK), (t, st, c.err())
+        if want == vva.OK:
+            n = LIB.vva_last_decode_splits(c.h)
+            assert n * 16 * Hq * (d + 2) * 4 <= 36 << 20 < (n + 1) * 16 * Hq * (d + 2) * 4
+
+
+SCENARIOS = [bf16_v_window, one_token_precision, workspace_one_can_do_without, f32_step_without_workspace]
 
 if __name__ == "__main__":
     {f.__name__: f for f in SCENARIOS}[sys.argv[1]]()

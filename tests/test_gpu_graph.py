@@ -191,3 +191,45 @@ def test_prefill_chunk_graph_replays(ctx, torch_gpu, kt):
         print(f"  replay {r} ({splits} key splits): outputs equal the eager step", flush=True)
     del g
     kv.free()
+
+
+def test_f32_step_captured_on_a_fresh_context(torch_gpu):
+    """vva_decode_step on an F32 cache as the first call of a context, under
+    capture: it needs no workspace (one key split).  Three replays, with eager
+    work between them, equal each other bit for bit and the eager step, split
+    over the keys, to 32-bit rounding."""
+    torch = torch_gpu
+    d, Hq, Hkv, past = 64, 14, 2, 700
+    print(f"graph F32 step on a fresh context past={past}", flush=True)
+    c = vva.Context(0)
+    kv = vva.KVCache(c, 1, Hkv, d, past + 1, 1, vva.F32)
+    fill_cache(kv, [past], seed=81)
+    rng = np.random.default_rng(82)
+    q, k, v = (to_gpu(torch, rng.standard_normal((1, 1, n, d)), vva.F32) for n in (Hq, Hkv, Hkv))
+    pos = torch.full((1,), past, dtype=torch.int32, device="cuda")
+    qr, out, qe, eager = (torch.full((1, 1, Hq, d), float("nan"), device="cuda") for _ in range(4))
+    g = torch.cuda.CUDAGraph()
+    default = torch.cuda.current_stream()
+    torch.cuda.synchronize()
+    try:
+        with torch.cuda.graph(g):
+            c.set_stream(torch.cuda.current_stream())
+            c.decode_step(kv, 0, q, k, v, pos, qr, out, d ** -0.5)
+    finally:
+        c.set_stream(default)
+    assert c.last_decode_splits() == 1
+    got = []
+    for _ in range(3):
+        out.fill_(float("nan"))
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        got.append(out.clone())
+        c.decode_step(kv, 0, q, k, v, pos, qe, eager, d ** -0.5)
+        assert c.last_decode_splits() > 1
+        torch.cuda.synchronize()
+        assert torch.equal(got[-1], got[0]) and torch.equal(qr, qe)
+        assert (got[-1] - eager).abs().max().item() <= 1e-6   # sums of 701 terms of order 1/701 in another order
+    del g
+    kv.free()
+    c.close()

@@ -247,6 +247,18 @@ vva_status get_ws(vva_context* ctx, bool fixed, size_t bytes, float** ws) {
     return st;
 }
 
+// Key splits and workspace of a one-launch step or attention.  F32 caches have
+// never needed a workspace for it: where the partials cannot be held (under
+// capture, on a full device, in the static scratch) the window is split as far
+// as what is there allows, down to one split, which leaves none.
+vva_status plan_step(vva_context* ctx, bool fixed, const StepArgs& a, int* n_splits, float** ws) {
+    *n_splits = decode_step_splits(a, ctx->n_cu, ctx->sched_decode_wgs);
+    const size_t bytes = decode_step_ws_bytes(a, *n_splits);
+    if (a.cache_type == VVA_TYPE_F32 && !(fixed ? bytes <= kScratchBytes : try_ws(ctx, bytes)))
+        while (decode_step_ws_bytes(a, *n_splits) > (fixed ? kScratchBytes : ctx->ws_bytes)) --*n_splits;
+    return get_ws(ctx, fixed, decode_step_ws_bytes(a, *n_splits), ws);
+}
+
 // Shared by vva_attn, vva_attn_noalloc (fixed) and vva_flash_attn_ext once
 // AttnArgs is filled.
 vva_status run_attention(vva_context* ctx, AttnArgs& a, bool fixed = false) {
@@ -289,10 +301,9 @@ vva_status run_attention(vva_context* ctx, AttnArgs& a, bool fixed = false) {
         sa.tickets = ctx->tickets;
         sa.d = a.d; sa.Hq = a.Hq; sa.Hkv = a.Hkv; sa.B = a.B; sa.G = a.Hq / a.Hkv;
         if (decode_step_supported(sa)) {
-            const int n_splits = decode_step_splits(sa, ctx->n_cu, ctx->sched_decode_wgs);
-            vva_status st = get_ws(ctx, fixed, decode_step_ws_bytes(sa, n_splits), &ws);
+            int n_splits;
+            vva_status st = plan_step(ctx, fixed, sa, &n_splits, &sa.ws);
             if (st != VVA_OK) return st;
-            sa.ws = ws;
             e = launch_decode_attn(sa, n_splits, ctx->stream);
             if (e != hipSuccess) return hip_fail(ctx, e, "decode launch");
             if (n_splits != ctx->logged_splits)
@@ -1418,9 +1429,8 @@ extern "C" vva_status vva_decode_step(vva_context* ctx, vva_kv* kv, int layer, c
         if ((st = vva_rope_append(ctx, kv, layer, q, k, v, pos, seq_ids, freq_base, q_out)) != VVA_OK) return st;
         return vva_attn(ctx, kv, layer, q_out, seq_ids, nullptr, scale, out);
     }
-    const int n_splits = decode_step_splits(a, ctx->n_cu, ctx->sched_decode_wgs);
-    if ((st = ensure_ws(ctx, decode_step_ws_bytes(a, n_splits))) != VVA_OK) return st;
-    a.ws = ctx->ws;
+    int n_splits;
+    if ((st = plan_step(ctx, false, a, &n_splits, &a.ws)) != VVA_OK) return st;
     hipError_t e = launch_decode_step(a, n_splits, ctx->stream);
     if (e != hipSuccess) return hip_fail(ctx, e, "decode_step launch");
     ctx->last_splits = n_splits;
