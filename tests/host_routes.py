@@ -247,7 +247,20 @@ def f32_step_without_workspace():
             assert n * 16 * Hq * (d + 2) * 4 <= 36 << 20 < (n + 1) * 16 * Hq * (d + 2) * 4
 
 
-SCENARIOS = [bf16_v_window, one_token_precision, workspace_one_can_do_without, f32_step_without_workspace]
+def step_output_alignment():
+    """Output rows on 8-byte boundaries stay in the one-launch step, merged in
+    the launch (decode_merge_kernel writes 16-byte aligned rows); 4-byte ones
+    take the two calls."""
+    for t in (vva.F32, vva.F16, vva.BF16):
+        for L, off, one in ((1000, 8, True), (8192, 8, True), (1000, 4, False)):
+            st, kernels, _ = step_call(t, 4, 28, 128, L, out_off=off)
+            assert st == vva.OK and ("decode_step_kernel" in kernels[0]) == one and (len(kernels) == 1) == one, kernels
+    st, kernels, _ = step_call(vva.F16, 4, 28, 128, 8192)
+    assert kernels[1].startswith("decode_merge_kernel")
+
+
+SCENARIOS = [bf16_v_window, one_token_precision, workspace_one_can_do_without, f32_step_without_workspace,
+             step_output_alignment]
 
 if __name__ == "__main__":
     {f.__name__: f for f in SCENARIOS}[sys.argv[1]]()

@@ -142,3 +142,32 @@ def test_other_head_counts_keep_fp32_probabilities(ctx, torch_gpu, d, Hkv, t):
     assert torch.equal(outs[0], outs[2]) and torch.equal(outs[1], outs[2])
     a.free()
     u.free()
+
+
+@pytest.mark.parametrize("t,L", [(vva.F16, 1000), (vva.BF16, 130), (vva.F32, 60), (vva.F16, 5000)])
+def test_step_output_on_8_byte_boundaries(ctx, torch_gpu, t, L):
+    """Output rows 8 bytes off a 16-byte boundary: the one-launch step with the
+    bits of the aligned call (the same splits), at most 16 splits otherwise."""
+    torch = torch_gpu
+    d, Hq, Hkv = 128, 28, 4
+    print(f"8-byte output type={t} L={L}", flush=True)
+    kv = vva.KVCache(ctx, 1, Hkv, d, L, 1, t)
+    fill_cache(kv, [L - 1], seed=L)
+    rng = np.random.default_rng(L)
+    q, k, v = (to_gpu(torch, rng.standard_normal((1, 1, n, d)), vva.F32) for n in (Hq, Hkv, Hkv))
+    pos = torch.tensor([L - 1], dtype=torch.int32, device="cuda")
+    qo = torch.empty_like(q)
+    wide = torch.full((2 + Hq * (d + 2),), float("nan"), device="cuda")
+    outs = [torch.full((1, 1, Hq, d), float("nan"), device="cuda"), wide[2:].view(1, 1, Hq, d + 2)[..., :d]]
+    splits = []
+    for out in outs:
+        ctx.decode_step(kv, 0, q, k, v, pos, qo, out, d ** -0.5)
+        splits.append(ctx.last_decode_splits())
+    torch.cuda.synchronize()
+    if splits[0] <= 16:
+        assert torch.equal(outs[0], outs[1]) and splits[0] == splits[1]
+    else:
+        assert splits[1] <= 16
+        assert_close(as_f32(torch, outs[1]), as_f32(torch, outs[0]), *TOL[t], what="fewer splits")
+    assert torch.isnan(wide[2:].view(Hq, d + 2)[:, d:]).all() and torch.isnan(wide[:2]).all()
+    kv.free()

@@ -85,6 +85,16 @@ __device__ __forceinline__ float raw_elem(const uint32_t* row, int i, int type) 
     return type == VVA_TYPE_F16 ? f16_to_f32(x) : bf16_to_f32(x);
 }
 
+// Four floats of an output row whose alignment is 16 bytes or only 8.
+__device__ __forceinline__ void store_out(char* p, const float4& v) {
+    if (((uintptr_t)p & 15) == 0) {
+        *(float4*)p = v;
+    } else {
+        *(float2*)p = make_float2(v.x, v.y);
+        *(float2*)(p + 8) = make_float2(v.z, v.w);
+    }
+}
+
 // The cache types: stored element, value -> stored element, keys per wave and chunk
 template <int KT> struct Cell {
     typedef uint16_t elem;
@@ -421,7 +431,7 @@ decode_step_kernel(StepArgs a) {
         const size_t rowi = ((size_t)b * Hq + h * G + r) * n_splits + split;
         if (n_splits == 1) {
             const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
-            *(float4*)((float*)(ob + r * o_nb_h) + d0) = make_float4(ot.x * inv, ot.y * inv, ot.z * inv, ot.w * inv);
+            store_out(ob + r * o_nb_h + d0 * 4, make_float4(ot.x * inv, ot.y * inv, ot.z * inv, ot.w * inv));
         } else if (in_launch) {
             store_coherent2(ws + rowi * D + d0, ot.x, ot.y);
             store_coherent2(ws + rowi * D + d0 + 2, ot.z, ot.w);
@@ -471,7 +481,7 @@ decode_step_kernel(StepArgs a) {
             den = fmaf(ml[e].y, f, den);
         }
         const float inv = den > 0.0f ? 1.0f / den : 0.0f;
-        *(float4*)((float*)(ob + r * o_nb_h) + d0) = make_float4(n0 * inv, n1 * inv, n2 * inv, n3 * inv);
+        store_out(ob + r * o_nb_h + d0 * 4, make_float4(n0 * inv, n1 * inv, n2 * inv, n3 * inv));
     }
     if (tid == 0) __hip_atomic_store(tk, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -491,8 +501,8 @@ bool decode_step_supported(const StepArgs& a) {
     for (int b = 0; b < a.B; ++b)
         if ((uintptr_t)a.kc[b] % 16 || (uintptr_t)a.vc[b] % 16) return false;
     if (a.k_nb_tok % 16 || a.k_nb_head % 16 || a.v_nb_tok % 16 || a.v_nb_head % 16) return false;
-    // the output as 16-byte vectors
-    return (uintptr_t)a.out % 16 == 0 && a.o_nb_h % 16 == 0 && a.o_nb_b % 16 == 0;
+    // the output as 16- or 8-byte vectors
+    return (uintptr_t)a.out % 8 == 0 && a.o_nb_h % 8 == 0 && a.o_nb_b % 8 == 0;
 }
 
 // One chunk per workgroup up to kPlanWgsPerCu workgroups per CU (every byte
@@ -502,7 +512,9 @@ int decode_step_splits(const StepArgs& a, int n_cu, int wgs) {
     int Lmax = 1;
     for (int b = 0; b < a.B; ++b) Lmax = max(Lmax, a.past[b] + 1);
     const int chunks = (Lmax + kc - 1) / kc;
-    const int most = max(1, (wgs > 0 ? wgs : n_cu * kPlanWgsPerCu) / (a.B * a.Hkv));
+    int most = max(1, (wgs > 0 ? wgs : n_cu * kPlanWgsPerCu) / (a.B * a.Hkv));
+    // decode_merge_kernel writes 16-byte aligned rows only
+    if ((uintptr_t)a.out % 16 || a.o_nb_h % 16 || a.o_nb_b % 16) most = min(most, kInLaunchMerge);
     const int per = (chunks + most - 1) / most;
     return (chunks + per - 1) / per;
 }
