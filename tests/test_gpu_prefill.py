@@ -562,3 +562,43 @@ def test_bf16_v_window_of_ragged_and_strided_views(ctx, torch_gpu):
         torch.cuda.synchronize()
         got.append(o)
     assert torch.equal(got[0], got[1])
+
+
+@pytest.mark.parametrize("masked", [False, True])
+def test_merge_of_ten_splits_with_infinite_values(ctx, torch_gpu, masked):
+    """The merge kernel (10 splits in batches of 8) over partials that are not
+    finite: a V element that is infinite makes its dim infinite and nothing
+    else; a row whose keys are all masked is zero although the infinite V
+    element times its zero probability is not a number."""
+    torch = torch_gpu
+    d, Hq, Hkv, T, past, inf_dim = 64, 14, 2, 8, 612, 5
+    print(f"merge of infinite partials masked={masked}", flush=True)
+    L = past + T
+    kv = vva.KVCache(ctx, 1, Hkv, d, L, 1, vva.F16)
+    rng = np.random.default_rng(12)
+    k, v = (rng.standard_normal((L, Hkv, d)).astype(np.float32) for _ in range(2))
+    v[600, :, inf_dim] = np.inf                            # in the last split, seen by every row
+    kv.upload(0, 0, 0, k, v)
+    kv.set_len(0, past)
+    q = to_gpu(torch, rng.standard_normal((1, T, Hq, d)), vva.F32)
+    out = torch.full((1, T, Hq, d), float("nan"), device="cuda")
+    mask = None
+    if masked:
+        m = np.where(np.arange(L)[None, :] <= past + np.arange(T)[:, None], 0.0, -np.inf).astype(np.float32)
+        m[3] = -np.inf
+        mask = torch.from_numpy(m[None]).cuda()
+    with ctx.schedule(prefill_splits=10):
+        ctx.attn(kv, 0, q, out, d ** -0.5, mask=mask)
+    torch.cuda.synchronize()
+    assert ctx.last_decode_splits() == 10
+    got = as_f32(torch, out)[0]
+    rows = [t for t in range(T) if not (masked and t == 3)]
+    if masked:
+        assert (got[3] == 0.0).all()
+    assert np.isposinf(got[rows][..., inf_dim]).all()
+    rest = np.arange(d) != inf_dim
+    v[600, :, inf_dim] = 0.0
+    kv.upload(0, 0, 0, k, v)
+    ref = oracle_attn(as_f32(torch, q), kv, 0, [0], [L], T, d ** -0.5)[0]
+    assert_close(got[rows][..., rest], ref[rows][..., rest], 2e-3, 1e-3, what="the other dims")
+    kv.free()

@@ -693,7 +693,10 @@ __global__ void __launch_bounds__(256) prefill_merge_kernel(AttnArgs a, const fl
             const int64_t r = (int64_t)min(k0 + u, n_ks - 1) * nr_all + rg;     // clamped: unconditional loads
             e[u] = *(const float2*)(ml + r * 2);
             v[u] = *(const float4*)(ws + r * D + 4 * d4);
-            if (k0 + u >= n_ks) e[u] = make_float2(-INFINITY, 0.0f);
+            if (k0 + u >= n_ks) {                                               // (0 times an infinite sum is not 0)
+                e[u] = make_float2(-INFINITY, 0.0f);
+                v[u] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            }
         }
         float mb = M;
 #pragma unroll
@@ -716,6 +719,8 @@ __global__ void __launch_bounds__(256) prefill_merge_kernel(AttnArgs a, const fl
             den = fmaf(e[u].y, f, den);
         }
     }
+    // a row that sees no key: zeros, whatever its partials hold (0 times a V that is not finite)
+    if (M == -INFINITY) num = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     const float inv = den > 0.0f ? 1.0f / den : 0.0f;
     float* orow = (float*)((char*)a.out + b * a.o_nb_b + t * a.o_nb_t + h * a.o_nb_h);
     *(float4*)(orow + 4 * d4) = make_float4(num.x * inv, num.y * inv, num.z * inv, num.w * inv);
