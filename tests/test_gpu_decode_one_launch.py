@@ -171,3 +171,34 @@ def test_step_output_on_8_byte_boundaries(ctx, torch_gpu, t, L):
         assert_close(as_f32(torch, outs[1]), as_f32(torch, outs[0]), *TOL[t], what="fewer splits")
     assert torch.isnan(wide[2:].view(Hq, d + 2)[:, d:]).all() and torch.isnan(wide[:2]).all()
     kv.free()
+
+
+@pytest.mark.parametrize("L,key", [(500, 3), (3000, 2990)])
+def test_infinite_value_on_an_f32_cache(ctx, torch_gpu, L, key):
+    """An infinite V element: that dim is infinite and the others as the row
+    kernel has them, merged in the launch (8 splits of 16 slots) and by the
+    merge kernel (47 splits; the slots past the last one hold nothing)."""
+    torch = torch_gpu
+    d, Hq, Hkv = 128, 12, 2
+    print(f"infinite V element L={L} key={key}", flush=True)
+    kv = vva.KVCache(ctx, 1, Hkv, d, L, 1, vva.F32)
+    rng = np.random.default_rng(L)
+    k, v = (rng.standard_normal((L, Hkv, d)).astype(np.float32) for _ in range(2))
+    v[key, :, 7] = np.inf
+    kv.upload(0, 0, 0, k, v)
+    kv.set_len(0, L - 1)
+    q = to_gpu(torch, rng.standard_normal((1, 1, Hq, d)), vva.F32)
+    outs = [torch.full((1, 1, Hq, d), float("nan"), device="cuda") for _ in range(2)]
+    ctx.attn(kv, 0, q, outs[0], d ** -0.5)
+    assert (ctx.last_decode_splits() > 16) == (L == 3000)
+    ctx.set_attn_path(1)
+    try:
+        ctx.attn(kv, 0, q, outs[1], d ** -0.5)
+    finally:
+        ctx.set_attn_path(0)
+    torch.cuda.synchronize()
+    a, b = (as_f32(torch, o) for o in outs)
+    assert np.isposinf(a[..., 7]).all() and np.isposinf(b[..., 7]).all()
+    rest = np.arange(d) != 7
+    assert_close(a[..., rest], b[..., rest], *TOL[vva.F32], what="the other dims")
+    kv.free()

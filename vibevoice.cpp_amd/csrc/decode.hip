@@ -528,6 +528,7 @@ __global__ void __launch_bounds__(kMergeThreads) decode_merge_kernel(AttnArgs a,
         av[k] = wacc[(size_t)s * (D / 4) + i4];
         const float2 ml = *(const float2*)(wml + 2 * s);
         mv[k] = grp + k * NG < n_splits ? ml.x : -INFINITY;
+        if (grp + k * NG >= n_splits) av[k] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);   // (0 times an infinite sum is not 0)
         lv[k] = ml.y;
     }
     float mt = -INFINITY;

@@ -464,7 +464,10 @@ decode_step_kernel(StepArgs a) {
             ml[e] = load_coherent2(ws + ml_off + ri * 2);
             a0[e] = load_coherent2(ws + ri * D + d0);
             a1[e] = load_coherent2(ws + ri * D + d0 + 2);
-            if (!in) ml[e] = make_float2(-INFINITY, 0.0f);
+            if (!in) {                                 // (0 times an infinite sum is not 0)
+                ml[e] = make_float2(-INFINITY, 0.0f);
+                a0[e] = a1[e] = make_float2(0.0f, 0.0f);
+            }
         }
         float M = -INFINITY;
 #pragma unroll
