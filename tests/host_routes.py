@@ -259,8 +259,43 @@ def step_output_alignment():
     assert kernels[1].startswith("decode_merge_kernel")
 
 
+def output_over_inputs():
+    """A step's output rows laid over its inputs: q itself in one launch, any
+    other overlap as the two calls (whose attention starts when the inputs have
+    been read); rows of several sequences side by side do not overlap."""
+    d, Hq, Hkv, B = 64, 14, 2, 2
+    row = (Hq + 2 * Hkv) * d * 4                                   # [q | k | v] of a sequence
+    for t in (vva.F32, vva.F16):
+        for L in (300, 9000):
+            def step(out, q_out=None):
+                st, kernels, _ = step_call(t, Hkv, Hq, d, L, B=B, q_out=q_out, out=out)
+                assert st == vva.OK
+                return kernels[0].split("<")[0]
+            at = lambda c, x, off=0, nb=None: c.tensor(vva.F32, [d, Hq, 1, B], nb, data=x.data + off)    # noqa: E731
+            one, two = "decode_step_kernel", "rope_append_vec_kernel"
+            assert step(lambda c, q, k, v, qo: at(c, q)) == one
+            assert step(lambda c, q, k, v, qo: at(c, qo)) == two
+            assert step(lambda c, q, k, v, qo: at(c, k)) == two
+            assert step(lambda c, q, k, v, qo: at(c, v, -d * 4)) == two
+            assert step(lambda c, q, k, v, qo: at(c, q, d * 4)) == two
+            assert step(lambda c, q, k, v, qo: at(c, q, 0, [4, d * 4, d * Hq * 4, row])) == two
+            # q_out and out side by side in each sequence's record
+            nb = [4, d * 4, 2 * d * Hq * 4, 2 * d * Hq * 4]
+            assert step(lambda c, q, k, v, qo: at(c, qo, d * Hq * 4, nb),
+                        lambda c, q, k, v: c.tensor(vva.F32, [d, Hq, 1, B], nb)) == one
+            # vva_attn: out over a [q | k | v] record's q, dense and at the record's stride
+            c = Host()
+            kv = c.kv(Hkv, d, L, B, t, [L - 1] * B)
+            q = c.tensor(vva.F32, [d, Hq, 1, B], [4, d * 4, row, row])
+            for nb, want in (([4, d * 4, row, row], "decode_step_kernel"),
+                             (None, "decode_kernel" if t == vva.F16 else "attn_gqa_f32_kernel")):
+                out = c.tensor(vva.F32, [d, Hq, 1, B], nb, data=q.data)
+                st, kernels, _ = c.call("vva_attn", kv, 0, ref(q), None, None, 0.1, ref(out))
+                assert st == vva.OK and kernels[0].split("<")[0] == want, kernels
+
+
 SCENARIOS = [bf16_v_window, one_token_precision, workspace_one_can_do_without, f32_step_without_workspace,
-             step_output_alignment]
+             step_output_alignment, output_over_inputs]
 
 if __name__ == "__main__":
     {f.__name__: f for f in SCENARIOS}[sys.argv[1]]()

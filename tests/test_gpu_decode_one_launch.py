@@ -202,3 +202,29 @@ def test_infinite_value_on_an_f32_cache(ctx, torch_gpu, L, key):
     rest = np.arange(d) != 7
     assert_close(a[..., rest], b[..., rest], *TOL[vva.F32], what="the other dims")
     kv.free()
+
+
+@pytest.mark.parametrize("t,past", [(vva.F32, 900), (vva.F16, 8300)])
+def test_step_output_over_its_projections(ctx, torch_gpu, t, past):
+    """The output written densely over the [q | k | v] records that the step
+    reads: the values of a step whose output lies elsewhere."""
+    torch = torch_gpu
+    d, Hq, Hkv, B = 64, 14, 2, 2
+    print(f"output over the projections type={t} past={past}", flush=True)
+    rng = np.random.default_rng(past)
+    y0 = to_gpu(torch, rng.standard_normal((B, 1, (Hq + 2 * Hkv) * d)), vva.F32)
+    pos = torch.full((1,), past, dtype=torch.int32, device="cuda")
+    outs = []
+    for over in (False, True):
+        y = y0.clone()
+        q, k, v = (x.view(B, 1, -1, d) for x in (y[..., :Hq * d], y[..., Hq * d:-Hkv * d], y[..., -Hkv * d:]))
+        kv = vva.KVCache(ctx, 1, Hkv, d, past + 1, B, t)
+        fill_cache(kv, [past] * B, seed=3)
+        out = y.view(-1)[:B * Hq * d].view(B, 1, Hq, d) if over else torch.empty((B, 1, Hq, d), device="cuda")
+        ctx.decode_step(kv, 0, q, k, v, pos, torch.empty((B, 1, Hq, d), device="cuda"), out, d ** -0.5)
+        torch.cuda.synchronize()
+        outs.append((as_f32(torch, out), [kv.download(0, s, past + 1) for s in range(B)]))
+        kv.free()
+    assert_close(outs[1][0], outs[0][0], *TOL[t], what="over the records")
+    for a, b in zip(outs[0][1], outs[1][1]):
+        assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1])

@@ -247,6 +247,24 @@ vva_status get_ws(vva_context* ctx, bool fixed, size_t bytes, float** ws) {
     return st;
 }
 
+// One token's head rows of every sequence, and whether two such sets share
+// memory (each sequence's rows taken as one range).
+struct TokenRows {
+    const char* p; int64_t nb_b, nb_h; int H, d, type, B;
+    int64_t bytes() const { return (H - 1) * nb_h + (int64_t)d * type_elem_bytes(type); }
+    bool same(const TokenRows& o) const {
+        return p == o.p && (nb_b == o.nb_b || B == 1) && (nb_h == o.nb_h || H == 1) && H == o.H && type == o.type;
+    }
+    bool meets(const TokenRows& o) const {
+        for (int i = 0; i < B; ++i)
+            for (int j = 0; j < B; ++j) {
+                const char *x = p + i * nb_b, *y = o.p + j * o.nb_b;
+                if (x < y + o.bytes() && y < x + bytes()) return true;
+            }
+        return false;
+    }
+};
+
 // Key splits and workspace of a one-launch step or attention.  F32 caches have
 // never needed a workspace for it: where the partials cannot be held (under
 // capture, on a full device, in the static scratch) the window is split as far
@@ -281,8 +299,12 @@ vva_status run_attention(vva_context* ctx, AttnArgs& a, bool fixed = false) {
         ctx->last_splits = ctx->logged_splits = n_splits;
         return VVA_OK;
     }
+    // The one-launch kernel writes a kv group's output while other groups may
+    // still read their q: out may be q itself, but not other memory of it.
+    const TokenRows q_rows{a.q, a.q_nb_b, a.q_nb_h, a.Hq, a.d, a.q_type, a.B};
+    const TokenRows o_rows{(const char*)a.out, a.o_nb_b, a.o_nb_h, a.Hq, a.d, VVA_TYPE_F32, a.B};
     if (ctx->attn_path != 1 && a.T == 1 && a.k_type == a.v_type && a.mask_mode != kMaskExplicit &&
-        (a.k_type == VVA_TYPE_F32 || decode_supported(a))) {
+        (a.k_type == VVA_TYPE_F32 || decode_supported(a)) && (o_rows.same(q_rows) || !o_rows.meets(q_rows))) {
         // F32 / F16 / BF16 rows without an explicit mask: every key is visible to the one token.
         // 16-bit rows: the kernel rounds the probabilities (and BF16 V) to f16, as decode_kernel
         // does, so it takes that kernel's calls; the others keep the row kernel's fp32
@@ -1421,7 +1443,15 @@ extern "C" vva_status vva_decode_step(vva_context* ctx, vva_kv* kv, int layer, c
             return VVA_OK;
         }
     }
-    bool one_launch = !alias && decode_step_supported(a);
+    // out over the inputs (other than q itself) or q_out: a kv group's output is
+    // written while other groups read theirs, and q_out from another workgroup
+    auto rows = [&](const vva_tensor* t) {
+        return TokenRows{(const char*)t->data, (int64_t)t->nb[3], (int64_t)t->nb[1], (int)t->ne[1], (int)d, t->type, (int)B};
+    };
+    const TokenRows o = rows(out);
+    const bool over = o.meets(rows(k)) || o.meets(rows(v)) || o.meets(rows(q_out)) ||
+                      (o.meets(rows(q)) && !o.same(rows(q)));
+    bool one_launch = !alias && !over && decode_step_supported(a);
     if (one_launch && kv->desc.type != VVA_TYPE_F32 && *std::max_element(a.past, a.past + B) >= kStepAnyHeads)
         one_launch = decode_supported(attn_args(q_out));
     if (!one_launch) {
