@@ -2289,16 +2289,15 @@ constexpr int kDqMaxK = 8192;                  // inputs of a Q8_0 row that proj
 // (256 x 128) against 76.1 (the big kernel, whose 128 tiles leave half the CUs
 // idle).  What sets the larger tiles' steps is the operands' way from L2:
 // ~9 TB/s over the chip, at every tile size.
-struct GemmPlan { int tm, tn, ks; };
-GemmPlan gemm_plan(const ProjArgs& a, int n_cu, bool allow_big) {
+// `direct`: the 64 x 64 tiles may read x themselves.
+ProjPlan gemm_plan(const ProjArgs& a, bool q8, bool direct, int n_cu) {
     struct Tile { int tm, tn; double lone, shared, merge, merge_x; };   // merge_x: per workgroup and CU
     static const Tile kF16[] = {{64, 64, 0.28, 0.33, 2.3, 0.5}, {64, 128, 0.45, 0.55, 4.0, 0.0}, {128, 128, 0.85, 0.85, 9.0, 0.0},
                                 {256, 128, 1.20, 1.20, 0.0, 0.0}};
     static const Tile kQ8[] = {{64, 64, 0.33, 0.40, 2.3, 0.5}, {64, 128, 0.50, 0.62, 4.0, 0.0}, {128, 128, 0.95, 0.95, 9.0, 0.0},
                                {256, 128, 1.35, 1.35, 0.0, 0.0}};
-    const bool q8 = a.w_type == VVA_TYPE_Q8_0;
     const int nk = a.K / kTK;
-    GemmPlan best{64, 64, 1};
+    ProjPlan best{64, 64, 1, 0, false, direct};
     double best_us = 1e30;
     // a tile lies in one matrix (every matrix has a multiple of 128 rows); 256
     // rows never came first below kBigMinRows token rows, nor in pieces
@@ -2312,58 +2311,54 @@ GemmPlan gemm_plan(const ProjArgs& a, int n_cu, bool allow_big) {
             if (t.tm == 256) x = std::ceil(x);                 // one workgroup per CU
             double us = (double)nk / ks * (x <= 1.0 ? t.lone : std::max(1.6, x) * t.shared) +
                         (ks > 1 ? t.merge + t.merge_x * x : 0.0);
-            if (t.tn == 64 && a.direct) us -= 3.5;    // no prep launch
+            if (t.tn == 64 && direct) us -= 3.5;    // no prep launch
             if (us < best_us) {
                 best_us = us;
-                best = GemmPlan{t.tm, t.tn, ks};
+                best = ProjPlan{t.tm, t.tn, ks, 0, false, direct && t.tn == 64};
             }
         }
     }
     // the big kernel: 1.45 us a step and 25 us around them, whatever the share
     // of the CUs that its tiles fill; Q8_0 weights are dequantized for it first
-    if (allow_big && a.N >= kBigMinRows && !(q8 && a.K > kDqMaxK)) {
+    if (a.N >= kBigMinRows && !(q8 && a.K > kDqMaxK)) {
         const int64_t tiles = (int64_t)((a.M + kBM - 1) / kBM) * ((a.N + kBN - 1) / kBN);
         const int64_t tail = tiles % n_cu;
         const double rounds = (double)(tiles / n_cu) + (tail == 0 ? 0.0 : (tiles > n_cu && 4 * tail <= n_cu) ? 0.6 : 1.0);
         const double us = rounds * (25.0 + 1.45 * nk) + (q8 ? 2.0 + (double)a.M * a.K * 6.4e-7 : 0.0);
-        if (us < best_us) best = GemmPlan{kBM, kBN, 1};
+        if (us < best_us) {
+            best = ProjPlan{kBM, kBN, 1, 0, q8, false};
+            // the last round's tiles, when they fill at most a quarter of the CUs,
+            // split along K (at most kBMaxSplit pieces of at least 8 k steps)
+            if (tail > 0 && 4 * tail <= n_cu && tail <= kMaxProjTickets && nk >= 16) {
+                best.ks = (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(kBMaxSplit, n_cu / tail), nk / 8));
+                best.tail0 = (int)(tiles - tail);
+            }
+        }
     }
     return best;
 }
-bool proj_direct(const ProjArgs& a, int n_cu) {
-    const GemmPlan t = gemm_plan(a, n_cu, true);
-    return t.tm == 64 && t.tn == 64 && a.direct;
-}
-bool proj_big(const ProjArgs& a, int n_cu) { return gemm_plan(a, n_cu, true).tn == kBN; }
-}  // namespace
-
 // the output projection, F16 weights, 16-byte aligned rows within 32-bit offsets
-bool proj_direct_ok(const ProjArgs& a) {
+bool direct_ok(const ProjArgs& a) {
     return a.mode == kProjResidual && a.w_type == VVA_TYPE_F16 && (uintptr_t)a.x % 16 == 0 && a.x_nb_t % 16 == 0 && a.x_nb_b % 16 == 0 &&
            a.x_nb_t >= 0 && a.x_nb_b >= 0 &&
            (a.N / a.T - 1) * a.x_nb_b + (a.T - 1) * a.x_nb_t + (int64_t)a.K * 4 < ((int64_t)1 << 31);
 }
-bool proj_needs_prep(const ProjArgs& a, int n_cu) { return !proj_direct(a, n_cu); }
+}  // namespace
 
-int proj_ksplit(const ProjArgs& a, int n_cu, int* tail0) {
-    *tail0 = 0;
-    if (!proj_big(a, n_cu)) return gemm_plan(a, n_cu, false).ks;
-    // the last round's tiles, when they fill at most a quarter of the CUs,
-    // split along K (at most kBMaxSplit pieces of at least 8 k steps)
-    const int tiles = ((a.M + kBM - 1) / kBM) * ((a.N + kBN - 1) / kBN);
-    const int nk = a.K / kBK, r = tiles % n_cu;
-    if (r == 0 || 4 * r > n_cu || r > kMaxProjTickets || nk < 16) return 1;
-    *tail0 = tiles - r;
-    return max(1, min(min(kBMaxSplit, n_cu / r), nk / 8));
-}
-size_t proj_part_bytes(const ProjArgs& a, int n_cu) {
-    if (a.ksplit <= 1) return 0;
-    if (proj_big(a, n_cu)) {
-        const size_t tiles = (size_t)((a.M + kBM - 1) / kBM) * ((a.N + kBN - 1) / kBN);
-        return (tiles - a.tail0) * a.ksplit * kBPiece;
+ProjPlan proj_plan(const ProjArgs& a, int n_cu) {
+    const bool q8 = a.w_type == VVA_TYPE_Q8_0;
+    ProjPlan p = gemm_plan(a, q8, direct_ok(a), n_cu);
+    if (p.dequant) {
+        // the weights are f16 then: the best F16 kernel (x in its Q8_0 round trip: the prep's rows)
+        p = gemm_plan(a, false, false, n_cu);
+        p.dequant = true;
     }
-    const GemmPlan t = gemm_plan(a, n_cu, false);
-    return (size_t)(a.M / t.tm) * ((a.N + t.tn - 1) / t.tn) * a.ksplit * t.tm * t.tn * sizeof(float);
+    return p;
+}
+size_t proj_part_bytes(const ProjArgs& a, const ProjPlan& p) {
+    if (p.ks <= 1) return 0;
+    const size_t tiles = (size_t)((a.M + p.tm - 1) / p.tm) * ((a.N + p.tn - 1) / p.tn) - p.tail0;
+    return tiles * p.ks * p.tm * p.tn * sizeof(float);
 }
 
 // Q8_0 weight rows dequantized to f16 rows of d * q: the products the Q8_0
@@ -2416,8 +2411,6 @@ __global__ void __launch_bounds__(kDqThreads) proj_dequant_q8_kernel(ProjArgs a,
     }
 }
 
-bool proj_dequant_q8(const ProjArgs& a, int n_cu) { return a.w_type == VVA_TYPE_Q8_0 && proj_big(a, n_cu); }
-
 hipError_t launch_proj_dequant_q8(const ProjArgs& a, uint16_t* dst, hipStream_t s) {
     hipLaunchKernelGGL(proj_dequant_q8_kernel, dim3((unsigned)a.M), dim3(kDqThreads), 0, s, a, dst);
     return hipGetLastError();
@@ -2430,14 +2423,14 @@ size_t proj_ws_bytes(int N, int K, int P) {
 
 namespace {
 template <int MODE>
-void launch_gemm(const ProjArgs& a, const GemmPlan& t, dim3 g, hipStream_t s) {
+void launch_gemm(const ProjArgs& a, const ProjPlan& t, dim3 g, hipStream_t s) {
     const bool q8 = a.w_type == VVA_TYPE_Q8_0;
     const dim3 b(t.tm == 256 ? 512 : 256);
 #define VVA_GEMM(TM, TN, PF)                                                                                   \
     if (q8) hipLaunchKernelGGL((proj_gemm_kernel<true, MODE, TM, TN, PF, 0>), g, b, 0, s, a);                  \
     else    hipLaunchKernelGGL((proj_gemm_kernel<false, MODE, TM, TN, PF, 0>), g, b, 0, s, a)
     if constexpr (MODE == kProjResidual) {
-        if (t.tn == 64 && a.direct) {
+        if (t.direct) {
             if (a.x_type == VVA_TYPE_F32) hipLaunchKernelGGL((proj_gemm_kernel<false, MODE, 64, 64, 4, 4>), g, b, 0, s, a);
             else                          hipLaunchKernelGGL((proj_gemm_kernel<false, MODE, 64, 64, 6, 2>), g, b, 0, s, a);
             return;
@@ -2451,9 +2444,9 @@ void launch_gemm(const ProjArgs& a, const GemmPlan& t, dim3 g, hipStream_t s) {
 }
 }  // namespace
 
-hipError_t launch_proj(ProjPrepArgs& p, ProjArgs& a, void* ws, int n_cu, hipStream_t s) {
+hipError_t launch_proj(ProjPrepArgs& p, ProjArgs& a, const ProjPlan& t, void* ws, hipStream_t s) {
     hipError_t e = hipSuccess;
-    if (!proj_direct(a, n_cu)) {
+    if (!t.direct) {
         p.xh = (uint16_t*)ws;
         p.rope = p.P > 0 ? (float2*)((char*)ws + ((size_t)p.N * p.K * 2 + 255) / 256 * 256) : nullptr;
         a.xh = p.xh;
@@ -2461,25 +2454,21 @@ hipError_t launch_proj(ProjPrepArgs& p, ProjArgs& a, void* ws, int n_cu, hipStre
         hipLaunchKernelGGL(proj_prep_kernel, dim3(p.N), dim3(256), 0, s, p);
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
-    if (a.ksplit < 1 || !a.part || !a.tickets) {
-        a.ksplit = 1;
-        a.tail0 = 0;
-    }
+    a.ksplit = t.ks;
+    a.tail0 = t.tail0;
+    const int tiles = ((a.M + t.tm - 1) / t.tm) * ((a.N + t.tn - 1) / t.tn);
     // every tile's pieces, or the unsplit tiles then the split tail's pieces
-    auto grid = [&](int tiles) { return a.tail0 > 0 ? a.tail0 + (tiles - a.tail0) * a.ksplit : tiles * a.ksplit; };
-    if (proj_big(a, n_cu)) {
-        const int tiles = ((a.M + kBM - 1) / kBM) * ((a.N + kBN - 1) / kBN);
-        const dim3 g(grid(tiles)), b(kBWaves * 64);
+    const dim3 g(t.tail0 + (tiles - t.tail0) * t.ks);
+    if (t.tn == kBN) {
+        const dim3 b(kBWaves * 64);
         if (a.mode == kProjQKV) hipLaunchKernelGGL((proj_gemm_big_kernel<kProjQKV>), g, b, 0, s, a);
         else                    hipLaunchKernelGGL((proj_gemm_big_kernel<kProjResidual>), g, b, 0, s, a);
-        if ((e = hipGetLastError()) != hipSuccess || a.ksplit <= 1) return e;
-        const dim3 gm((tiles - a.tail0) * (kBN / kBSlab));
+        if ((e = hipGetLastError()) != hipSuccess || t.ks <= 1) return e;
+        const dim3 gm((tiles - t.tail0) * (kBN / kBSlab));
         if (a.mode == kProjQKV) hipLaunchKernelGGL((proj_big_merge_kernel<kProjQKV>), gm, dim3(256), 0, s, a);
         else                    hipLaunchKernelGGL((proj_big_merge_kernel<kProjResidual>), gm, dim3(256), 0, s, a);
         return hipGetLastError();
     }
-    const GemmPlan t = gemm_plan(a, n_cu, false);
-    const dim3 g((a.M / t.tm) * ((a.N + t.tn - 1) / t.tn) * a.ksplit);
     if (a.mode == kProjQKV) launch_gemm<kProjQKV>(a, t, g, s);
     else                    launch_gemm<kProjResidual>(a, t, g, s);
     return hipGetLastError();

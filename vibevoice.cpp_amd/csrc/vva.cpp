@@ -1051,55 +1051,47 @@ bool rows16(const vva_tensor* x) {
 
 }  // namespace
 
-// The prep + GEMM launches of a projection with their workspace: the
-// converted token rows (and RoPE table), then, for Q8_0 weights over a long
-// call, the weights dequantized to f16 (the GEMM then runs on those), then,
+// The prep + GEMM launches of a projection, planned once, with their
+// workspace: the converted token rows (and RoPE table), then Q8_0 weights
+// dequantized to f16 where the plan says so (the GEMM then runs on those), then,
 // when the GEMM is split along K, the pieces' partials; the split tickets
 // follow the decode step's and the prefill's in the context's ticket buffer.
-struct ProjGemmPlan {
-    ProjArgs g;                                        // the GEMM's view of the call
-    bool dq;
+struct ProjGemm {
+    ProjPlan plan;
     size_t base, wbytes, total;                        // workspace: prep rows, dequantized weights, all
 };
-static ProjGemmPlan plan_proj_gemm(vva_context* ctx, const ProjPrepArgs& p, const ProjArgs& a, int N, int K, int P) {
-    ProjGemmPlan r{a, proj_dequant_q8(a, ctx->n_cu), 0, 0, 0};
-    ProjArgs& g = r.g;
-    g.x = p.x; g.x_type = p.x_type; g.x_nb_t = p.x_nb_t; g.x_nb_b = p.x_nb_b;
-    if (r.dq) g.w_type = VVA_TYPE_F16;
-    // (dequantized weights meet x in its Q8_0 round trip: the prep's rows)
-    g.direct = !r.dq && proj_direct_ok(g);
-    g.ksplit = proj_ksplit(g, ctx->n_cu, &g.tail0);
-    g.tickets = ctx->tickets + kMaxStepTickets + kMaxPrefillTickets;
-    r.base = proj_needs_prep(g, ctx->n_cu) ? (proj_ws_bytes(N, K, P) + 255) / 256 * 256 : 0;
-    r.wbytes = r.dq ? ((size_t)a.M * K * 2 + 255) / 256 * 256 : 0;
-    r.total = r.base + r.wbytes + proj_part_bytes(g, ctx->n_cu);
-    return r;
+static ProjGemm plan_proj_gemm(vva_context* ctx, ProjArgs& a, int P) {
+    ProjGemm g{proj_plan(a, ctx->n_cu), 0, 0, 0};
+    g.base = g.plan.direct ? 0 : (proj_ws_bytes(a.N, a.K, P) + 255) / 256 * 256;
+    g.wbytes = g.plan.dequant ? ((size_t)a.M * a.K * 2 + 255) / 256 * 256 : 0;
+    g.total = g.base + g.wbytes + proj_part_bytes(a, g.plan);
+    return g;
 }
-// Whether a call of few token rows takes the GEMV: the rows are 16-byte
-// aligned, and the GEMM is not the faster one (or its workspace cannot be
-// had: under capture, or on a full device).
-static bool takes_gemv(vva_context* ctx, const vva_tensor* x, const ProjPrepArgs& p, const ProjArgs& a, int N, int K, int P) {
-    if (!proj_gemv_supported(N, K, a.M) || !rows16(x)) return false;
-    return !proj_few_rows_gemm(a) || !try_ws(ctx, plan_proj_gemm(ctx, p, a, N, K, P).total);
+// Whether a call takes the GEMV: few token rows, 16-byte aligned, and the GEMM
+// is not the faster one (or its workspace cannot be had: under capture, or on
+// a full device).  Otherwise *g is the GEMM's plan.
+static bool takes_gemv(vva_context* ctx, const vva_tensor* x, ProjArgs& a, int P, ProjGemm* g) {
+    const bool can = proj_gemv_supported(a.N, a.K, a.M) && rows16(x);
+    if (can && !proj_few_rows_gemm(a)) return true;
+    *g = plan_proj_gemm(ctx, a, P);
+    return can && !try_ws(ctx, g->total);
 }
-static vva_status run_proj_gemm(vva_context* ctx, ProjPrepArgs& p, ProjArgs& a, int N, int K, int P) {
-    ProjGemmPlan pl = plan_proj_gemm(ctx, p, a, N, K, P);
-    ProjArgs& g = pl.g;
-    const bool dq = pl.dq;
-    const size_t base = pl.base, wbytes = pl.wbytes;
-    vva_status st = ensure_ws(ctx, pl.total);
+static vva_status run_proj_gemm(vva_context* ctx, ProjPrepArgs& p, ProjArgs& a, const ProjGemm& g) {
+    vva_status st = ensure_ws(ctx, g.total);
     if (st != VVA_OK) return st;
-    if (dq) {
-        uint16_t* wd = (uint16_t*)((char*)ctx->ws + base);
+    if (g.plan.dequant) {
+        uint16_t* wd = (uint16_t*)((char*)ctx->ws + g.base);
         const hipError_t e = launch_proj_dequant_q8(a, wd, ctx->stream);
         if (e != hipSuccess) return hip_fail(ctx, e, "projection weight dequantization");
+        a.w_type = VVA_TYPE_F16;
         for (int i = 0; i < 3; ++i) {
-            g.w[i] = (const char*)(wd + (int64_t)(i == 0 ? 0 : a.m_end[i - 1]) * K);
-            g.w_nb[i] = (int64_t)K * 2;
+            a.w[i] = (const char*)(wd + (int64_t)(i == 0 ? 0 : a.m_end[i - 1]) * a.K);
+            a.w_nb[i] = (int64_t)a.K * 2;
         }
     }
-    g.part = g.ksplit > 1 ? (char*)ctx->ws + base + wbytes : nullptr;
-    const hipError_t e = launch_proj(p, g, ctx->ws, ctx->n_cu, ctx->stream);
+    a.part = (char*)ctx->ws + g.base + g.wbytes;
+    a.tickets = ctx->tickets + kMaxStepTickets + kMaxPrefillTickets;
+    const hipError_t e = launch_proj(p, a, g.plan, ctx->ws, ctx->stream);
     return e == hipSuccess ? VVA_OK : hip_fail(ctx, e, "projection launch");
 }
 
@@ -1196,14 +1188,15 @@ extern "C" vva_status vva_qkv_rope_append(vva_context* ctx, vva_kv* kv, int laye
     p.pos = (const int32_t*)pos->data; p.pos_stride_b = ps;
     p.P = (int)(d / 2);
     p.theta_scale = powf(freq_base, -2.0f / (float)d);
-    DeviceGuard g(ctx->device);
-    if (takes_gemv(ctx, x, p, a, (int)N, (int)K, p.P)) {
+    DeviceGuard dev(ctx->device);
+    a.x = p.x; a.x_type = p.x_type; a.x_nb_t = p.x_nb_t; a.x_nb_b = p.x_nb_b;
+    ProjGemm g;
+    if (takes_gemv(ctx, x, a, p.P, &g)) {
         // a decode step: the weight-streaming GEMV.  F32 / F16 / BF16 caches:
         // it rotates q and k and stores q_out and the cache rows itself (each
         // wave computes two whole rotation pairs), one launch.  Q8_0 caches
         // (a block's scale needs 32 dims of a head): it writes the F32
         // projections and the RoPE + append kernel quantizes and stores them.
-        a.x = p.x; a.x_type = p.x_type; a.x_nb_t = p.x_nb_t; a.x_nb_b = p.x_nb_b;
         a.pos = p.pos; a.pos_stride_b = p.pos_stride_b; a.theta_scale = p.theta_scale;
         if (proj_gemv_rope_ok(a)) {
             a.mode = kProjQKVRope;
@@ -1225,7 +1218,7 @@ extern "C" vva_status vva_qkv_rope_append(vva_context* ctx, vva_kv* kv, int laye
         const vva_tensor tq = proj_view(0, Hq), tk = proj_view(Hq * d, Hkv), tv = proj_view((Hq + Hkv) * d, Hkv);
         return vva_rope_append(ctx, kv, layer, &tq, &tk, &tv, pos, seq_ids, freq_base, q_out);
     }
-    return run_proj_gemm(ctx, p, a, (int)N, (int)K, p.P);
+    return run_proj_gemm(ctx, p, a, g);
 }
 
 extern "C" vva_status vva_qkv_proj(vva_context* ctx, const vva_tensor* x, const vva_tensor* wq, const vva_tensor* wk,
@@ -1333,13 +1326,13 @@ extern "C" vva_status vva_out_proj_residual(vva_context* ctx, const vva_tensor* 
     p.q8 = wt == VVA_TYPE_Q8_0;
     p.P = 0;
     DeviceGuard g(ctx->device);
-    hipError_t e;
-    if (takes_gemv(ctx, o, p, a, (int)N, (int)K, 0)) {
-        a.x = p.x; a.x_type = p.x_type; a.x_nb_t = p.x_nb_t; a.x_nb_b = p.x_nb_b;
-        e = launch_proj_gemv(a, nullptr, ctx->n_cu, ctx->stream);
+    a.x = p.x; a.x_type = p.x_type; a.x_nb_t = p.x_nb_t; a.x_nb_b = p.x_nb_b;
+    ProjGemm pg;
+    if (takes_gemv(ctx, o, a, 0, &pg)) {
+        const hipError_t e = launch_proj_gemv(a, nullptr, ctx->n_cu, ctx->stream);
         return e == hipSuccess ? VVA_OK : hip_fail(ctx, e, "out_proj_residual launch");
     }
-    return run_proj_gemm(ctx, p, a, (int)N, (int)K, 0);
+    return run_proj_gemm(ctx, p, a, pg);
 }
 
 // --------------------------------------------------------- decode step

@@ -163,7 +163,7 @@ struct ProjArgs {
     // kProjResidual: h = y + res (F32 rows; may alias)
     const char* res; int64_t res_nb_t, res_nb_b;
     char* h; int64_t h_nb_t, h_nb_b;
-    // few-row path and `direct`: the token rows themselves (converted in each workgroup),
+    // few-row path and ProjPlan::direct: the token rows themselves (converted in each workgroup),
     // and, for kProjQKV, the projections y = x w^T + bias as F32 [N][M]
     const char* x; int x_type; int64_t x_nb_t, x_nb_b;
     float* y;
@@ -179,13 +179,19 @@ struct ProjArgs {
     // kProjQKVRope: the positions of the token rows and powf(base, -2 / d)
     const int32_t* pos; int64_t pos_stride_b;
     float theta_scale;
-    int direct;                  // kProjResidual: the GEMM's 64 x 64 tiles read x themselves (it overlaps no output)
 };
 constexpr int kMaxProjTickets = 1024;
-// K split of the GEMM of a call (1: none; *tail0 > 0: only the last round's
-// tiles) and the bytes of its partials
-int proj_ksplit(const ProjArgs& a, int n_cu, int* tail0);
-size_t proj_part_bytes(const ProjArgs& a, int n_cu);
+// How a call's GEMM runs: its tile (256 x 256: the big kernel), the pieces of
+// k (1: none; tail0 > 0: only the last round's tiles), whether Q8_0 weights are
+// dequantized to f16 (M x K) ahead of an F16 kernel, and whether the GEMM reads
+// the token rows itself (else the prep kernel's rows)
+struct ProjPlan {
+    int tm, tn, ks, tail0;
+    bool dequant, direct;
+};
+ProjPlan proj_plan(const ProjArgs& a, int n_cu);
+// bytes of the pieces' partials
+size_t proj_part_bytes(const ProjArgs& a, const ProjPlan& p);
 
 // --------------------------------------------------------- host launchers
 
@@ -247,17 +253,12 @@ bool prefill_supported(const AttnArgs& a);
 // allow_in_launch: the caller passes the tickets (otherwise the merge kernel)
 PrefillPlan prefill_plan(const AttnArgs& a, int n_cu, int forced, size_t ws_cap, bool allow_in_launch);
 size_t prefill_ws_bytes(const AttnArgs& a, const PrefillPlan& p);
-// Prep + GEMM of a linear layer; ws holds proj_ws_bytes(N, K, P) bytes where
-// the GEMM needs the prep kernel's rows.
-bool proj_needs_prep(const ProjArgs& a, int n_cu);
-// whether a call's token rows can be read by the GEMM itself
-bool proj_direct_ok(const ProjArgs& a);
+// Prep + GEMM of a linear layer.  ws holds proj_ws_bytes(N, K, P) bytes unless
+// the plan is direct; a.w names the dequantized weights where it says so, and
+// a.part proj_part_bytes.
 size_t proj_ws_bytes(int N, int K, int P);
-// Q8_0 weights over a call that the big F16 GEMM runs: the rows are
-// dequantized to f16 d * q (M x K) for it
-bool proj_dequant_q8(const ProjArgs& a, int n_cu);
 hipError_t launch_proj_dequant_q8(const ProjArgs& a, uint16_t* dst, hipStream_t s);
-hipError_t launch_proj(ProjPrepArgs& p, ProjArgs& a, void* ws, int n_cu, hipStream_t s);
+hipError_t launch_proj(ProjPrepArgs& p, ProjArgs& a, const ProjPlan& plan, void* ws, hipStream_t s);
 // Few token rows (decode steps): one weight-streaming GEMV launch that
 // converts the rows itself.  kProjQKV writes y = x w^T + bias (F32 [N][M],
 // at `ws`) for the caller's RoPE + append; kProjResidual writes h.
