@@ -693,10 +693,20 @@ __global__ void __launch_bounds__(256) prefill_merge_kernel(AttnArgs a, const fl
             const int64_t r = (int64_t)min(k0 + u, n_ks - 1) * nr_all + rg;     // clamped: unconditional loads
             e[u] = *(const float2*)(ml + r * 2);
             v[u] = *(const float4*)(ws + r * D + 4 * d4);
-            if (k0 + u >= n_ks) {                                               // (0 times an infinite sum is not 0)
-                e[u] = make_float2(-INFINITY, 0.0f);
-                v[u] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            }
+        }
+        // slots past the last split hold nothing (0 times an infinite sum is not
+        // 0): selects behind every load, not branches that wait among them
+#pragma unroll
+        for (int u = 0; u < kMergeBatch; ++u)
+            asm volatile("" : "+v"(e[u].x), "+v"(e[u].y), "+v"(v[u].x), "+v"(v[u].y), "+v"(v[u].z), "+v"(v[u].w));
+#pragma unroll
+        for (int u = 0; u < kMergeBatch; ++u) {
+            const bool in = k0 + u < n_ks;
+            e[u].x = in ? e[u].x : -INFINITY;
+            v[u].x = in ? v[u].x : 0.0f;
+            v[u].y = in ? v[u].y : 0.0f;
+            v[u].z = in ? v[u].z : 0.0f;
+            v[u].w = in ? v[u].w : 0.0f;
         }
         float mb = M;
 #pragma unroll

@@ -204,8 +204,9 @@ bool decode_supported(const AttnArgs& a);
 int decode_waves(const AttnArgs& a);            // waves per workgroup (one key sub-range each)
 int decode_max_splits();
 // Second pass of a split decode: combines the (m, l, acc) partials of `ws`
-// (layout of launch_decode) into the output rows.
-hipError_t launch_decode_merge(const AttnArgs& a, const float* ws, int n_splits, hipStream_t s);
+// (layout of launch_decode) into the output rows.  inf: partials may be
+// infinite where a V element is (F32 caches), and give infinity.
+hipError_t launch_decode_merge(const AttnArgs& a, const float* ws, int n_splits, hipStream_t s, bool inf = false);
 // LDS-streamed split-K decode over dense Q8_0 caches (T == 1): the cache
 // tiles of each split are DMA'd into a 4-stage LDS ring.  Partials use the
 // layout of launch_decode and are combined by launch_decode_merge.
