@@ -216,3 +216,32 @@ def test_vector_path_edges_equal_the_scalar_path(ctx, torch_gpu, d, Hq, Hkv, T, 
         for x, y in zip(kv.download(0, b, T + 3), kv.download(1, b, T + 3)):
             np.testing.assert_array_equal(x, y)
     kv.free()
+
+
+def test_bf16_rounding_bit_for_bit(ctx, torch_gpu):
+    """F32 V rows into a BF16 cache: nearest even on every kind of value (ties,
+    denormals, overflow to infinity, infinities), NaNs quieted with their upper
+    bits, as the integer formula has it; scalar and vector path."""
+    torch = torch_gpu
+    d, H, T = 64, 2, 4096
+    print("bf16 rounding bits", flush=True)
+    rng = np.random.default_rng(16)
+    u = rng.integers(0, 1 << 32, (1, T, H, d), dtype=np.uint64).astype(np.uint32)
+    u[0, :64] = (u[0, :64] & 0xffff0000) | 0x8000                       # ties
+    u[0, 64:96] &= 0x807fffff                                           # denormals
+    u[0, 96:128] |= 0x7f800000                                          # NaNs
+    u[0, 128, 0, :6] = [0x7f7fffff, 0xff7fffff, 0x7f800000, 0xff800000, 0x7f800001, 0x80000000]
+    nan = (u & 0x7fffffff) > 0x7f800000
+    want = np.where(nan, (u >> 16) | 0x40, (u.astype(np.uint64) + 0x7fff + ((u >> 16) & 1)) >> 16).astype(np.uint16)
+    v = torch.from_numpy(u.view(np.float32)).cuda()
+    big = torch.zeros((1, T, H, d + 8), device="cuda")
+    big[..., 2:2 + d] = v                                               # 8 bytes off: the scalar path
+    k = torch.zeros_like(v)
+    q = torch.zeros((1, T, H, d), device="cuda")
+    kv = vva.KVCache(ctx, 1, H, d, T, 1, vva.BF16)
+    for rows in (v, big[..., 2:2 + d]):
+        ctx.rope_append(kv, 0, q, k, rows, torch.zeros(T, dtype=torch.int32, device="cuda"), torch.empty_like(q))
+        torch.cuda.synchronize()
+        got = kv.download(0, 0, T)[1].view(np.uint16).reshape(T, H, d)
+        np.testing.assert_array_equal(got, want[0])
+    kv.free()

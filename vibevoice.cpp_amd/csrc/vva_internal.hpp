@@ -341,9 +341,13 @@ __device__ __forceinline__ float bf16_to_f32(uint16_t h) {
 }
 // round to nearest even; NaN kept quiet
 __device__ __forceinline__ uint16_t f32_to_bf16(float f) {
-    uint32_t x = __float_as_uint(f);
-    if ((x & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((x >> 16) | 0x40u);
-    return (uint16_t)((x + 0x7fffu + ((x >> 16) & 1u)) >> 16);
+    // v_cvt_pk_bf16_f32: nearest even, NaNs quieted, denormals kept (the bits of
+    // the integer formula for each of the 2^32 inputs, in one instruction for its
+    // six: 8 of them a lane made the vector RoPE of short calls the slower one)
+    const __bf16 b = (__bf16)f;
+    uint16_t r;
+    __builtin_memcpy(&r, &b, 2);
+    return r;
 }
 // value -> value as rounded to `type` and back (Q8_0 not handled here)
 __device__ __forceinline__ float round_to_type(float f, int type) {
