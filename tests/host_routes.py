@@ -294,8 +294,24 @@ def output_over_inputs():
                 assert st == vva.OK and kernels[0].split("<")[0] == want, kernels
 
 
+def rope_of_few_rows():
+    """Fewer than 80 rows of 64-dim heads into a Q8_0 cache take the scalar
+    kernel, other calls of aligned rows the vector one."""
+    for d, Hq, Hkv in ((64, 14, 2), (128, 28, 4)):
+        for t in (vva.F32, vva.F16, vva.BF16, vva.Q8_0):
+            for T, B in ((1, 1), (79, 1), (39, 2), (80, 1), (40, 2), (1100, 1)):
+                c = Host()
+                kv = c.kv(Hkv, d, T, B, t, [0] * B)
+                q, k, v = (c.tensor(vva.F32, [d, h, T, B]) for h in (Hq, Hkv, Hkv))
+                qo, pos = c.tensor(vva.F32, [d, Hq, T, B]), c.tensor(vva.I32, [T])
+                st, kernels, _ = c.call("vva_rope_append", kv, 0, ref(q), ref(k), ref(v), ref(pos), None, 1e6, ref(qo))
+                scalar = d == 64 and t == vva.Q8_0 and T * B < 80
+                assert st == vva.OK and kernels[0].split("<")[0] == ("rope_append_kernel" if scalar else
+                                                                     "rope_append_vec_kernel"), (d, t, T, B, kernels)
+
+
 SCENARIOS = [bf16_v_window, one_token_precision, workspace_one_can_do_without, f32_step_without_workspace,
-             step_output_alignment, output_over_inputs]
+             step_output_alignment, output_over_inputs, rope_of_few_rows]
 
 if __name__ == "__main__":
     {f.__name__: f for f in SCENARIOS}[sys.argv[1]]()

@@ -7,7 +7,8 @@
 // rotated Q is written in the attention's input type.
 //
 // rope_append_vec_kernel takes head dims 64 and 128 with aligned rows, every
-// cache type; rope_append_kernel the rest.
+// cache type; rope_append_kernel the rest, and few rows of 64-dim heads into a
+// Q8_0 cache.
 //
 // rope_append_kernel: one workgroup per (token t, batch b), 256 threads.
 // Threads 0..d/2-1 first build the angle table of the token in LDS with the
@@ -285,9 +286,15 @@ hipError_t launch_rope_append(const RopeAppendArgs& a, hipStream_t s) {
     if (a.T <= 0 || a.B <= 0) return hipSuccess;
     const int items = ((a.do_q ? a.Hq : 0) + (a.do_kv ? 2 * a.Hkv : 0)) * (a.d / 2);
     if (items <= 0) return hipSuccess;
-    if (rope_vec_ok(a)) {
+    const int64_t n = (int64_t)a.T * a.B;
+    // Few rows of 64-dim heads into a Q8_0 cache: the scalar kernel's workgroups
+    // (3 a token at 0.5B heads) fit the CUs and its lanes have one pair each to
+    // quantize (us per call, 9 rows 4.00 against 4.16 of the vector kernel, 64
+    // rows 4.11 against 4.25 (BF16 input 4.37); 100 rows 4.32 against 4.25; 128-dim
+    // heads, 9 rows 4.72 against 3.96).
+    const bool few_q8 = a.d == 64 && n < 80 && a.do_kv && a.cache_type == VVA_TYPE_Q8_0;
+    if (!few_q8 && rope_vec_ok(a)) {
         const int per_tok = items / 8;
-        const int64_t n = (int64_t)a.T * a.B;
         // Tokens per workgroup: short calls need the workgroups (512 tokens at
         // 7B heads, BF16 in, Q8_0 cache: 5.9 us at 1 in slices of 256 items,
         // 6.5 unsliced, 8.6 at 2), long ones pay less per token for the angles
