@@ -149,15 +149,15 @@ def one_token_precision():
             assert st == vva.OK and kernels[1].split("<")[0] == "attn_rows_kernel", kernels
 
 
-def proj_call(mode, wt, heads, N, T=None, xt=vva.F32, cache=vva.F16, host=None, **kw):
+def proj_call(mode, wt, heads, N, T=None, xt=vva.F32, cache=vva.F16, host=None, stride=0, **kw):
     """vva_qkv_rope_append ("qkv") or vva_out_proj_residual ("out") of N token
-    rows: status, kernels, allocations."""
+    rows: status, kernels, allocations.  stride: bytes of a weight row, if not dense."""
     c = host or Host()
     d, Hq, Hkv, hidden = heads
     T = T or N
     B = N // T
     def weight(M, K):
-        return c.tensor(wt, [K, M])
+        return c.tensor(wt, [K, M], [ES[wt], stride, stride * M, stride * M] if stride else None)
     if mode == "out":
         o, x, h = c.tensor(xt, [Hq * d, T, B]), c.tensor(vva.F32, [hidden, T, B]), c.tensor(vva.F32, [hidden, T, B])
         return c.call("vva_out_proj_residual", ref(o), ref(weight(hidden, Hq * d)), ref(x), ref(h), **kw)
@@ -310,8 +310,57 @@ def rope_of_few_rows():
                                                                      "rope_append_vec_kernel"), (d, t, T, B, kernels)
 
 
+def gemm_of(kernels, grids):
+    """(kernel, tile rows, tile columns, workgroups, dequantized weights)"""
+    i = next(i for i, k in enumerate(kernels) if "gemm" in k)
+    k, wgs = kernels[i], int(grids[i].split(",")[0])
+    name = k.split("<")[0][len("proj_gemm_"):]
+    a = k.split("<")[1].rstrip(">").split(", ")
+    tm, tn = (int(a[2]), int(a[3])) if name == "kernel" else (256, 128) if name.startswith("wide") else (256, 256)
+    return name.split("_")[0], tm, tn, wgs, "vva::proj_dequant_q8_kernel" in kernels
+
+
+def projection_plans():
+    """The GEMM's plan over shapes: the tiles cover the rows, a tile of
+    proj_gemm_kernel lies in one matrix, its pieces are resident at once and
+    within the tickets, dequantized weights meet an F16 kernel of whole 256
+    rows; and matrices past the reach of the wide and the big kernel's offsets
+    stay with the small tiles."""
+    for heads in (H05, H15, H7, (128, 8, 8, 1024), (64, 2, 2, 64)):
+        d, Hq, Hkv, hidden = heads
+        for wt in (vva.F16, vva.Q8_0):
+            for mode, rows, K in (("qkv", [Hq * d, Hkv * d], hidden), ("out", [hidden], Hq * d)):
+                if any(r % 128 for r in rows):
+                    continue
+                M = sum(rows) + (rows[1] if mode == "qkv" else 0)
+                for N in [*range(9, 1100, 13), *range(1100, 9000, 171)]:
+                    c = Host()
+                    st, kernels, _ = proj_call(mode, wt, heads, N, host=c)
+                    assert st == vva.OK, c.err()
+                    name, tm, tn, wgs, dq = gemm_of(kernels, c.grids)
+                    tiles = -(-M // tm) * -(-N // tn)
+                    if name == "kernel":
+                        ks = wgs // tiles
+                        assert all(r % tm == 0 for r in rows) and wgs == tiles * ks and not dq
+                        assert 1 <= ks <= 4 and (ks == 1 or (wgs <= 512 and tiles <= 1024 and K // 64 >= 4 * ks))
+                    else:
+                        assert wgs == tiles if name == "wide" else wgs >= tiles
+                        assert (wt == vva.Q8_0) == dq and (not dq or N >= 1024)
+    # 900 rows of the 7B q/k/v: one round of wide tiles, not 288 of 128 x 128
+    c = Host()
+    assert gemm_of(proj_call("qkv", vva.F16, H7, 900, host=c)[1], c.grids)[0] == "wide"
+    # weight rows 8 MiB apart: more than 1 GiB of a matrix, 2 GiB of 256 rows
+    for wt in (vva.F16, vva.Q8_0):
+        for N in (1000, 3000):
+            c = Host()
+            st, kernels, _ = proj_call("qkv", wt, H7, N, host=c, stride=1 << 23)
+            name, tm, *_ = gemm_of(kernels, c.grids)
+            assert st == vva.OK and (tm < 256 or (wt == vva.Q8_0 and N >= 1024)), (wt, N, kernels)
+
+
 SCENARIOS = [bf16_v_window, one_token_precision, workspace_one_can_do_without, f32_step_without_workspace,
-             step_output_alignment, output_over_inputs, rope_of_few_rows]
+             step_output_alignment, output_over_inputs, rope_of_few_rows,
+             projection_plans]
 
 if __name__ == "__main__":
     {f.__name__: f for f in SCENARIOS}[sys.argv[1]]()

@@ -351,29 +351,35 @@ def test_4096_token_projection_with_split_tail(ctx, torch_gpu, wt):
 
 
 TILE_CASES = [
-    # hidden, Hq, Hkv, d, weights, cache, T, B: the tile and pieces of k that the call takes
+    # hidden, Hq, Hkv, d, weights, cache, T, B: the kernels of the q/k/v and the output call
     (896, 14, 2, 64, vva.F16, vva.F16, 7, 1),        # 64 x 64 for 7 rows of F16 weights
     (3584, 28, 4, 128, vva.F16, vva.Q8_0, 1, 4),     # and for 4 rows of the largest ones
     (1024, 14, 2, 64, vva.Q8_0, vva.F32, 3, 1),      # GEMV, half waves, all 32 blocks
     (1088, 12, 2, 128, vva.Q8_0, vva.F16, 3, 2),     # GEMV, one round of blocks
-    (2112, 12, 2, 128, vva.Q8_0, vva.Q8_0, 4, 1),    # GEMV, two rounds of blocks
+    (2112, 12, 2, 128, vva.Q8_0, vva.Q8_0, 4, 1),    # GEMV, two rounds of blocks (x at odd strides: 64 x 64)
     (64, 2, 2, 64, vva.F16, vva.F16, 9, 1),          # 64 x 64, one k step (fewer than loads in flight), 9 rows
     (384, 14, 2, 64, vva.Q8_0, vva.Q8_0, 65, 1),     # 64 x 64, a second token tile of one row
     (448, 2, 1, 128, vva.Q8_0, vva.Q8_0, 33, 2),     # 64 features of a 128-dim head, Q8_0 cache (pair epilogue)
-    (832, 2, 1, 128, vva.F16, vva.BF16, 63, 1),      # the same, vector epilogue, 13 steps
-    (1536, 12, 2, 128, vva.Q8_0, vva.F32, 20, 1),    # 64 x 64 in pieces of k
+    (832, 2, 1, 128, vva.F16, vva.BF16, 63, 1),      # the same, vector epilogue, 13 steps in pieces
+    (1536, 12, 2, 128, vva.Q8_0, vva.F32, 20, 1),    # 64 x 64 in four pieces of k
     (896, 14, 2, 64, vva.F16, vva.Q8_0, 130, 1),     # two token rows past the second tile
     (1536, 12, 2, 128, vva.F16, vva.F16, 37, 3),     # pieces of k, three sequences
     (64, 2, 2, 64, vva.F16, vva.F32, 10, 1),         # F16 x
-    (3584, 28, 4, 128, vva.F16, vva.Q8_0, 31, 2),    # the same, pair epilogue
-    (320, 14, 2, 64, vva.Q8_0, vva.F16, 1400, 1),    # 64 x 128
-    (640, 28, 4, 128, vva.F16, vva.Q8_0, 385, 1),    # 64 x 128 or 64 x 64, ragged token tile, pair epilogue
-    (3584, 28, 4, 128, vva.Q8_0, vva.Q8_0, 513, 1),  # 128 x 128 in pieces
-    (192, 28, 4, 128, vva.Q8_0, vva.BF16, 500, 1),   # 128 x 128 or 64 x 64, 3 steps
+    (3584, 28, 4, 128, vva.F16, vva.Q8_0, 31, 2),    # pieces, pair epilogue
+    (320, 14, 2, 64, vva.Q8_0, vva.F16, 1400, 1),    # 64 x 128; 64 x 64
+    (640, 28, 4, 128, vva.F16, vva.Q8_0, 385, 1),    # 64 x 64, ragged token tile, pair epilogue
+    (3584, 28, 4, 128, vva.Q8_0, vva.Q8_0, 513, 1),  # 128 x 128; in three pieces
+    (192, 28, 4, 128, vva.Q8_0, vva.BF16, 500, 1),   # 64 x 128, 3 steps
     (192, 12, 2, 128, vva.Q8_0, vva.Q8_0, 4001, 1),  # 256 x 128, 3 steps, pair epilogue
-    (1536, 12, 2, 128, vva.F16, vva.F16, 1500, 2),   # 256 x 128, two sequences
+    (1536, 12, 2, 128, vva.F16, vva.F16, 1500, 2),   # wide, two sequences
     (3584, 28, 4, 128, vva.F16, vva.Q8_0, 3001, 1),  # 256 x 256, pair epilogue, ragged
     (3584, 28, 4, 128, vva.Q8_0, vva.F16, 1501, 2),  # 256 x 256 on dequantized weights, two sequences
+    (896, 14, 2, 64, vva.F16, vva.Q8_0, 3701, 1),    # wide, half a weight tile past the last row, pair epilogue
+    (3584, 28, 4, 128, vva.F16, vva.BF16, 301, 3),   # wide, vector epilogue, three sequences, 7 rows in the last tile
+    (3584, 28, 4, 128, vva.Q8_0, vva.Q8_0, 1100, 1), # wide on dequantized weights; 128 x 128
+    (3584, 28, 4, 128, vva.Q8_0, vva.F16, 951, 1),   # Q8_0 256 x 128; 128 x 128
+    (3584, 28, 4, 128, vva.F16, vva.F16, 485, 1),    # 128 x 128 in pieces; 64 x 128
+    (1536, 12, 2, 128, vva.F16, vva.Q8_0, 6001, 1),  # 128 x 128 or 256 x 256 (half the CUs)
 ]
 
 

@@ -15,11 +15,14 @@
 // ggml's integer block sums; each is below 2^-12 relative.)
 //
 // GEMM.  D[m][n] = sum_k W[m][k] X[n][k]: m = output feature, n = token row
-// (b * T + t), k = input feature.  Two kernels, chosen by gemm_plan: tiles of
-// 64 x 64 to 256 x 128 over either weight type (proj_gemm_kernel),
-// and 256 x 256 tiles over F16 weights for calls that fill the chip with them
-// (proj_gemm_big_kernel).  Both operands are k-contiguous rows, so every
-// v_mfma_f32_32x32x16_f16 fragment is one 16-byte LDS read.
+// (b * T + t), k = input feature.  Three kernels, chosen by proj_plan: tiles of
+// 64 x 64 to 128 x 128 over either weight type and of 256 x 128 over Q8_0
+// weights (proj_gemm_kernel), 256 x 128 tiles over F16 weights, one workgroup
+// per CU (proj_gemm_wide_kernel), and 256 x 256 tiles over F16 weights for calls
+// that fill the chip with them (proj_gemm_big_kernel).  Q8_0 weights of a long
+// call are dequantized to f16 ahead of the latter two.  Both operands are
+// k-contiguous rows, so every v_mfma_f32_32x32x16_f16 fragment is one 16-byte
+// LDS read.
 //
 // proj_gemm_kernel: 4 or 8 waves, each a share of 32 x 32 blocks, k in steps of
 // 64.  Tiles are staged through registers into two LDS stages of rows padded
@@ -731,7 +734,7 @@ constexpr int kBCBytes = kBHalf * kBCPitch * 4;
 constexpr int kBLds = kBRing > kBCBytes ? kBRing : kBCBytes;
 constexpr int kBPiece = kBWaves * 8 * 4096;     // bytes of one K piece's accumulators (256 x 256 f32)
 constexpr int kBMaxSplit = 8;
-constexpr int kBigMinRows = 1024;             // fewest token rows of a big GEMM (gemm_plan)
+constexpr int kBigMinRows = 1024;             // fewest token rows of a big GEMM (proj_plan)
 static_assert(kBStages == 2 && kBStages * kBLoads <= 63, "two stages of a wave's loads fit its 6-bit vmcnt");
 static_assert(kBLds <= 160 * 1024, "LDS");
 
@@ -818,7 +821,7 @@ __device__ __forceinline__ void residual_epilogue(const ProjArgs& a, const float
     }
 }
 
-// Tile order of the big GEMM: XCD x (workgroup i runs on XCD i % 8) takes a
+// Tile order of the big and the wide GEMM: XCD x (workgroup i runs on XCD i % 8) takes a
 // contiguous run of an order that walks groups of 4 token tiles, the 4 token
 // tiles of every weight tile in turn.  Returns (weight tile, token tile) of
 // place wo.
@@ -841,6 +844,158 @@ __device__ __forceinline__ void big_split_store(const f32x16 (&acc)[4][2], char*
                                  __float_as_uint(acc[i][j][4 * g + 2]), __float_as_uint(acc[i][j][4 * g + 3])};
                 __builtin_amdgcn_raw_buffer_store_b128(v, rs, (w * 32 + (i * 2 + j) * 4 + g) * 1024 + lane * 16, 0, 0);
             }
+}
+
+// ------------------------------------------------------------ wide GEMM (F16 weights)
+
+// 256 output features x 128 token rows per workgroup, k in steps of 64.
+// Eight producer waves DMA the tiles straight into a 3-stage LDS ring
+// (buffer_load_dwordx4 ... lds).  From L2 one wave's LDS loads stream at
+// ~20 GB/s whatever their number in flight, so eight issuing waves are what
+// a CU needs to feed its matrix cores (~110 GB/s at this tile shape); the
+// compute waves issue none, so they never wait behind a full load queue.
+// Eight compute waves, two per SIMD, each own a 64 x 64 quadrant of 2 x 2
+// v_mfma_f32_32x32x16_f16 blocks.  Rows are 128 bytes (64 f16 of k) in LDS;
+// a DMA instruction fills 8 rows, and its lane l writes LDS 16-byte slot
+// l % 8 of row l / 8 with the row's 16-byte k chunk (l % 8) ^ sw(row),
+// sw(row) = (row / 2) % 8: a fragment read (16 lanes x 16 bytes per LDS
+// cycle, rows r .. r + 15 at one k chunk) then touches every bank once.
+// (proj_gemm_kernel's register ring at this tile takes 1.1 us a step against
+// 1.0: 7B q/k/v, 1000 rows 69.4 us against 61.8.)
+constexpr int kWM = 256, kWN = 128, kWK = 64;
+constexpr int kWStages = 3;
+constexpr int kWA = kWM * kWK * 2;             // 32 KB of weights per stage
+constexpr int kWB = kWN * kWK * 2;             // 16 KB of token rows per stage
+constexpr int kWStage = kWA + kWB;
+constexpr int kWCompute = 8, kWProd = 8;
+constexpr int kWLoadsA = kWA / 1024 / kWProd;  // DMA loads per producer and stage
+constexpr int kWLoadsB = kWB / 1024 / kWProd;
+constexpr int kWLoads = kWLoadsA + kWLoadsB;
+constexpr int kWCPitch = kWM + 4;              // floats per token row of the epilogue tile
+static_assert(2 * kWLoads <= 63, "two stages of a producer's loads fit its 6-bit vmcnt");
+static_assert(kWN * kWCPitch * 4 <= kWStages * kWStage, "the epilogue tile reuses the ring");
+
+__device__ __forceinline__ void wlds_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : : : "memory");
+}
+
+template <int MODE>
+__global__ void __launch_bounds__((kWCompute + kWProd) * 64) proj_gemm_wide_kernel(ProjArgs a) {
+    prefetch_kernargs<sizeof(ProjArgs)>();
+    __shared__ __attribute__((aligned(16))) char lds[kWStages * kWStage];
+    const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, l32 = lane & 31;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+
+    // the big kernel's tile order: the tiles an XCD runs at one time share few
+    // weight and token rows in its L2
+    const int n_mt = (a.M + kWM - 1) / kWM, n_nt = (a.N + kWN - 1) / kWN;
+    const int q = gridDim.x / 8, r = gridDim.x % 8, x = blockIdx.x % 8;
+    const int2 mn = big_order(x * q + min(x, r) + (int)blockIdx.x / 8, n_mt, n_nt);
+    const int m0 = mn.x * kWM, n0 = mn.y * kWN;
+    const int nk = a.K / kWK;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
+
+    if (w >= kWCompute) {
+        // ---- producers: chunks p, p + 8, ... of each operand's stage
+        const int pw = w - kWCompute;
+        const int sub = lane >> 3, slot = lane & 7;
+        int aoff[kWLoadsA], boff[kWLoadsB];
+        i32x4 ars[kWLoadsA];
+#pragma unroll
+        for (int i = 0; i < kWLoadsA; ++i) {
+            const int row = (pw + kWProd * i) * 8 + sub;            // tile row of this lane
+            const int g = m0 + (pw + kWProd * i) * 8;               // its 8-row group (one matrix)
+            const int mat = g < a.m_end[0] ? 0 : (g < a.m_end[1] ? 1 : (g < a.m_end[2] ? 2 : 3));
+            const int mbeg = mat == 0 ? 0 : a.m_end[mat - 1];
+            const int mrows = mat < 3 ? a.m_end[mat] - mbeg : 0;
+            ars[i] = make_rsrc_sgpr(mat < 3 ? a.w[mat] : a.w[0], (uint32_t)(mrows * a.w_nb[mat < 3 ? mat : 0]));
+            const int mr = m0 + row - mbeg;
+            aoff[i] = mr * (int)a.w_nb[mat < 3 ? mat : 0] + (((slot ^ ((row >> 1) & 7))) << 4);
+        }
+        const int nrows = min(a.N - n0, kWN);
+        const i32x4 brs = make_rsrc_sgpr((const char*)(a.xh + (int64_t)n0 * a.K), (uint32_t)(nrows * a.K * 2));
+#pragma unroll
+        for (int i = 0; i < kWLoadsB; ++i) {
+            const int row = (pw + kWProd * i) * 8 + sub;
+            boff[i] = row * a.K * 2 + (((slot ^ ((row >> 1) & 7))) << 4);
+        }
+        // a stage past the last loads zeros (offsets past every range)
+        auto issue = [&](int kt) {
+            const uint32_t st = lds0 + (uint32_t)(kt % kWStages) * kWStage;
+            const bool live = kt < nk;
+            const int ko = kt * kWK * 2;
+#pragma unroll
+            for (int i = 0; i < kWLoadsA; ++i)
+                wdma16(ars[i], st + (pw + kWProd * i) * 1024, live ? aoff[i] + ko : 0x40000000);
+#pragma unroll
+            for (int i = 0; i < kWLoadsB; ++i)
+                wdma16(brs, st + kWA + (pw + kWProd * i) * 1024, live ? boff[i] + ko : 0x40000000);
+        };
+        issue(0);
+        issue(1);
+        for (int kt = 0; kt < nk; ++kt) {
+            wwait_barrier<kWLoads>();                      // T_kt: stage kt landed
+            issue(kt + 2);                                 // into the stage of kt - 1
+        }
+        asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
+        __syncthreads();                                   // every wave is done with the ring
+        __syncthreads();                                   // the epilogue tile is written
+        return;
+    }
+
+    // ---- compute waves: quadrant (wm, wn) of 64 features x 64 tokens
+    const int wm = w & 3, wn = w >> 2;
+    const int sw = (l32 >> 1) & 7;
+    const int a_rd = (wm * 64 + l32) * 128;
+    const int b_rd = kWA + (wn * 64 + l32) * 128;
+    f32x16 acc[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = f32x16{};
+    for (int kt = 0; kt < nk; ++kt) {
+        wlds_barrier();                                    // T_kt
+        const char* st = lds + (kt % kWStages) * kWStage;
+#pragma unroll
+        for (int ks = 0; ks < kWK / 16; ++ks) {
+            const int ch = ((2 * ks + half) ^ sw) << 4;
+            h8 af[2], bf[2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const u32x4 ua = *(const u32x4*)(st + a_rd + i * 32 * 128 + ch);
+                const u32x4 ub = *(const u32x4*)(st + b_rd + i * 32 * 128 + ch);
+                __builtin_memcpy(&af[i], &ua, 16);
+                __builtin_memcpy(&bf[i], &ub, 16);
+            }
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i], bf[j], acc[i][j], 0, 0, 0);
+        }
+    }
+    __syncthreads();                                       // every wave is done with the ring
+
+    // ---- accumulators to LDS as C[token][feature]: lane (half, l32) of
+    // block (i, j) holds features 8 (r / 4) + 4 half + r % 4 of token l32
+    float* C = (float*)lds;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            float* crow = C + (wn * 64 + 32 * j + l32) * kWCPitch + wm * 64 + 32 * i + 4 * half;
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+                *(float4*)(crow + 8 * g) = make_float4(acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2],
+                                                       acc[i][j][4 * g + 3]);
+        }
+    __syncthreads();
+    if constexpr (MODE == kProjQKV) {
+        if (a.vec_store) qkv_epilogue_vec<kWM, kWN, kWCompute * 64>(a, C, kWCPitch, m0, n0, tid);
+        else             qkv_epilogue_pair<kWN, kWCompute * 64>(a, C, kWCPitch, m0, n0, tid);
+    } else {
+        residual_epilogue<kWN, kWCompute * 64>(a, C, kWCPitch, m0, n0, tid);
+    }
 }
 
 template <int MODE>
@@ -2274,70 +2429,37 @@ hipError_t launch_proj_gemv(ProjArgs& a, float* y_ws, int n_cu, hipStream_t s) {
 namespace {
 constexpr int kDqMaxK = 8192;                  // inputs of a Q8_0 row that proj_dequant_q8_kernel holds
 // Kernel, tile and K pieces of a call: the least of the estimates (us)
-//   steps x workgroups per CU x time of a step + cost of exchanging the pieces.
-// The times of a step are measured ones (0.5B, 1.5B and 7B shapes, 16 to 4096
-// token rows), of a workgroup that has its CU to itself and of one of several
-// on it; between one and 1.6 workgroups per CU the fuller CUs set the time.
-// Pieces are for calls whose workgroups are all resident at once.  At the
-// choices that fall out (us of the whole call, prep included; the kernel that
-// runs against the next best one): q/k/v 0.5B, 257 rows 13.8 (64 x 64) against
-// 17.3 (64 x 128); 7B, 64 rows 18.8 (3 pieces) against 25.3 (one); 7B, 512 rows
-// 45.6 (128 x 128, 3 pieces) against 50.4 (64 x 64); 7B output, 1024 rows 48.1
-// (128 x 128) against 53.4 (the big kernel); 7B q/k/v, 1024 rows 69.5 (256 x
-// 128) against 80.7 (64 x 128) and 112 (the big kernel); 7B q/k/v, 3000 rows
-// 132 (the big kernel) against 151 (256 x 128); 1.5B q/k/v, 4096 rows 57.5
-// (256 x 128) against 76.1 (the big kernel, whose 128 tiles leave half the CUs
-// idle).  What sets the larger tiles' steps is the operands' way from L2:
-// ~9 TB/s over the chip, at every tile size.
-// `direct`: the 64 x 64 tiles may read x themselves.
-ProjPlan gemm_plan(const ProjArgs& a, bool q8, bool direct, int n_cu) {
-    struct Tile { int tm, tn; double lone, shared, merge, merge_x; };   // merge_x: per workgroup and CU
-    static const Tile kF16[] = {{64, 64, 0.28, 0.33, 2.3, 0.5}, {64, 128, 0.45, 0.55, 4.0, 0.0}, {128, 128, 0.85, 0.85, 9.0, 0.0},
-                                {256, 128, 1.20, 1.20, 0.0, 0.0}};
-    static const Tile kQ8[] = {{64, 64, 0.33, 0.40, 2.3, 0.5}, {64, 128, 0.50, 0.62, 4.0, 0.0}, {128, 128, 0.95, 0.95, 9.0, 0.0},
-                               {256, 128, 1.35, 1.35, 0.0, 0.0}};
-    const int nk = a.K / kTK;
-    ProjPlan best{64, 64, 1, 0, false, direct};
-    double best_us = 1e30;
-    // a tile lies in one matrix (every matrix has a multiple of 128 rows); 256
-    // rows never came first below kBigMinRows token rows, nor in pieces
-    const bool m256 = a.N >= kBigMinRows && a.M % 256 == 0 && a.m_end[0] % 256 == 0 && a.m_end[1] % 256 == 0;
-    for (const Tile& t : q8 ? kQ8 : kF16) {
-        if (t.tm == 256 && !m256) continue;
-        const int64_t tiles = (int64_t)(a.M / t.tm) * ((a.N + t.tn - 1) / t.tn);
-        for (int ks = 1; ks <= 4; ++ks) {
-            if (ks > 1 && (t.tm == 256 || tiles > kMaxProjTickets || tiles * ks > 2 * n_cu || nk < 4 * ks)) break;
-            double x = (double)(tiles * ks) / n_cu;
-            if (t.tm == 256) x = std::ceil(x);                 // one workgroup per CU
-            double us = (double)nk / ks * (x <= 1.0 ? t.lone : std::max(1.6, x) * t.shared) +
-                        (ks > 1 ? t.merge + t.merge_x * x : 0.0);
-            if (t.tn == 64 && direct) us -= 3.5;    // no prep launch
-            if (us < best_us) {
-                best_us = us;
-                best = ProjPlan{t.tm, t.tn, ks, 0, false, direct && t.tn == 64};
-            }
-        }
-    }
-    // the big kernel: 1.45 us a step and 25 us around them, whatever the share
-    // of the CUs that its tiles fill; Q8_0 weights are dequantized for it first
-    if (a.N >= kBigMinRows && !(q8 && a.K > kDqMaxK)) {
-        const int64_t tiles = (int64_t)((a.M + kBM - 1) / kBM) * ((a.N + kBN - 1) / kBN);
-        const int64_t tail = tiles % n_cu;
-        const double rounds = (double)(tiles / n_cu) + (tail == 0 ? 0.0 : (tiles > n_cu && 4 * tail <= n_cu) ? 0.6 : 1.0);
-        const double us = rounds * (25.0 + 1.45 * nk) + (q8 ? 2.0 + (double)a.M * a.K * 6.4e-7 : 0.0);
-        if (us < best_us) {
-            best = ProjPlan{kBM, kBN, 1, 0, q8, false};
-            // the last round's tiles, when they fill at most a quarter of the CUs,
-            // split along K (at most kBMaxSplit pieces of at least 8 k steps)
-            if (tail > 0 && 4 * tail <= n_cu && tail <= kMaxProjTickets && nk >= 16) {
-                best.ks = (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(kBMaxSplit, n_cu / tail), nk / 8));
-                best.tail0 = (int)(tiles - tail);
-            }
-        }
-    }
-    return best;
-}
-// the output projection, F16 weights, 16-byte aligned rows within 32-bit offsets
+//   prep + (k steps x time of a step + epilogue) x G(x) + exchange of the pieces,
+// x workgroups per CU and G the share of the time that they take from each
+// other: 1 up to x = 1, beyond that the fuller CUs set it.  The constants are a
+// fit to the measured calls of every tile in 1 to 4 pieces at 0.5B, 1.5B and 7B
+// shapes and at 8 heads of 128 over 1024 inputs, 9 to 8192 token rows (1520
+// shapes; the tile that falls out takes 0.4 % more than the best one on average,
+// 13 % at most).  Some of its lines, us of the whole call: q/k/v 7B F16, 896
+// rows 57.8 (128 x 128; 64 x 128 59.0), 900 rows 59.8 (256 x 128; 128 x 128
+// 77.1), 2000 rows 121 (256 x 256; 128 x 128 151); 1.5B output, 2048 rows 28.3
+// (128 x 128; 64 x 64 45.3); 7B output, 2500 rows 103 (256 x 256; 256 x 128
+// 108), Q8_0 109 (dequantized; 128 x 128 126).  What sets the larger tiles'
+// steps is the operands' way from L2: ~9 TB/s over the chip.
+struct TileCost {
+    int tm, tn;
+    double step, epi_qkv, epi_out;                     // us: a step, the epilogue by mode
+    double share, blend, knee;                         // G past x = 1: max(knee, share (blend x + (1 - blend) ceil x))
+    double merge, merge_x;                             // pieces: merge + merge_x x
+};
+const TileCost kF16Tiles[] = {{64, 64, 0.312, 3.9, 3.3, 0.65, 0.0, 1.64, 1.0, 2.7},
+                              {64, 128, 0.381, 6.9, 5.4, 0.78, 0.0, 1.37, 4.1, 0.0},
+                              {128, 128, 0.718, 11.5, 7.4, 0.74, 0.61, 1.33, 5.4, 0.0}};
+const TileCost kF16Direct = {64, 64, 0.368, 2.3, 1.9, 0.82, 0.14, 1.5, 1.6, 2.5};      // F32 rows: twice the bytes
+const TileCost kF16Wide = {256, 128, 0.645, 13.4, 1.8, 0.94, 0.0, 2.5, 0.0, 0.0};
+const TileCost kQ8Tiles[] = {{64, 64, 0.384, 3.5, 0.8, 0.89, 0.0, 1.67, 0.0, 2.8},
+                             {64, 128, 0.504, 4.8, 2.6, 0.9, 0.15, 1.13, 4.0, 0.7},
+                             {128, 128, 0.719, 11.3, 3.9, 0.81, 0.49, 1.5, 8.0, 1.7},
+                             {256, 128, 1.063, 12.2, 6.8, 1.23, 0.24, 2.19, 0.0, 0.0}};
+constexpr double kDirectUs = 0.3;                      // in place of the prep
+
+// Whether the 64 x 64 tiles may read x themselves: the output projection, F16
+// weights, 16-byte aligned rows within 32-bit offsets
 bool direct_ok(const ProjArgs& a) {
     return a.mode == kProjResidual && a.w_type == VVA_TYPE_F16 && (uintptr_t)a.x % 16 == 0 && a.x_nb_t % 16 == 0 && a.x_nb_b % 16 == 0 &&
            a.x_nb_t >= 0 && a.x_nb_b >= 0 &&
@@ -2346,14 +2468,73 @@ bool direct_ok(const ProjArgs& a) {
 }  // namespace
 
 ProjPlan proj_plan(const ProjArgs& a, int n_cu) {
-    const bool q8 = a.w_type == VVA_TYPE_Q8_0;
-    ProjPlan p = gemm_plan(a, q8, direct_ok(a), n_cu);
-    if (p.dequant) {
-        // the weights are f16 then: the best F16 kernel (x in its Q8_0 round trip: the prep's rows)
-        p = gemm_plan(a, false, false, n_cu);
-        p.dequant = true;
+    const bool q8 = a.w_type == VVA_TYPE_Q8_0, qkv = a.mode == kProjQKV, direct = direct_ok(a);
+    const int nk = a.K / kTK;
+    const double NK = (double)a.N * a.K * 1e-6;
+    const double prep = q8 ? 4.48 + 0.98 * NK : 3.54 + 0.59 * NK;
+    ProjPlan best{64, 64, 1, 0, false, false};
+    double best_us = 1e30;
+    auto offer = [&](double us, const ProjPlan& p) {
+        if (us < best_us) {
+            best_us = us;
+            best = p;
+        }
+    };
+    auto price = [&](const TileCost& t, int64_t wgs, int ks) {
+        const double x = (double)wgs / n_cu;
+        const double G = x <= 1.0 ? 1.0 : std::max(t.knee, t.share * (t.blend * x + (1.0 - t.blend) * std::ceil(x)));
+        return ((double)nk / ks * t.step + (qkv ? t.epi_qkv : t.epi_out)) * G + (ks > 1 ? t.merge + t.merge_x * x : 0.0);
+    };
+    auto tiles_of = [&](int tm, int tn) { return (int64_t)((a.M + tm - 1) / tm) * ((a.N + tn - 1) / tn); };
+    // bytes of the largest matrix (wnb: its row stride, 0: as it is)
+    auto matrix_bytes = [&](int64_t wnb) {
+        int64_t most = 0;
+        for (int i = 0, m0 = 0; i < 3; m0 = a.m_end[i], ++i)
+            most = std::max(most, (int64_t)(a.m_end[i] - m0) * (wnb ? wnb : a.w_nb[i]));
+        return most;
+    };
+    // proj_gemm_kernel: a tile lies in one matrix (every matrix has a multiple of
+    // 128 rows), its rows within 2 GiB; pieces of 4 steps at least, all resident at once
+    auto small = [&](const TileCost& t, bool dir) {
+        if (t.tm == 256 && (a.N <= 256 || a.M % 256 || a.m_end[0] % 256 || a.m_end[1] % 256 ||
+                            std::max({a.w_nb[0], a.w_nb[1], a.w_nb[2]}) >= ((int64_t)1 << 23)))
+            return;
+        const int64_t tiles = tiles_of(t.tm, t.tn);
+        for (int ks = 1; ks <= 4; ++ks) {
+            if (ks > 1 && (t.tm == 256 || tiles > kMaxProjTickets || tiles * ks > 2 * n_cu || nk < 4 * ks)) break;
+            offer((dir ? kDirectUs : prep) + price(t, tiles * ks, ks), ProjPlan{t.tm, t.tn, ks, 0, false, dir});
+        }
+    };
+    // the wide and the big kernel, which take F16 weights (`dq`: dequantized ones)
+    // of any 128 rows and read zeros past 1 GiB of a matrix
+    auto large = [&](double extra, bool dq) {
+        if (a.N > 256) offer(extra + prep + price(kF16Wide, tiles_of(256, 128), 1), ProjPlan{256, 128, 1, 0, dq, false});
+        if (a.N < kBigMinRows) return;
+        const int64_t tiles = tiles_of(kBM, kBN), tail = tiles % n_cu;
+        ProjPlan p{kBM, kBN, 1, 0, dq, false};
+        const double round = 0.876 * nk + (qkv ? 33.5 : 11.5);
+        double us = extra + prep + (double)(tiles / n_cu) * round + (tail ? round : 0.0);
+        // the last round's tiles, when they fill at most a quarter of the CUs,
+        // split along K (at most kBMaxSplit pieces of at least 8 k steps)
+        if (tail > 0 && 4 * tail <= n_cu && tail <= kMaxProjTickets && nk >= 16) {
+            p.ks = (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(kBMaxSplit, n_cu / tail), nk / 8));
+            p.tail0 = (int)(tiles - tail);
+            if (p.ks > 1) us += 0.2 * round / p.ks + 4.4 + 40.0 * tail * p.ks / n_cu - round;
+        }
+        offer(us, p);
+    };
+    const int64_t kReach = (int64_t)1 << 30;
+    if (q8) {
+        for (const TileCost& t : kQ8Tiles) small(t, false);
+        if (a.N >= kBigMinRows && a.K <= kDqMaxK && matrix_bytes((int64_t)a.K * 2) < kReach)
+            large(5.5 + (double)a.M * a.K * 0.49e-6, true);
+    } else {
+        for (const TileCost& t : kF16Tiles)
+            if (!(direct && t.tn == 64)) small(t, false);
+        if (direct) small(kF16Direct, true);
+        if (matrix_bytes(0) < kReach) large(0.0, false);
     }
-    return p;
+    return best;
 }
 size_t proj_part_bytes(const ProjArgs& a, const ProjPlan& p) {
     if (p.ks <= 1) return 0;
@@ -2425,7 +2606,7 @@ namespace {
 template <int MODE>
 void launch_gemm(const ProjArgs& a, const ProjPlan& t, dim3 g, hipStream_t s) {
     const bool q8 = a.w_type == VVA_TYPE_Q8_0;
-    const dim3 b(t.tm == 256 ? 512 : 256);
+    const dim3 b(256);
 #define VVA_GEMM(TM, TN, PF)                                                                                   \
     if (q8) hipLaunchKernelGGL((proj_gemm_kernel<true, MODE, TM, TN, PF, 0>), g, b, 0, s, a);                  \
     else    hipLaunchKernelGGL((proj_gemm_kernel<false, MODE, TM, TN, PF, 0>), g, b, 0, s, a)
@@ -2439,7 +2620,8 @@ void launch_gemm(const ProjArgs& a, const ProjPlan& t, dim3 g, hipStream_t s) {
     if (t.tm == 64 && t.tn == 64) { VVA_GEMM(64, 64, 6); }
     else if (t.tm == 64) { VVA_GEMM(64, 128, 4); }
     else if (t.tm == 128) { VVA_GEMM(128, 128, 4); }
-    else { VVA_GEMM(256, 128, 4); }
+    else if (q8) hipLaunchKernelGGL((proj_gemm_kernel<true, MODE, 256, 128, 4, 0>), g, dim3(512), 0, s, a);
+    else hipLaunchKernelGGL((proj_gemm_wide_kernel<MODE>), g, dim3((kWCompute + kWProd) * 64), 0, s, a);
 #undef VVA_GEMM
 }
 }  // namespace
