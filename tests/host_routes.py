@@ -358,9 +358,24 @@ def projection_plans():
             assert st == vva.OK and (tm < 256 or (wt == vva.Q8_0 and N >= 1024)), (wt, N, kernels)
 
 
+def whole_row_windows():
+    """vva_attn of one token over 16-bit caches: the register-streamed kernel
+    for one query head per kv head over many long windows and for 8 heads of 64
+    dims from HBM, the one-launch kernel for the rest (every model's heads)."""
+    for d, Hkv, G, B, L, whole in ((64, 8, 1, 4, 1023, False), (64, 8, 1, 4, 1024, True), (64, 2, 1, 15, 4000, False),
+                                   (128, 2, 1, 16, 4000, True), (128, 2, 1, 1, 32768, False), (64, 8, 4, 16, 4000, True),
+                                   (64, 8, 4, 4, 8000, False), (64, 8, 8, 16, 4000, False), (64, 8, 8, 16, 8192, True),
+                                   (128, 8, 8, 16, 16000, False), (64, 2, 7, 16, 32768, False),
+                                   (128, 2, 6, 16, 32768, False), (128, 4, 7, 16, 32768, False)):
+        for t in (vva.F16, vva.BF16, vva.F32):
+            kernel = one_token_call(t, Hkv, Hkv * G, d, L, B=B)[0].split("<")[0]
+            want = "decode_kernel" if whole and t != vva.F32 else "decode_step_kernel"
+            assert kernel == want, (d, Hkv, G, B, L, t, kernel)
+
+
 SCENARIOS = [bf16_v_window, one_token_precision, workspace_one_can_do_without, f32_step_without_workspace,
              step_output_alignment, output_over_inputs, rope_of_few_rows,
-             projection_plans]
+             projection_plans, whole_row_windows]
 
 if __name__ == "__main__":
     {f.__name__: f for f in SCENARIOS}[sys.argv[1]]()

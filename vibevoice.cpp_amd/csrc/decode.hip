@@ -658,6 +658,26 @@ bool decode_supported(const AttnArgs& a) {
     return true;
 }
 
+// This kernel reads whole cache rows, the one-launch kernel one head's part of
+// them.  Where the arithmetic (which MFMA makes cheaper) is not what bounds the
+// call, that is the faster way: one query head per kv head over many windows
+// (us per call, here against there: 8 heads of 64, 4 x 4000 keys 10.4 against
+// 11.4, 4 x 16000 28.4 against 32.5; 2 heads of 64, 16 x 4000 10.7 against 11.6;
+// 500 keys 8.4 against 7.2), and 8 heads of 64 dims from HBM (4 query heads per
+// kv head, 16 x 16000 keys 97.9 against 114.8, 4 x 16000 30.2 against 32.7; 8
+// per kv head, 16 x 16000 105 against 116, 4 x 16000 34.0 against 33.3).
+bool decode_whole_rows(const AttnArgs& a) {
+    const int G = a.Hq / a.Hkv;
+    int Lmax = 0;
+    double bytes = 0.0;
+    for (int b = 0; b < a.B; ++b) {
+        Lmax = a.L[b] > Lmax ? a.L[b] : Lmax;
+        bytes += 4.0 * a.L[b] * a.Hkv * a.d;           // K and V of 16-bit rows
+    }
+    if (G == 1 && a.B * a.Hkv >= 32 && Lmax >= 1024) return true;
+    return a.d == 64 && a.Hkv == 8 && bytes >= (G <= 4 ? 128e6 : 256e6);
+}
+
 hipError_t launch_decode(const AttnArgs& a, float* ws, int n_splits, int split_len, hipStream_t s) {
     if (a.d == 64) {
         switch (a.k_type) {

@@ -304,7 +304,8 @@ vva_status run_attention(vva_context* ctx, AttnArgs& a, bool fixed = false) {
     const TokenRows q_rows{a.q, a.q_nb_b, a.q_nb_h, a.Hq, a.d, a.q_type, a.B};
     const TokenRows o_rows{(const char*)a.out, a.o_nb_b, a.o_nb_h, a.Hq, a.d, VVA_TYPE_F32, a.B};
     if (ctx->attn_path != 1 && a.T == 1 && a.k_type == a.v_type && a.mask_mode != kMaskExplicit &&
-        (a.k_type == VVA_TYPE_F32 || decode_supported(a)) && (o_rows.same(q_rows) || !o_rows.meets(q_rows))) {
+        (a.k_type == VVA_TYPE_F32 || (decode_supported(a) && !decode_whole_rows(a))) &&
+        (o_rows.same(q_rows) || !o_rows.meets(q_rows))) {
         // F32 / F16 / BF16 rows without an explicit mask: every key is visible to the one token.
         // 16-bit rows: the kernel rounds the probabilities (and BF16 V) to f16, as decode_kernel
         // does, so it takes that kernel's calls; the others keep the row kernel's fp32

@@ -203,6 +203,9 @@ hipError_t launch_decode(const AttnArgs& a, float* ws, int n_splits, int split_l
 bool decode_supported(const AttnArgs& a);
 int decode_waves(const AttnArgs& a);            // waves per workgroup (one key sub-range each)
 int decode_max_splits();
+// Whether a call of decode_supported over 16-bit rows is faster there than in
+// the one-launch kernel
+bool decode_whole_rows(const AttnArgs& a);
 // Second pass of a split decode: combines the (m, l, acc) partials of `ws`
 // (layout of launch_decode) into the output rows.  inf: partials may be
 // infinite where a V element is (F32 caches), and give infinity.
