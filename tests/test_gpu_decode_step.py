@@ -1,6 +1,6 @@
 """GPU parity of vva_decode_step: on F16 / BF16 caches decode_step.hip (RoPE +
-append + split attention + in-kernel merge of the splits in one launch), on
-Q8_0 caches the streamed decode kernel in step mode (RoPE + append +
+append + split attention + merge of the splits in one launch, two past 16
+splits), on Q8_0 caches the streamed decode kernel in step mode (RoPE + append +
 attention, then its merge kernel).
 
 Each step is checked three ways on the same inputs: the appended cache rows

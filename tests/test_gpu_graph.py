@@ -8,9 +8,9 @@ between the replays.  Cache lengths are kernel arguments, so a replay
 repeats the captured step at the same positions: every replay must write
 the same cache rows and outputs as the eager step, bit for bit (same
 kernels, same inputs).  Shapes: the TTS CFG decode of the 0.5B LM (B = 2,
-14 q / 2 kv heads, d = 64, F16 caches at L = 1024: the register-streamed
-decode and its merge) and the 7B ASR CFG decode on Q8_0 caches (the
-LDS-streamed decode and its merge).
+14 q / 2 kv heads, d = 64, F16 caches at L = 1024: the one-launch kernel,
+whose last workgroup merges the splits and resets its ticket) and the 7B ASR
+CFG decode on Q8_0 caches (the LDS-streamed decode and its merge).
 """
 import numpy as np
 import pytest

@@ -16,7 +16,8 @@ B = vva.MAX_BATCH
 
 @pytest.mark.parametrize("d,Hq,Hkv,t", [
     (128, 28, 4, vva.Q8_0),     # the streamed Q8_0 decode kernel: grid (splits, 16 sequences x 2 head pairs)
-    (64, 14, 2, vva.F16),       # the register-streamed kernel
+    (64, 14, 2, vva.F16),       # the one-launch kernel: grid (splits, 2 kv heads, 16), a merge launch past 16 splits
+    (64, 8, 8, vva.F16),        # one query head per kv head over long windows: the register-streamed kernel
 ])
 def test_decode_sixteen_sequences(ctx, torch_gpu, d, Hq, Hkv, t):
     torch = torch_gpu

@@ -180,8 +180,11 @@ def test_vector_and_scalar_paths_agree_bit_for_bit(ctx, torch_gpu, in_t, cache_t
 
 @pytest.mark.parametrize("d,Hq,Hkv", [(128, 28, 4), (64, 14, 2)])
 @pytest.mark.parametrize("T,B,cache_t,q_t,kv_t,out_t", [
+    # Q8_0 caches of 64-dim heads: the scalar kernel either way below 80 rows, compared from there on
     (1, 2, vva.Q8_0, vva.F32, vva.F32, vva.F32),       # a decode step: slices of one token's items
     (33, 1, vva.Q8_0, vva.BF16, vva.BF16, vva.BF16),
+    (40, 2, vva.Q8_0, vva.BF16, vva.F32, vva.F16),     # 80 rows
+    (33, 1, vva.F16, vva.F32, vva.BF16, vva.BF16),     # few rows into a float cache
     (511, 2, vva.Q8_0, vva.F32, vva.F16, vva.F16),     # 1022 rows: the last one-token count; mixed input types
     (1025, 1, vva.F32, vva.F16, vva.BF16, vva.F32),    # two tokens per workgroup, the last one alone
 ])
