@@ -337,7 +337,8 @@ VVA_API int        vva_last_decode_splits(const vva_context* ctx);
 /* Scheduling overrides for tests and benchmarks, per context; 0 restores the
  * automatic choice:
  *   decode_wgs      workgroups a single-token call is planned for (default:
- *                   the device's CU count);
+ *                   the device's CU count for the streamed kernels, twice
+ *                   that for the one-launch kernel);
  *   decode_splits   key splits per (sequence, head group) of the LDS-streamed
  *                   Q8_0 decode, 1..1024;
  *   prefill_splits  key splits per row tile of the MFMA prefill, 1..32.

@@ -2,6 +2,11 @@
 // Q8_0 KV cache: the per-step attention of the TTS / ASR decode loops
 // (src/vibevoice_tts.cpp:862-880, src/vibevoice_asr.cpp:760-800), i.e.
 // ggml_flash_attn_ext with one query row per head (src/qwen2.cpp:332-334).
+// It takes the calls of decode_supported that the one-launch kernel
+// (decode_step.hip) and the streamed Q8_0 kernel (decode_stream.hip) do not:
+// explicit masks, Q8_0 caches of other shapes (or all of them, attn_path 2),
+// out over other memory of q than its own, and the 16-bit windows of
+// decode_whole_rows.  decode_merge_kernel serves all three.
 //
 // Bandwidth-bound, no MFMA.
 //

@@ -46,8 +46,9 @@
 // P and V enter the second product as f16 (BF16 V is converted after the
 // transposing read, or ahead of the kernel where window_bf16_v_bytes says so:
 // 8 waves x 32 rows each convert every fragment otherwise; 1.5B, 4096 tokens
-// 111 -> 97 us with the RoPE + append, 0.5B 83.7 -> 74.8): an 8-bit-mantissa P would cost up to ~4e-3 on short
-// rows, f16 P stays below 4e-4.  Q is rounded to K's type, as ggml's CPU
+// 111 -> 97 us with the RoPE + append as it was then, 88 now; 0.5B 83.7 -> 74.8):
+// an 8-bit-mantissa P would cost up to ~4e-3 on short rows, f16 P stays below
+// 4e-4.  Q is rounded to K's type, as ggml's CPU
 // flash attention does.  Q8_0 and F32 windows are converted to f16 first by
 // window_to_f16_kernel (the reference casts F32 windows the same way before
 // flash attention, src/qwen2.cpp:328-331; for Q8_0 K, Q takes the Q8_0
