@@ -45,7 +45,7 @@
 //              src/qwen2.cpp:269-270).
 //   supports   the flash-attention probe shape of src/backend.cpp:157-196.
 //
-// The oracle (oracle/vvo.h) is the checker only.  Usage: test_qwen2_resident
+// The oracle (oracle/vvo.h) only checks results.  Usage: test_qwen2_resident
 // [--list | name ...]; no names runs everything.
 #include <hip/hip_runtime_api.h>
 #include <math.h>
